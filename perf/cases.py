@@ -35,13 +35,13 @@ def listed():
         # the 64,000-particle dam break, its step captured once and replayed
         _case("fluid_64k", "lattice", 40, graph=True),
         # a viscous liquid with cohesion and surface tension, an odd particle count
-        _case("viscous_300k", "fill", 300_007, warm=4, viscosity=0.2, cohesion=0.05, tension=0.3),
+        _case("viscous_300k", "fill", 300_007, warm=4, radius=0.03, viscosity=50.0, cohesion=0.5, tension=5000.0),
         # the large random fill at rest density, a few steps in
         _case("fluid_4m", "fill", 4_194_304, warm=4),
         # the same fluid after it has slumped: more neighbors, unequal cell blocks
         _case("fluid_settled_1m", "fill", 1_048_573, warm=36),
         # a rendered fluid: vorticity confinement and the anisotropy frames the renderer reads back
-        _case("render_200k", "fill", 200_003, warm=4, vorticity=0.3, anisotropy=True),
+        _case("render_200k", "fill", 200_003, warm=4, radius=0.03, vorticity=0.6, anisotropy=True),
         # fluid, tet soft body and cloth in one scene, with contacts between them
         _case("mixed_360k", "mixed", 64, graph=True, warm=4, tet=32, cloth=256),
         # one cloth, and one tet soft body (the solids of the batched workload, alone)
@@ -72,12 +72,13 @@ def draw(rng):
         c = _case("", "fill", _log_uniform(rng, 20_000, 2_500_000) | 1, warm=rng.choice([4, 12]), **p)
     elif kind == "liquid":
         p.update(substeps=4, iterations=4, cap=64)
-        c = _case("", "fill", _log_uniform(rng, 20_000, 500_000), warm=4, viscosity=rng.choice([0.01, 0.2]),
-                  cohesion=rng.choice([0.0, 0.05]), tension=rng.choice([0.0, 0.3]), **p)
+        c = _case("", "fill", _log_uniform(rng, 20_000, 500_000), warm=4, radius=rng.choice([0.02, 0.03]),
+                  viscosity=rng.choice([0.01, 20.0, 50.0]), cohesion=rng.choice([0.0, 0.5]),
+                  tension=rng.choice([0.0, 5000.0]), **p)
     elif kind == "render":
         p.update(substeps=4, iterations=4, cap=64)
-        c = _case("", "fill", _log_uniform(rng, 20_000, 300_000), warm=4, vorticity=rng.choice([0.0, 0.3]),
-                  anisotropy=True, **p)
+        c = _case("", "fill", _log_uniform(rng, 20_000, 300_000), warm=4, radius=rng.choice([0.02, 0.03]),
+                  vorticity=rng.choice([0.0, 0.6]), anisotropy=True, **p)
     elif kind == "mixed":
         p.update(substeps=4, iterations=4, cap=64)
         c = _case("", "mixed", rng.randint(16, 56), warm=4, tet=rng.randint(6, 28), cloth=rng.randint(24, 220), **p)
@@ -102,7 +103,11 @@ def _scene(case, seed):
     if kind == "lattice":
         return scenes.dam_break_64k(seed=seed, side=n)
     if kind == "fill":
-        sc = scenes.large_pbf(n, seed=seed, box=scenes.scaled_box_for(n))
+        box = scenes.scaled_box_for(n)
+        if "radius" in case:  # the same fill of larger particles (and a box as much larger)
+            scale = case["radius"] / scenes.random_fill_radius(n, float(np.prod(box)))
+            box = tuple(scale * b for b in box)
+        sc = scenes.large_pbf(n, seed=seed, box=box)
         sc.fluid_mats = cnhip.fluid_material(
             float(sc.radii[0]), viscosity=case.get("viscosity", 0.01), cohesion=case.get("cohesion", 0.0),
             surface_tension=case.get("tension", 0.0), vorticity_confinement=case.get("vorticity", 0.0))
