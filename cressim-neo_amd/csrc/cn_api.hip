@@ -612,6 +612,7 @@ SubstepConsts make_consts(const cn_ctx *ctx, const SceneBuffers &s, const cn_ste
     c.grid_max = ctx->grid_max;
     c.superset = (p->flags & CN_STEP_CANDIDATE_REUSE) && s.slist ? 1u : 0u;
     c.fluid_iters = p->fluid_iterations > 0 ? p->fluid_iterations : std::max<uint32_t>(p->default_iterations, 1u);
+    c.pairs = ctx->any_pairs ? 1u : 0u;
     c.fluid_scenes = ctx->fluid_scenes;
     fluid_tiles(c);
     c.cfl_guard = 1.001f;
@@ -644,7 +645,7 @@ uint2 *broadphase(cn_ctx *ctx, SceneBuffers &s, const SubstepConsts &c, uint32_t
     if (c.key_mode == CN_KEY_MORTON) {
         ProfScope ps(ctx, "blocks");
         launch_blocks(s, c, ctx->stream);
-        if (ctx->has_fluid) launch_blk_halo(s, c, ctx->stream);
+        if (ctx->has_fluid || ctx->any_pairs) launch_blk_halo(s, c, ctx->stream);
     }
     return sorted;
 }

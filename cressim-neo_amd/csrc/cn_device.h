@@ -35,6 +35,9 @@ constexpr int kCfgFluidBndDensity = 34;
 constexpr int kCfgFluidBndDelta = 35;
 constexpr int kCfgFluidMaxUnder = 36;
 
+constexpr uint32_t kPhaseGroupMask = 0x7fffffffu;    // particle phase: the group, and
+constexpr uint32_t kPhaseSelfCollide = 0x80000000u;  // whether its particles collide with each other
+
 // Static per-particle attributes, deduplicated on upload; each particle stores a class index.
 struct ParticleClass {
     float radius;
@@ -132,6 +135,7 @@ struct SubstepConsts {
     uint32_t grid_max;       // workgroups of a persistent fluid launch (upper bound)
     uint32_t superset;       // 1: LDS blocks of fluid-only scenes reuse iteration 0's candidate lists
     uint32_t fluid_iters;    // fluid iterations per substep
+    uint32_t pairs;          // 1: some scene can hold a particle-particle contact pair
     uint32_t fluid_scenes;   // scenes with fluid particles: they hold key prefixes [0, fluid_scenes)
     float cfl_guard;         // relative margin of the CFL-term skip test
     float cfg[CN_SOLVER_CONFIG_FLOATS];

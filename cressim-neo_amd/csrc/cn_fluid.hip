@@ -677,21 +677,32 @@ __device__ __forceinline__ void flush_disp(float d2, const FluidArgs &a)
 __global__ __launch_bounds__(kBlock) void k_blk_halo(FluidArgs a, SubstepConsts c)
 {
     __shared__ uint32_t scan[kBlock];
-    const uint32_t nb = min(a.nblk[1], c.blk_cap);
+    __shared__ uint32_t s_kinds, s_gmin, s_gmax;  // what the halo holds: kHas* bits, solid phase groups
+    constexpr uint32_t kHasFluid = 1, kHasSolid = 2, kHasOther = 4;
+    // blocks of scenes with fluid are a prefix; contact pairs can exist in any scene
+    const uint32_t nb = min(a.nblk[c.pairs ? 0 : 1], c.blk_cap);
     const uint32_t tid = threadIdx.x;
     for (uint32_t b = blockIdx.x; b < nb; b += gridDim.x) {
         const uint32_t p0 = a.run_start[a.blk_first_run[b]], p1 = a.run_start[a.blk_first_run[b + 1]];
         const uint32_t scene = a.classes[a.cls[p0]].scene;
         uint32_t *hd = a.blk_halo + (size_t)b * kHaloStride;
-        if (!a.scenes[scene].has_fluid) {  // a scene without fluid: no fluid pass visits the block
+        const bool fluid = a.scenes[scene].has_fluid != 0u, pairs = a.scenes[scene].pairs != 0u;
+        if (!fluid && !pairs) {  // no fluid pass visits the block and no contact pair exists in it
             if (tid == 0) {
                 hd[kHdFlags] = kHdNoFluid;
+                hd[kHdPairs] = 0u;
                 hd[kHdP0] = p0;
                 hd[kHdP1] = p1;
                 hd[kHdScene] = scene;
             }
             continue;
         }
+        if (tid == 0) {
+            s_kinds = 0u;
+            s_gmin = kInvalid;
+            s_gmax = 0u;
+        }
+        __syncthreads();
         const int4 c0 = a.cellc[p0];
         const int bx = c0.x & ~3, by = c0.y & ~3, bz = c0.z & ~3;
         // particles of a wrapped Morton block that lie outside the aligned block, particles whose own
@@ -710,10 +721,27 @@ __global__ __launch_bounds__(kBlock) void k_blk_halo(FluidArgs a, SubstepConsts 
                 const int r = find_run(cell_key(tx, ty, tz, (uint32_t)c0.w, c.key_mode, c.morton_bits), run_table(a));
                 if (r >= 0) {
                     const int4 info = a.run_info[r];
-                    if (info.w == 0) bad = true;
+                    if (!(info.w & kRunPure)) bad = true;
                     else if (info.x == tx && info.y == ty && info.z == tz) {
                         st = a.run_start[r];
                         cnt = a.run_start[r + 1] - st;
+                        if (pairs) {
+                            // what the cell holds; a cell of several classes may hold anything, and
+                            // so may a self-colliding group
+                            const uint32_t k = run_class(info.w);
+                            uint32_t has = kHasOther;
+                            if (k != kInvalid) {
+                                const ParticleClass pc = a.classes[k];
+                                if (pc.kind == CN_PARTICLE_KIND_FLUID) {
+                                    has = kHasFluid;
+                                } else if (pc.kind == CN_PARTICLE_KIND_SOLID && !(pc.phase & kPhaseSelfCollide)) {
+                                    has = kHasSolid;
+                                    atomicMin(&s_gmin, pc.phase & kPhaseGroupMask);
+                                    atomicMax(&s_gmax, pc.phase & kPhaseGroupMask);
+                                }
+                            }
+                            atomicOr(&s_kinds, has);
+                        }
                     }
                 }
             }
@@ -727,10 +755,14 @@ __global__ __launch_bounds__(kBlock) void k_blk_halo(FluidArgs a, SubstepConsts 
         }
         if (tid == 0) {
             // blocks the delta pass stages only in the wide tile get their own launch
-            if (!any_bad && total > c.tile_delta && total <= c.tile_wide)
+            if (fluid && !any_bad && total > c.tile_delta && total <= c.tile_wide)
                 a.wide_blk[atomicAdd(a.iter_state + kStateWideCount, 1u)] = b;
             hd[kHdOff + kHalo] = total;
             hd[kHdFlags] = any_bad ? 0u : 1u;
+            hd[kHdPairs] = (s_kinds & kHasOther) || (s_kinds & (kHasFluid | kHasSolid)) == (kHasFluid | kHasSolid) ||
+                                   ((s_kinds & kHasSolid) && s_gmin != s_gmax)
+                               ? 1u
+                               : 0u;
             hd[kHdP0] = p0;
             hd[kHdP1] = p1;
             hd[kHdBase] = (uint32_t)bx;

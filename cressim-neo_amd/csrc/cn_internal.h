@@ -35,8 +35,10 @@ constexpr uint32_t kHdP0 = kHdFlags + 1;
 constexpr uint32_t kHdP1 = kHdFlags + 2;
 constexpr uint32_t kHdBase = kHdFlags + 3;      // 3 words
 constexpr uint32_t kHdScene = kHdFlags + 6;
+constexpr uint32_t kHdPairs = kHdFlags + 7;     // 1: a contact pair can exist between particles of the halo
 constexpr uint32_t kHaloStride = 448;
-constexpr uint32_t kHdNoFluid = 2u;  // kHdFlags value of a block in a scene without fluid particles
+// kHdFlags value of a block in a scene without fluid particles or contact pairs (no halo written)
+constexpr uint32_t kHdNoFluid = 2u;
 // candidate contact partners a particle keeps per substep; more are counted as overflows
 constexpr uint32_t kContactPartners = 32;
 constexpr uint32_t kMetaWords = 16;  // device diagnostics words

@@ -12,6 +12,7 @@
 #include <algorithm>
 
 #include "cn_internal.h"
+#include "cn_walk.h"
 
 namespace cn {
 
@@ -318,12 +319,14 @@ __global__ __launch_bounds__(kBlock) void k_reorder(
                                  grp + sc.grp0, bndl + (size_t)t * kBndListCap, meta, p.x, p.y, p.z);
 }
 
-// (cx, cy, cz, pure): pure runs hold a single cell; mixed runs (hash collisions or wrapped
-// Morton coordinates) are filtered per particle like the reference (:94-98).
+// (cx, cy, cz, w): pure runs hold a single cell; mixed runs (hash collisions or wrapped
+// Morton coordinates) are filtered per particle like the reference (:94-98).  cls: the slots'
+// classes when the contact candidates want each run's one class (null otherwise).  The members are
+// read four at a time, so a run of a few particles costs one round trip.
 __global__ __launch_bounds__(kBlock) void k_run_info(const uint32_t *__restrict__ run_start,
                                                      const uint32_t *__restrict__ run_count,
-                                                     const int4 *__restrict__ cellc, int4 *__restrict__ run_info,
-                                                     uint32_t *__restrict__ meta)
+                                                     const int4 *__restrict__ cellc, const uint32_t *__restrict__ cls,
+                                                     int4 *__restrict__ run_info, uint32_t *__restrict__ meta)
 {
     const uint32_t r = blockIdx.x * kBlock + threadIdx.x;
     uint32_t occ = 0;
@@ -331,15 +334,24 @@ __global__ __launch_bounds__(kBlock) void k_run_info(const uint32_t *__restrict_
         const uint32_t s = run_start[r], e = run_start[r + 1];
         occ = e - s;
         const int4 c0 = cellc[s];
-        int pure = 1;
-        for (uint32_t q = s + 1; q < e; ++q) {
-            const int4 cq = cellc[q];
-            if (cq.x != c0.x || cq.y != c0.y || cq.z != c0.z) {
-                pure = 0;
-                break;
+        const uint32_t k0 = cls ? cls[s] : 0u;
+        bool pure = true, one = cls != nullptr;
+        for (uint32_t q = s + 1; q < e && (pure || one); q += 4) {
+            int4 cq[4];
+            uint32_t kq[4];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) {
+                const uint32_t i = min(q + u, e - 1u);
+                cq[u] = cellc[i];
+                kq[u] = cls ? cls[i] : 0u;
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) {
+                pure &= cq[u].x == c0.x && cq[u].y == c0.y && cq[u].z == c0.z;
+                one &= kq[u] == k0;
             }
         }
-        run_info[r] = make_int4(c0.x, c0.y, c0.z, pure);
+        run_info[r] = make_int4(c0.x, c0.y, c0.z, (pure ? kRunPure : 0) | (one ? run_class_word(k0) : 0));
     }
     // longest run: wave maximum, and an atomic only when it beats the value already stored
     for (int o = 32; o > 0; o >>= 1) occ = max(occ, (uint32_t)__shfl_xor((int)occ, o));
@@ -355,7 +367,7 @@ void launch_reorder(SceneBuffers &s, const SubstepConsts &c, hipStream_t st)
                        s.ne + s.nb + s.nd + s.nt ? s.slot_of : nullptr, s.classes, s.fluid_mats, s.colliders,
                        s.col_groups, s.scenes, s.scene_active, s.meta, c);
     hipLaunchKernelGGL(k_run_info, dim3(grid1(c.n)), dim3(kBlock), 0, st, s.run_start, s.run_count, s.cellc,
-                       s.run_info, s.meta);
+                       c.pairs ? s.cls[nw] : nullptr, s.run_info, s.meta);
     s.cur = nw;
 }
 

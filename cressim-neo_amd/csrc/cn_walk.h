@@ -10,19 +10,34 @@ namespace cn {
 struct RunTable {
     const uint32_t *run_key;
     const uint32_t *run_start;
-    const int4 *run_info;   // (cx, cy, cz, pure)
+    const int4 *run_info;   // (cx, cy, cz, kRunPure | run_class or 0)
     const uint32_t *bucket;
     uint32_t bucket_shift;
     const int4 *cellc;
 };
 
+// run_info.w: bit 0 the run holds a single cell; above it the particle class of every member plus
+// one, or 0 when they differ (or the substep has no use for it).
+constexpr int kRunPure = 1;
+__device__ __forceinline__ int run_class_word(uint32_t cls) { return (int)((cls + 1u) << 1); }
+__device__ __forceinline__ uint32_t run_class(int w) { return ((uint32_t)w >> 1) - 1u; }  // kInvalid: differ
+
+// The run of a key: a binary search of its bucket's runs.  A bucket is a range of keys, so where a
+// scene fills a corner of its key range (a pool whose key holds the scene, a small body in a large
+// box) one bucket holds hundreds of runs: the linear scan it replaces made the 48-scene pool's halo
+// lookups 312 us a substep.
 __device__ __forceinline__ int find_run(uint32_t key, const RunTable &t)
 {
     const uint32_t b = key >> t.bucket_shift;
-    uint32_t r = t.bucket[b];
+    uint32_t lo = t.bucket[b];
     const uint32_t e = t.bucket[b + 1];
-    while (r < e && t.run_key[r] < key) ++r;
-    return (r < e && t.run_key[r] == key) ? (int)r : -1;
+    uint32_t hi = e;
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (t.run_key[mid] < key) lo = mid + 1u;
+        else hi = mid;
+    }
+    return (lo < e && t.run_key[lo] == key) ? (int)lo : -1;
 }
 
 // f(slot) for the particles of the 27 cells around cell ci in dz, dy, dx order, each cell's
@@ -41,7 +56,7 @@ __device__ __forceinline__ void walk_runs(int4 ci, const RunTable &t, const Subs
                 const int r = find_run(cell_key(tx, ty, tz, (uint32_t)ci.w, c.key_mode, c.morton_bits), t);
                 if (r < 0) continue;
                 const int4 info = t.run_info[r];
-                const bool pure = info.w != 0;
+                const bool pure = (info.w & kRunPure) != 0;
                 if (pure && (info.x != tx || info.y != ty || info.z != tz)) continue;
                 const uint32_t qe = t.run_start[r + 1];
                 for (uint32_t q = t.run_start[r]; q < qe; ++q) {
