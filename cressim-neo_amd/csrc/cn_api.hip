@@ -99,6 +99,7 @@ struct cn_ctx {
     std::vector<SceneInfo> scene_info;    // host copy of the device scene records
     std::vector<uint32_t> scene_fm;       // per scene: first fluid material, count (pairs)
     std::vector<uint32_t> scene_pm;       // per scene: first particle material, count (pairs)
+    float max_viscosity = 0.0f;  // largest viscosity of the table (kernel choice)
     std::vector<cn_fluid_material> fm_host;  // host copy of the pool's fluid material table
     std::vector<uint8_t> fm_fluid_used;      // per fluid material: referenced by a fluid particle
     std::vector<uint32_t> scene_con;      // per scene: first edge, bend, dihedral, tet (4 words)
@@ -211,12 +212,11 @@ void free_scene(SceneBuffers &s)
     dfree(s.blk_halo);
     dfree(s.wide_blk);
     dfree(s.iter_state);
-    dfree(s.fluid_t2);
+    dfree(s.fluid_consts);
     dfree(s.list);
     dfree(s.lcnt);
     dfree(s.slist);
     dfree(s.scnt);
-    dfree(s.disp);
     dfree(s.adj_off);
     dfree(s.adj_cnt);
     dfree(s.adj_idx);
@@ -543,6 +543,22 @@ float sqrt_threshold(float h)
     return x;
 }
 
+// The operations are those of the kernels' helpers (spiky_coef and the plain products).
+FluidConst fluid_const(const cn_fluid_material &m)
+{
+    FluidConst f{};
+    f.h = m.smoothing_radius > 1.0e-4f ? m.smoothing_radius : 1.0e-4f;
+    f.t2 = sqrt_threshold(f.h);
+    const float h2 = f.h * f.h, h3 = h2 * f.h;
+    f.kw = 15.0f / (kKernelPi * h3);
+    f.ih = 1.0f / f.h;
+    const float skin = kSkinFrac * f.h, hs = f.h + skin;
+    f.ts2 = hs * hs * 1.00001f;
+    f.rs = std::sqrt(f.ts2);
+    f.allow = 0.98f * skin;
+    return f;
+}
+
 struct ProfScope {
     cn_ctx *ctx;
     int slot;
@@ -589,6 +605,14 @@ uint32_t key_bits_of(const cn_ctx *ctx, const cn_step_params *p)
     return p->key_mode == CN_KEY_HASH ? 32u : 3u * ctx->morton_bits + ctx->scene_bits;
 }
 
+// every scene of the context takes part in the step (the active flags last written are all set)
+bool all_active(const cn_ctx *ctx)
+{
+    for (uint32_t f : ctx->active_host)
+        if (!f) return false;
+    return true;
+}
+
 SubstepConsts make_consts(const cn_ctx *ctx, const SceneBuffers &s, const cn_step_params *p, float dt)
 {
     SubstepConsts c{};
@@ -613,6 +637,8 @@ SubstepConsts make_consts(const cn_ctx *ctx, const SceneBuffers &s, const cn_ste
     c.superset = (p->flags & CN_STEP_CANDIDATE_REUSE) && s.slist ? 1u : 0u;
     c.fluid_iters = p->fluid_iterations > 0 ? p->fluid_iterations : std::max<uint32_t>(p->default_iterations, 1u);
     c.pairs = ctx->any_pairs ? 1u : 0u;
+    c.viscous = dt * ctx->max_viscosity > kEps ? 1u : 0u;
+    c.all_active = all_active(ctx) ? 1u : 0u;
     c.fluid_scenes = ctx->fluid_scenes;
     fluid_tiles(c);
     c.cfl_guard = 1.001f;
@@ -849,7 +875,7 @@ cn_status cn_scene_reserve(cn_ctx *ctx, uint32_t n, uint32_t cap)
     s.blk_cap = (uint32_t)std::max<size_t>(256, N / 32);
     CN_HIP(ctx, dalloc(&s.blk_halo, (size_t)s.blk_cap * kHaloStride));
     CN_HIP(ctx, dalloc(&s.wide_blk, s.blk_cap));
-    CN_HIP(ctx, dalloc(&s.list, list_slots(N) * (cap ? cap : 1)));
+    CN_HIP(ctx, dalloc(&s.list, list_entries(N, cap)));
     CN_HIP(ctx, dalloc(&s.lcnt, N));
     CN_HIP(ctx, dalloc(&s.iter_state, kStateWords));
     CN_HIP(ctx, hipMemsetAsync(s.iter_state, 0, kStateWords * sizeof(uint32_t), ctx->stream));
@@ -1234,7 +1260,7 @@ cn_status upload_pool(cn_ctx *ctx, uint32_t count, const cn_scene_desc *descs)
     dfree(s.part_mats);
     dfree(s.colliders);
     dfree(s.scenes);
-    dfree(s.fluid_t2);
+    dfree(s.fluid_consts);
     dfree(s.scene_active);
     dfree(s.pid_scene);
     s.scene_active = nullptr;
@@ -1244,7 +1270,7 @@ cn_status upload_pool(cn_ctx *ctx, uint32_t count, const cn_scene_desc *descs)
     s.part_mats = nullptr;
     s.colliders = nullptr;
     s.scenes = nullptr;
-    s.fluid_t2 = nullptr;
+    s.fluid_consts = nullptr;
     dfree(s.adj_off);
     dfree(s.adj_cnt);
     dfree(s.adj_idx);
@@ -1307,15 +1333,18 @@ cn_status upload_pool(cn_ctx *ctx, uint32_t count, const cn_scene_desc *descs)
     }
     ctx->max_h = 1.0e-4f;
     ctx->has_tension = false;
-    std::vector<float> t2(fmh.size());
+    ctx->max_viscosity = 0.0f;
+    std::vector<FluidConst> fconst(fmh.size());
     for (size_t k = 0; k < fmh.size(); ++k) {
         const cn_fluid_material &m = fmh[k];
         ctx->max_h = std::max(ctx->max_h, m.smoothing_radius);
         ctx->has_tension |= (m.surface_tension > 0.0f ? m.surface_tension : 0.0f) > kEps;
-        t2[k] = sqrt_threshold(m.smoothing_radius > 1.0e-4f ? m.smoothing_radius : 1.0e-4f);
+        ctx->max_viscosity = std::max(ctx->max_viscosity, m.viscosity);
+        fconst[k] = fluid_const(m);
     }
-    CN_HIP(ctx, dalloc(&s.fluid_t2, t2.size()));
-    if (!t2.empty()) CN_HIP(ctx, hipMemcpy(s.fluid_t2, t2.data(), t2.size() * sizeof(float), hipMemcpyHostToDevice));
+    CN_HIP(ctx, dalloc(&s.fluid_consts, fconst.size()));
+    if (!fconst.empty())
+        CN_HIP(ctx, hipMemcpy(s.fluid_consts, fconst.data(), fconst.size() * sizeof(FluidConst), hipMemcpyHostToDevice));
 
 
     std::vector<uint32_t> ids(n);
@@ -1489,14 +1518,6 @@ namespace {
 
 // Enqueues one cn_step (every substep) on the context stream over the buffer set s (the pool's,
 // or a compact tick's view of the listed scenes); advances s's slot-order parity.
-// every scene of the context takes part in the step (the active flags last written are all set)
-bool all_active(const cn_ctx *ctx)
-{
-    for (uint32_t f : ctx->active_host)
-        if (!f) return false;
-    return true;
-}
-
 void record_step(cn_ctx *ctx, SceneBuffers &s, const cn_step_params *p)
 {
     const uint32_t substeps = std::max<uint32_t>(p->substeps, 1u);
@@ -1698,12 +1719,11 @@ cn_status ensure_tick(cn_ctx *ctx, uint32_t m)
     t.blk_cap = (uint32_t)std::max<size_t>(256, N / 32);
     CN_HIP(ctx, dalloc(&t.blk_halo, (size_t)t.blk_cap * kHaloStride));
     CN_HIP(ctx, dalloc(&t.wide_blk, t.blk_cap));
-    CN_HIP(ctx, dalloc(&t.list, list_slots(N) * std::max<uint32_t>(ctx->cap_alloc, 1u)));
+    CN_HIP(ctx, dalloc(&t.list, list_entries(N, ctx->cap_alloc)));
     CN_HIP(ctx, dalloc(&t.lcnt, N));
     if (want_sl) {
-        CN_HIP(ctx, dalloc(&t.slist, list_slots(N) * kSuperSlots));
+        CN_HIP(ctx, dalloc(&t.slist, list_entries(N, kSuperSlots)));
         CN_HIP(ctx, dalloc(&t.scnt, N));
-        CN_HIP(ctx, dalloc(&t.disp, N));
     }
     if (want_ct) {
         CN_HIP(ctx, dalloc(&t.ct_list, N * kContactPartners));
@@ -1762,7 +1782,6 @@ SceneBuffers tick_view(const cn_ctx *ctx, uint32_t m, const cn_step_params *p)
     v.lcnt = t.lcnt;
     v.slist = t.slist;
     v.scnt = t.scnt;
-    v.disp = t.disp;
     v.nbr = nullptr;
     v.nbr_cnt = nullptr;
     v.nbr_alloc = 0;
@@ -1874,9 +1893,8 @@ static cn_status step_impl(cn_ctx *ctx, const cn_step_params *p)
     if ((p->flags & CN_STEP_CANDIDATE_REUSE) && !ctx->s.slist && ctx->has_fluid &&
         (uint64_t)list_slots(ctx->capacity) * kSuperSlots * sizeof(uint16_t) <= kListBytesMax) {
         CN_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        CN_HIP(ctx, dalloc(&ctx->s.slist, list_slots(ctx->capacity) * kSuperSlots));
+        CN_HIP(ctx, dalloc(&ctx->s.slist, list_entries(ctx->capacity, kSuperSlots)));
         CN_HIP(ctx, dalloc(&ctx->s.scnt, std::max<uint32_t>(ctx->capacity, 1u)));
-        CN_HIP(ctx, dalloc(&ctx->s.disp, std::max<uint32_t>(ctx->capacity, 1u)));
         ctx->graph_valid = false;
     }
     // the vorticity and anisotropy passes' neighbor lists on first use (the pass entry's list
@@ -2289,12 +2307,15 @@ cn_status cn_scene_set_materials(cn_ctx *ctx, uint32_t scene, const cn_fluid_mat
     // whole table, vorticity over the materials a fluid particle references; the passes still
     // test each particle's own material), and a captured graph holds the old choice
     bool tension = false, vort = false;
+    float visc = 0.0f;
     for (size_t k = 0; k < ctx->fm_host.size(); ++k) {
         const cn_fluid_material &m = ctx->fm_host[k];
         tension |= (m.surface_tension > 0.0f ? m.surface_tension : 0.0f) > kEps;
+        visc = std::max(visc, m.viscosity);
         if (ctx->fm_fluid_used[k]) vort |= std::max(m.vorticity_confinement, 0.0f) > kEps;
     }
-    if (tension != ctx->has_tension || vort != ctx->has_vorticity) ctx->graph_valid = false;
+    if (tension != ctx->has_tension || vort != ctx->has_vorticity || visc != ctx->max_viscosity) ctx->graph_valid = false;
+    ctx->max_viscosity = visc;
     ctx->has_tension = tension;
     ctx->has_vorticity = vort;
     // the host tables may go as soon as the call returns

@@ -48,7 +48,7 @@ struct ContactArgs {
     float4 *pos;              // slot order
     float4 *vel;
     const float4 *prev;
-    float4 *cur;              // fluid solver positions x* + delta
+    float4 *cur;              // fluid solver positions x* + delta (free particles: w = 0)
     const float4 *dacc;       // current fluid delta
     const uint32_t *cls;
     const uint32_t *id;
@@ -477,7 +477,8 @@ __global__ __launch_bounds__(kBlock) void k_contact_apply(ContactArgs a)
     a.pos[t] = p;
     if (pc.kind == CN_PARTICLE_KIND_FLUID) {
         const float4 dl = a.dacc[t];
-        a.cur[t] = make_float4(p.x + dl.x, p.y + dl.y, p.z + dl.z, p.w);
+        // D is of no use here: a scene with contacts keeps no candidate lists
+        a.cur[t] = make_float4(p.x + dl.x, p.y + dl.y, p.z + dl.z, 0.0f);
     }
 }
 

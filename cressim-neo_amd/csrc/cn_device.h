@@ -135,6 +135,8 @@ struct SubstepConsts {
     uint32_t grid_max;       // workgroups of a persistent fluid launch (upper bound)
     uint32_t superset;       // 1: LDS blocks of fluid-only scenes reuse iteration 0's candidate lists
     uint32_t fluid_iters;    // fluid iterations per substep
+    uint32_t viscous;        // 1: some fluid material's viscosity term is on from the second iteration
+    uint32_t all_active;     // 1: every scene takes part in the step
     uint32_t pairs;          // 1: some scene can hold a particle-particle contact pair
     uint32_t fluid_scenes;   // scenes with fluid particles: they hold key prefixes [0, fluid_scenes)
     float cfl_guard;         // relative margin of the CFL-term skip test
@@ -162,11 +164,15 @@ __device__ __forceinline__ float fdiv_rcp(float a, float b, float y) { return -f
 // two Newton steps in fma, which reach the correctly rounded reciprocal from any estimate within
 // two ulps except for the significand 1.11...1 (checked exhaustively over significands); that one
 // takes the IEEE division.
-__device__ __forceinline__ float frcp_exact(float b)
+__device__ __forceinline__ float frcp_newton(float b)
 {
     float y = __builtin_amdgcn_rcpf(b);
     y = __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
-    y = __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
+    return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
+}
+__device__ __forceinline__ float frcp_exact(float b)
+{
+    float y = frcp_newton(b);
     if ((__float_as_uint(b) & 0x7fffffu) == 0x7fffffu) {
         __asm__ volatile("");  // a side effect keeps this rare path a branch rather than a select
         y = fdiv(1.0f, b);
@@ -307,29 +313,55 @@ __device__ __forceinline__ void quat_rotate(float qx, float qy, float qz, float 
     oz = __fadd_rn(__fadd_rn(vz, __fmul_rn(qw, tz)), __fsub_rn(__fmul_rn(qx, ty), __fmul_rn(qy, tx)));
 }
 
+// len3 of a vector known to have at most one nonzero component, of magnitude at least 2^-60 when
+// nonzero: the correctly rounded root of a correctly rounded square is the magnitude itself.
+__device__ __forceinline__ bool one_axis(float x, float y, float z)
+{
+    return (x != 0.0f) + (y != 0.0f) + (z != 0.0f) == 1;
+}
+__device__ __forceinline__ float len3_axis(float x, float y, float z) { return fabsf(x) + fabsf(y) + fabsf(z); }
+// Length and direction v / |v| of a vector that often lies along one axis (dl > 0 wherever the
+// direction is used): the root and the divisions only where some lane's does not.
+__device__ __forceinline__ float len3_dir(float x, float y, float z, float &nx, float &ny, float &nz)
+{
+    const float da = len3_axis(x, y, z);
+    if (one_axis(x, y, z) && da >= 0x1p-60f && da < 0x1p60f) {
+        // a zero component over the length is a zero of its own sign
+        nx = x != 0.0f ? copysignf(1.0f, x) : x;
+        ny = y != 0.0f ? copysignf(1.0f, y) : y;
+        nz = z != 0.0f ? copysignf(1.0f, z) : z;
+        return da;
+    }
+    const float dl = len3(x, y, z);
+    nx = fdiv(x, dl);
+    ny = fdiv(y, dl);
+    nz = fdiv(z, dl);
+    return dl;
+}
+
 // The box branch of ComputeFluidBoundaryContactInfo in the box's frame (local position l):
 // closest point, outside distance and normal, or the inside depth and ClosestFaceNormalLocal
-// (physics_shape_common.hlsli:100-108).
+// (physics_shape_common.hlsli:100-108).  Outside a face (not past an edge) the offset has one
+// component, which len3_dir takes without a root or a division.
 __device__ __forceinline__ void box_local_contact(const float *he, float lx, float ly, float lz, float &sd,
                                                   float &nx, float &ny, float &nz)
 {
     const float dx = __fsub_rn(lx, fclamp(lx, -he[0], he[0]));
     const float dy = __fsub_rn(ly, fclamp(ly, -he[1], he[1]));
     const float dz = __fsub_rn(lz, fclamp(lz, -he[2], he[2]));
-    const float dl = len3(dx, dy, dz);
+    const float dl = len3_dir(dx, dy, dz, nx, ny, nz);
     if (dl > kEps) {
-        nx = fdiv(dx, dl); ny = fdiv(dy, dl); nz = fdiv(dz, dl);
         sd = dl;
-    } else {
-        const float ex = __fsub_rn(he[0], fabsf(lx));
-        const float ey = __fsub_rn(he[1], fabsf(ly));
-        const float ez = __fsub_rn(he[2], fabsf(lz));
-        nx = 0.0f; ny = 0.0f; nz = 0.0f;
-        if (ex <= ey && ex <= ez) nx = lx >= 0.0f ? 1.0f : -1.0f;
-        else if (ey <= ez) ny = ly >= 0.0f ? 1.0f : -1.0f;
-        else nz = lz >= 0.0f ? 1.0f : -1.0f;
-        sd = -fmind(ex, fmind(ey, ez));
+        return;
     }
+    const float ex = __fsub_rn(he[0], fabsf(lx));
+    const float ey = __fsub_rn(he[1], fabsf(ly));
+    const float ez = __fsub_rn(he[2], fabsf(lz));
+    nx = 0.0f; ny = 0.0f; nz = 0.0f;
+    if (ex <= ey && ex <= ez) nx = lx >= 0.0f ? 1.0f : -1.0f;
+    else if (ey <= ez) ny = ly >= 0.0f ? 1.0f : -1.0f;
+    else nz = lz >= 0.0f ? 1.0f : -1.0f;
+    sd = -fmind(ex, fmind(ey, ez));
 }
 
 // ComputeFluidBoundaryContactInfo, physics_fluid_boundary_common.hlsli:10-84: signed distance and

@@ -43,16 +43,15 @@ struct FluidArgs {
     const uint16_t *bndl;
     const float4 *din;        // accumulated delta of the previous iteration
     float4 *dout;
-    float4 *cur;              // (x* + delta, inverse mass) at the start of the iteration
+    float4 *cur;              // (x* + delta, D) at the start of the iteration (kNoMass: no neighbor)
     float4 *cs;               // density-pass records: (x* + delta, C)
     float4 *nc;               // surface normal * tension, C
     uint32_t *nbr;
     uint32_t *nbr_cnt;
-    uint16_t *list;           // listed neighbors as halo offsets in slot groups (list_entry_base)
-    uint32_t *lcnt;           // listed neighbor count
+    uint16_t *list;           // listed neighbors as halo offsets in slot groups (list_words)
+    uint32_t *lcnt;           // what the delta pass walks (list_word)
     uint16_t *slist;          // iteration-0 candidates as halo offsets in slot groups, LDS blocks
-    uint16_t *scnt;           // candidate count, or kSuperNone
-    float *disp;              // per slot: bound on the displacement since iteration 0 (null: not kept)
+    uint32_t *scnt;           // the same for the candidate list
     const uint32_t *run_key;
     const uint32_t *run_start;
     const int4 *run_info;
@@ -65,13 +64,14 @@ struct FluidArgs {
     uint32_t *iter_state;
     const ParticleClass *classes;
     const cn_fluid_material *fm;
-    const float *t2;          // per fluid material: d2 < t2 <=> sqrt(d2) < h
+    const FluidConst *fc;     // per fluid material: what follows from its radius
     const Collider *col;
     const SceneInfo *scenes;
     const uint32_t *active;   // per scene: stepped this cn_step
     uint32_t *meta;
     uint32_t it;
     uint32_t tile;            // halo particles this launch can stage in LDS
+    uint32_t wide_only;       // the delta pass takes the listed wide blocks only
 };
 
 __device__ __forceinline__ RunTable run_table(const FluidArgs &a)
@@ -117,33 +117,48 @@ __device__ __forceinline__ void walk_rows(const uint32_t *hoff, int hc, F &&f)
         }
 }
 
-// Halo cell holding staged particle f: the last cell whose offset is <= f.
-__device__ __forceinline__ uint32_t halo_cell_of(const uint32_t *hoff, uint32_t f)
-{
-    uint32_t lo = 0, hi = kHalo;
-    while (hi - lo > 1) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (hoff[mid] <= f) lo = mid;
-        else hi = mid;
-    }
-    return lo;
-}
-
 // Block queue: the blocks are split into kXcds contiguous chunks, one per die, so neighboring
 // blocks (which share halo cells) run under the same L2; a workgroup drains its die's chunk, then
-// helps the others.  Called by one thread; returns kInvalid when every chunk is drained.
+// helps the others.  Each workgroup's first block is its rank among its die's workgroups, without a
+// counter; the counters hand out what is left, and none is touched when a chunk has no more blocks
+// than workgroups with a fixed first one.  (A counter's atomic is a round trip to the memory side of
+// about a microsecond: taking the first block and finding eight drained chunks by atomics cost a
+// launch over the 64,000-particle dam break some 10 us of its 40.)  Run by one thread.
+constexpr uint32_t kFixedPerDie = 96;  // workgroups of a die with a fixed first block: those resident
 struct BlockQueue {
-    uint32_t die, tries;
-    __device__ explicit BlockQueue(uint32_t wg) : die(wg % kXcds), tries(0) {}
+    uint32_t die, open;  // open: bit d set while chunk d may have blocks
+    bool helping;
+    __device__ explicit BlockQueue(uint32_t wg) : die(wg % kXcds), open((1u << kXcds) - 1u), helping(false) {}
+    __device__ static uint32_t begin(uint32_t nblk, uint32_t d) { return (uint32_t)(((uint64_t)nblk * d) / kXcds); }
+    __device__ static uint32_t fixed(uint32_t d) { return min((gridDim.x - d + kXcds - 1u) / kXcds, kFixedPerDie); }
+    // the fixed first block of workgroup wg, or kInvalid (the same for every thread)
+    __device__ static uint32_t first(uint32_t wg, uint32_t nblk)
+    {
+        const uint32_t d = wg % kXcds, r = wg / kXcds, b0 = begin(nblk, d);
+        return r < kFixedPerDie && r < begin(nblk, d + 1) - b0 ? b0 + r : kInvalid;
+    }
     __device__ uint32_t next(uint32_t *q, uint32_t nblk)
     {
-        while (tries < kXcds) {
-            const uint32_t b0 = (uint32_t)(((uint64_t)nblk * die) / kXcds);
-            const uint32_t b1 = (uint32_t)(((uint64_t)nblk * (die + 1)) / kXcds);
-            const uint32_t t = atomicAdd(q + die * kQueueStride, 1u);
-            if (t < b1 - b0) return b0 + t;
+        while (open) {
+            if (open & (1u << die)) {
+                const uint32_t b0 = begin(nblk, die), cnt = begin(nblk, die + 1) - b0, fx = fixed(die);
+                if (cnt > fx) {
+                    const uint32_t t = fx + atomicAdd(q + die * kQueueStride, 1u);
+                    if (t < cnt) return b0 + t;
+                }
+                open &= ~(1u << die);
+                if (!helping) {
+                    // its own chunk is drained: one look at all counters tells which others are not
+                    helping = true;
+#pragma unroll
+                    for (uint32_t d = 0; d < kXcds; ++d) {
+                        const uint32_t c = begin(nblk, d + 1) - begin(nblk, d), f = fixed(d);
+                        if (c <= f || f + __hip_atomic_load(q + d * kQueueStride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= c)
+                            open &= ~(1u << d);
+                    }
+                }
+            }
             die = (die + 1) % kXcds;
-            ++tries;
         }
         return kInvalid;
     }
@@ -237,13 +252,13 @@ __device__ __forceinline__ bool quot_fast_ok(float h, float sx, float sy, float 
 
 // LIVE: the caller adds the pair's terms only for eps < dist < h (a listed neighbor that is not
 // coincident), so the zero the derivative takes outside that range is never read.
+// y = 1 / dist, correctly rounded (FAST); k2 = 2 k.
 template <bool FAST, bool LIVE = false>
-__device__ __forceinline__ void pair_quot(PairQuot &p, float dx, float dy, float dz, float dist, float h, float ih,
-                                          float k)
+__device__ __forceinline__ void pair_quot_y(PairQuot &p, float dx, float dy, float dz, float dist, float h, float ih,
+                                            float k2, float y)
 {
     float &nq = p.nq;
     if (FAST) {
-        const float y = frcp_exact(dist);
         p.nnx = fdiv_rcp_neg(dx, dist, y);
         p.nny = fdiv_rcp_neg(dy, dist, y);
         p.nnz = fdiv_rcp_neg(dz, dist, y);
@@ -255,9 +270,16 @@ __device__ __forceinline__ void pair_quot(PairQuot &p, float dx, float dy, float
         nq = -fdiv(dist, h);
     }
     p.omq = __fadd_rn(1.0f, nq);
-    const float num = __fmul_rn(__fmul_rn(2.0f, k), p.omq);
+    const float num = __fmul_rn(k2, p.omq);
     const float der = FAST ? fdiv_rcp_neg(num, h, ih) : -fdiv(num, h);
     p.der = LIVE ? der : ((dist <= kEps || dist >= h) ? 0.0f : der);
+}
+
+template <bool FAST, bool LIVE = false>
+__device__ __forceinline__ void pair_quot(PairQuot &p, float dx, float dy, float dz, float dist, float h, float ih,
+                                          float k)
+{
+    pair_quot_y<FAST, LIVE>(p, dx, dy, dz, dist, h, ih, __fmul_rn(2.0f, k), FAST ? frcp_exact(dist) : 0.0f);
 }
 
 struct DensitySelf {
@@ -266,42 +288,25 @@ struct DensitySelf {
     float h, t2, kw, ih;  // ih = 1 / h
     bool tension;
     bool fd;          // the neighbor quotients may use fdiv_rcp (pair_quot)
-    bool sup;         // candidate lists apply (fluid-only scene, tiled pass)
-    float ts2, allow; // candidate threshold; bound on D_i + D_j under which they stay complete
 };
 
 // Returns false (and writes the unreachable record) for particles that take no part in the solve.
-// sup_on: candidate lists apply to fluid-only scenes (only the fluid passes move their particles
-// within a substep, and they record every displacement).
 __device__ __forceinline__ bool density_begin(DensitySelf &x, uint32_t i, const float4 s, uint32_t ic,
-                                              const FluidArgs &a, bool sup_on = false)
+                                              const FluidArgs &a)
 {
     x.pc = a.classes[ic];
     x.s = s;
-    x.sup = false;
-    if (x.pc.kind != CN_PARTICLE_KIND_FLUID || s.w <= kEps) {
+    if (x.pc.kind != CN_PARTICLE_KIND_FLUID || s.w < 0.0f) {
         a.cs[i] = make_float4(kFarAway, kFarAway, kFarAway, 0.0f);
         return false;
     }
-    const cn_fluid_material &m = a.fm[x.pc.fluid_mat];
-    x.h = fmaxd(m.smoothing_radius, 1.0e-4f);
-    x.t2 = a.t2[x.pc.fluid_mat];
-    x.kw = spiky_coef(x.h);
-    x.ih = fdiv(1.0f, x.h);
+    const FluidConst fc = a.fc[x.pc.fluid_mat];
+    x.h = fc.h;
+    x.t2 = fc.t2;
+    x.kw = fc.kw;
+    x.ih = fc.ih;
     x.fd = quot_fast_ok(x.h, s.x, s.y, s.z);
-    x.tension = fmaxd(m.surface_tension, 0.0f) > kEps;
-    if (sup_on && a.scenes[x.pc.scene].fluid_only) {
-        // a pair j within h of particle i at iteration k was within h + D_i + D_j at iteration 0
-        // (D: displacement since iteration 0, x* to x* + delta), so the candidates within
-        // h + skin hold every later list while D_i + D_j < skin; D_j is bounded by the largest D in
-        // the block's halo, which holds all of i's 27 cells.  The margins cover the rounding of the
-        // squared distances (a few ulps) and of the recorded displacements.
-        const float skin = kSkinFrac * x.h;
-        const float hs = x.h + skin;
-        x.sup = true;
-        x.ts2 = hs * hs * 1.00001f;
-        x.allow = 0.98f * skin;
-    }
+    x.tension = fmaxd(a.fm[x.pc.fluid_mat].surface_tension, 0.0f) > kEps;
     return true;
 }
 
@@ -315,34 +320,33 @@ template <bool UNIFORM>
 __device__ __forceinline__ bool density_test(const DensitySelf &x, const float4 pj, uint32_t qcls, const FluidArgs &a)
 {
     if (!UNIFORM && !neighbor_ok(x.pc, a.classes[qcls])) return false;
-    if (pj.w <= kEps) return false;
+    if (pj.w < 0.0f) return false;
     const float dx = x.s.x - pj.x, dy = x.s.y - pj.y, dz = x.s.z - pj.z;
     return dot3(dx, dy, dz, dx, dy, dz) < x.t2;
 }
 
-// Density and (negated) surface-normal terms of one listed neighbor.
+// Density and (negated) surface-normal terms of one listed neighbor, and its squared distance.
 struct DensityTerm {
-    float w, ngx, ngy, ngz;
+    float w, ngx, ngy, ngz, d2;
 };
 
 // TENSION = false: the particle's material has no surface tension (x.tension false), so the normal
-// terms are left out at compile time.
-template <bool TENSION = true>
+// terms are left out at compile time.  FAST: quotients through reciprocals (x.fd holds).
+template <bool TENSION, bool FAST>
 __device__ __forceinline__ DensityTerm density_term(const DensitySelf &x, const float4 pj)
 {
     DensityTerm t;
     const float dx = x.s.x - pj.x, dy = x.s.y - pj.y, dz = x.s.z - pj.z;
-    const float dist = fsqrt_nearzero_free(dot3(dx, dy, dz, dx, dy, dz));
-    float omq = __fadd_rn(1.0f, fdiv_rcp_neg(dist, x.h, x.ih));  // 1 - dist / h
-    if (!x.fd) omq = __fsub_rn(1.0f, fdiv(dist, x.h));
+    t.d2 = dot3(dx, dy, dz, dx, dy, dz);
+    const float dist = fsqrt_nearzero_free(t.d2);
+    const float omq = FAST ? __fadd_rn(1.0f, fdiv_rcp_neg(dist, x.h, x.ih)) : __fsub_rn(1.0f, fdiv(dist, x.h));
     // every term the callers add is a neighbor's (dist < h): the kernel's range test is left out
     t.w = spiky_w_om_in(omq, x.kw);
     t.ngx = t.ngy = t.ngz = 0.0f;
     if (TENSION && x.tension && !(dist <= kEps || dist >= x.h)) {
         // FluidSpikyKernelGradient, physics_fluid_common.hlsli:44-53, negated: der * -(d / dist)
         PairQuot p;
-        pair_quot<true>(p, dx, dy, dz, dist, x.h, x.ih, x.kw);
-        if (!x.fd) pair_quot<false>(p, dx, dy, dz, dist, x.h, x.ih, x.kw);
+        pair_quot<FAST>(p, dx, dy, dz, dist, x.h, x.ih, x.kw);
         t.ngx = p.der * p.nnx;
         t.ngy = p.der * p.nny;
         t.ngz = p.der * p.nnz;
@@ -361,6 +365,41 @@ __device__ __forceinline__ void density_add(DensitySum &d, const DensitySelf &x,
     }
 }
 
+// Calls f(collider) for every candidate collider of a slot in visit order, for a wave whose
+// particles belong to one scene (colliders col0 .. col0 + ncol).  Candidates held as a bitmask are
+// taken collider by collider over the whole wave, so each is read once through the scalar cache
+// (the tables are constant during a launch); a lane-by-lane walk of the bits made every collider a
+// round trip of vector loads, some 3 us of a block's latency near a wall.
+__device__ __forceinline__ Collider const_collider(const Collider *col)
+{
+    typedef const __attribute__((address_space(4))) uint32_t *ConstWords;
+    const ConstWords w = (ConstWords)(uintptr_t)col;
+    union {
+        uint32_t u[sizeof(Collider) / 4];
+        Collider c;
+    } v;
+#pragma unroll
+    for (uint32_t k = 0; k < sizeof(Collider) / 4; ++k) v.u[k] = w[k];
+    return v.c;
+}
+template <class F>
+__device__ __forceinline__ void each_collider(uint32_t word, const FluidArgs &a, uint32_t i, uint32_t col0, F &&f)
+{
+    const bool listed = (word & kBndList) != 0u;
+    const uint16_t *l = a.bndl + (listed ? (size_t)i * kBndListCap : 0);
+    uint32_t left = listed ? min(word & 0xffu, kBndListCap) : word;  // entries left, or bits left
+    for (uint64_t any = __ballot(left != 0u); any; any = __ballot(left != 0u)) {
+        // the next candidate of the first lane with one left; every lane whose next it is takes it
+        const uint32_t mine = !left ? kInvalid : (listed ? (uint32_t)*l : (uint32_t)__builtin_ctz(left));
+        const uint32_t k = (uint32_t)__builtin_amdgcn_readlane((int)mine, (int)__builtin_ctzll(any));
+        if (mine == k) {
+            f(const_collider(a.col + __builtin_amdgcn_readfirstlane(col0) + k));
+            left = listed ? left - 1u : left & (left - 1u);
+            l += listed ? 1 : 0;
+        }
+    }
+}
+
 // Boundary ghost density (physics_fluid_boundary_common.hlsli:112-138), the constraint and the record.
 __device__ __forceinline__ void density_end(uint32_t i, uint32_t bw, const DensitySum &d, const DensitySelf &x,
                                             MetaAcc &ma, const FluidArgs &a, const SubstepConsts &c)
@@ -368,10 +407,11 @@ __device__ __forceinline__ void density_end(uint32_t i, uint32_t bw, const Densi
     float density = d.density;
     const float bscale = c.cfg[kCfgFluidBndDensity];
     const uint32_t col0 = a.scenes[x.pc.scene].col0;
-    each_candidate(bw, a.bndl, i, [&](uint32_t k) {
+    each_collider(bw, a, i, col0, [&](const Collider &cc) {
         float gx, gy, gz;
-        if (!ghost_delta(a.col[col0 + k], x.s.x, x.s.y, x.s.z, x.h, gx, gy, gz)) return;
-        const float gd = len3(gx, gy, gz);
+        if (!ghost_delta(cc, x.s.x, x.s.y, x.s.z, x.h, gx, gy, gz)) return;
+        float ux, uy, uz;
+        const float gd = len3_dir(gx, gy, gz, ux, uy, uz);
         if (gd >= x.h) return;
         density = density + spiky_w_k(gd, x.h, x.kw) * bscale;
     });
@@ -408,7 +448,7 @@ __device__ __forceinline__ void density_global(uint32_t i, MetaAcc &ma, const Fl
             ++d.req;
             if (d.inr < c.cap) {
                 ++d.inr;
-                density_add(d, x, density_term(x, pj));
+                density_add(d, x, density_term<true, false>(x, pj));
             }
             return true;
         });
@@ -439,11 +479,12 @@ struct DeltaSelf {
     float4 di, nci;
     float sx, sy, sz, Ci, h, t2, kw, ih, cohesion, viscosity, cfl, dt;
     bool tension, visc_on, cfl_on, need_rel, fd;
+    bool plain;  // no cohesion, viscosity, CFL or tension term: the pressure term alone (delta_plain)
 };
 
 struct DeltaTerm {
     float x, y, z;
-    bool live;  // the neighbor is not coincident (dist > eps): it adds a term and a weight
+    bool live;  // a neighbor (dist < h) that is not coincident (dist > eps): it adds a term and a weight
 };
 
 // One listed neighbor's term (physics_fluid_compute_delta_positions.cs.hlsl:60-140).
@@ -453,8 +494,9 @@ __device__ __forceinline__ DeltaTerm delta_term(const DeltaSelf &x, const float4
 {
     DeltaTerm t;
     const float ddx = x.sx - cq.x, ddy = x.sy - cq.y, ddz = x.sz - cq.z;
-    const float dist = fsqrt_nearzero_free(dot3(ddx, ddy, ddz, ddx, ddy, ddz));
-    t.live = !(dist <= kEps);
+    const float d2 = dot3(ddx, ddy, ddz, ddx, ddy, ddz);
+    const float dist = fsqrt_nearzero_free(d2);
+    t.live = d2 < x.t2 && !(dist <= kEps);
     PairQuot p;
     // a listed neighbor (dist < h) whose term counts only when live (dist > eps)
     pair_quot<true, true>(p, ddx, ddy, ddz, dist, x.h, x.ih, x.kw);
@@ -537,17 +579,15 @@ __device__ __forceinline__ DeltaPre delta_pre(uint32_t i, const FluidArgs &a, ui
     return r;
 }
 
-// sum(x, d) adds the neighbor terms in list order.  own addresses the particle's record in
-// rcs / rnc (LDS offset or slot).  Returns (|delta| + slack)^2 of the particle.
-template <bool UNIFORM, class Sum>
-__device__ __forceinline__ float delta_particle(uint32_t i, uint32_t own, const DeltaPre &pre, Sum &&sum,
-                                                const float4 *rcs, const float4 *rnc, const FluidArgs &a,
-                                                const SubstepConsts &c)
+// sum(x, d) adds the neighbor terms in list order; own(nc) is the particle's record, or its surface
+// normal's.  Returns (|delta| + slack)^2 of the particle.
+template <bool UNIFORM, class Sum, class Own>
+__device__ __forceinline__ float delta_particle(uint32_t i, const DeltaPre &pre, Sum &&sum, Own &&own,
+                                                const FluidArgs &a, const SubstepConsts &c)
 {
     const ParticleClass pc = a.classes[pre.cls];
     if (pc.kind != CN_PARTICLE_KIND_FLUID) {
         a.dout[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (a.disp) a.disp[i] = 0.0f;
         return 0.0f;
     }
     const float4 p = pre.p;
@@ -557,16 +597,17 @@ __device__ __forceinline__ float delta_particle(uint32_t i, uint32_t own, const 
         DeltaSelf x;
         x.pc = pc;
         x.di = di;
-        const float4 csi = rcs[own];
+        const float4 csi = own(false);
         x.sx = csi.x;
         x.sy = csi.y;
         x.sz = csi.z;
         x.Ci = csi.w;
         const cn_fluid_material &m = a.fm[pc.fluid_mat];
-        x.h = fmaxd(m.smoothing_radius, 1.0e-4f);
-        x.t2 = a.t2[pc.fluid_mat];
-        x.kw = spiky_coef(x.h);
-        x.ih = fdiv(1.0f, x.h);
+        const FluidConst fc = a.fc[pc.fluid_mat];
+        x.h = fc.h;
+        x.t2 = fc.t2;
+        x.kw = fc.kw;
+        x.ih = fc.ih;
         x.fd = quot_fast_ok(x.h, x.sx, x.sy, x.sz);
         x.dt = c.dt;
         x.cohesion = c.dt * fmaxd(m.cohesion, 0.0f);
@@ -576,22 +617,24 @@ __device__ __forceinline__ float delta_particle(uint32_t i, uint32_t own, const 
         x.cfl_on = cfl_term_on(m, a, c);
         x.visc_on = visc_term_on(m, a, c);
         x.need_rel = x.cfl_on || x.visc_on;
-        x.nci = x.tension ? rnc[own] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        x.plain = !(x.need_rel || x.tension || x.cohesion > kEps);
+        x.nci = x.tension ? own(true) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         DeltaSum d;
         if (c.cap > 0 && (!UNIFORM || neighbor_ok(pc, pc))) sum(x, d);
         // ComputeFluidBoundaryDeltaFromCandidates, physics_fluid_boundary_common.hlsli:140-167
         float bx = 0.0f, by = 0.0f, bz = 0.0f;
         const float scn = fmaxd(x.Ci, 0.0f);
         const uint32_t col0 = a.scenes[pc.scene].col0;
-        each_candidate(pre.bnd, a.bndl, i, [&](uint32_t k) {
+        each_collider(pre.bnd, a, i, col0, [&](const Collider &cc) {
             float gx, gy, gz;
-            if (!ghost_delta(a.col[col0 + k], x.sx, x.sy, x.sz, x.h, gx, gy, gz)) return;
-            const float gd = len3(gx, gy, gz);
+            if (!ghost_delta(cc, x.sx, x.sy, x.sz, x.h, gx, gy, gz)) return;
+            float ux, uy, uz;
+            const float gd = len3_dir(gx, gy, gz, ux, uy, uz);
             if (gd <= kEps || gd >= x.h) return;
             const float f = -scn * spiky_dw_k(gd, x.h, x.kw);
-            bx = bx + f * fdiv(gx, gd);
-            by = by + f * fdiv(gy, gd);
-            bz = bz + f * fdiv(gz, gd);
+            bx = bx + f * ux;
+            by = by + f * uy;
+            bz = bz + f * uz;
         });
         const float solve = c.cfg[kCfgFluidSolve], bdel = c.cfg[kCfgFluidBndDelta];
         ox = d.x * solve + bx * bdel;
@@ -609,9 +652,9 @@ __device__ __forceinline__ float delta_particle(uint32_t i, uint32_t own, const 
     const uint32_t bcol0 = a.scenes[pc.scene].col0;
     for (int sweep = 0; sweep < 2; ++sweep) {
         bool changed = false;
-        each_candidate(bw, a.bndl, i, [&](uint32_t k) {
+        each_collider(bw, a, i, bcol0, [&](const Collider &cc) {
             float sd, nx, ny, nz;
-            if (!collider_contact(a.col[bcol0 + k], cx, cy, cz, sd, nx, ny, nz)) return;
+            if (!collider_contact(cc, cx, cy, cz, sd, nx, ny, nz)) return;
             if (sd >= r) return;
             const float push = r - sd;
             cx = cx + nx * push;
@@ -624,41 +667,42 @@ __device__ __forceinline__ float delta_particle(uint32_t i, uint32_t own, const 
     const float ex = cx - p.x, ey = cy - p.y, ez = cz - p.z;
     a.dout[i] = make_float4(ex, ey, ez, 0.0f);
     const float nx = p.x + ex, ny = p.y + ey, nz = p.z + ez;
-    a.cur[i] = make_float4(nx, ny, nz, p.w);
-    // |delta| plus a few ulps of the position: bounds the next iteration's relDelta for the CFL skip
+    // |delta| plus a few ulps of the position: D, the bound on the displacement since iteration 0
+    // that the candidate lists go by; it also bounds the next iteration's relDelta for the CFL skip
     const float slack = fmaxd(fmaxd(fabsf(nx), fabsf(ny)), fabsf(nz)) * 4.76837158e-7f + 1.0e-30f;
     const float dl = len3(ex, ey, ez) + slack;
-    if (a.disp) a.disp[i] = dl;
+    a.cur[i] = make_float4(nx, ny, nz, p.w > kEps ? dl : kNoMass);
     return dl * dl;
 }
 
-// Run-table walk: the list filter and the cap applied in the walk.
+// The terms over the run table: the list filter and the cap applied in the walk.
 template <bool UNIFORM>
-__device__ __forceinline__ float delta_global(uint32_t i, const FluidArgs &a, const SubstepConsts &c,
-                                              uint32_t ucls = 0u)
+__device__ __forceinline__ void delta_walk(uint32_t i, const DeltaSelf &x, DeltaSum &d, const FluidArgs &a,
+                                           const SubstepConsts &c)
 {
-    if (!a.active[a.classes[UNIFORM ? ucls : a.cls[i]].scene]) return 0.0f;
-    const int4 ci = a.cellc[i];
     const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    uint32_t inr = 0;
+    walk_runs(a.cellc[i], run_table(a), c, [&](uint32_t q) {
+        if (q == i) return true;
+        const uint32_t qc = UNIFORM ? 0u : a.cls[q];
+        if (!UNIFORM && !neighbor_ok(x.pc, a.classes[qc])) return true;
+        const float4 cq = a.cs[q];
+        const float ddx = x.sx - cq.x, ddy = x.sy - cq.y, ddz = x.sz - cq.z;
+        if (!(dot3(ddx, ddy, ddz, ddx, ddy, ddz) < x.t2)) return true;
+        if (inr >= c.cap) return false;
+        ++inr;
+        delta_add(d, delta_term<UNIFORM>(x, cq, x.need_rel ? a.din[q] : zero, x.tension ? a.nc[q] : zero, qc, a));
+        return true;
+    });
+}
+
+template <bool UNIFORM>
+__device__ __forceinline__ float delta_global(uint32_t i, const FluidArgs &a, const SubstepConsts &c)
+{
+    if (!a.active[a.classes[UNIFORM ? 0u : a.cls[i]].scene]) return 0.0f;
     return delta_particle<UNIFORM>(
-        i, i, delta_pre<UNIFORM>(i, a, ucls),
-        [&](const DeltaSelf &x, DeltaSum &d) {
-            uint32_t inr = 0;
-            walk_runs(ci, run_table(a), c, [&](uint32_t q) {
-                if (q == i) return true;
-                const uint32_t qc = UNIFORM ? 0u : a.cls[q];
-                if (!UNIFORM && !neighbor_ok(x.pc, a.classes[qc])) return true;
-                const float4 cq = a.cs[q];
-                const float ddx = x.sx - cq.x, ddy = x.sy - cq.y, ddz = x.sz - cq.z;
-                if (!(dot3(ddx, ddy, ddz, ddx, ddy, ddz) < x.t2)) return true;
-                if (inr >= c.cap) return false;
-                ++inr;
-                delta_add(d, delta_term<UNIFORM>(x, cq, x.need_rel ? a.din[q] : zero, x.tension ? a.nc[q] : zero, qc,
-                                                 a));
-                return true;
-            });
-        },
-        a.cs, a.nc, a, c);
+        i, delta_pre<UNIFORM>(i, a), [&](const DeltaSelf &x, DeltaSum &d) { delta_walk<UNIFORM>(i, x, d, a, c); },
+        [&](bool nc) { return nc ? a.nc[i] : a.cs[i]; }, a, c);
 }
 
 __device__ __forceinline__ void flush_disp(float d2, const FluidArgs &a)
@@ -759,6 +803,8 @@ __global__ __launch_bounds__(kBlock) void k_blk_halo(FluidArgs a, SubstepConsts 
                 a.wide_blk[atomicAdd(a.iter_state + kStateWideCount, 1u)] = b;
             hd[kHdOff + kHalo] = total;
             hd[kHdFlags] = any_bad ? 0u : 1u;
+            hd[kHdFluidOnly] = a.scenes[scene].fluid_only;
+            hd[kHdSuper] = 1u;  // the building density pass clears it where a candidate list overflows
             hd[kHdPairs] = (s_kinds & kHasOther) || (s_kinds & (kHasFluid | kHasSolid)) == (kHasFluid | kHasSolid) ||
                                    ((s_kinds & kHasSolid) && s_gmin != s_gmax)
                                ? 1u
@@ -774,67 +820,91 @@ __global__ __launch_bounds__(kBlock) void k_blk_halo(FluidArgs a, SubstepConsts 
 }
 
 constexpr int kTileBlock = 512;  // threads of a tiled fluid workgroup: one pass over a block's particles
-// waves per SIMD the tiled passes are compiled for (at most 80 VGPRs): three 8-wave workgroups per
-// CU, which their LDS budget (kDynLdsBytes) also allows
-constexpr int kTileWaves = 6;
-constexpr uint32_t kTermStep = 4;  // listed neighbors whose loads are issued together in the term loops
-constexpr uint32_t kDeltaStep = 4;  // the same in the delta pass
+// Waves per SIMD the tiled passes are compiled for.  The density pass fits 80 VGPRs with a few values
+// spilled between blocks: three 8-wave workgroups per CU, each a third of its LDS.  The delta pass
+// holds more across its term loops (its spills there cost three times the time: 1,320 us at six
+// waves with the terms unrolled by four) and runs two workgroups with half the LDS each, which also
+// stages larger halos.
+constexpr int kDensityWaves = 6, kDeltaWaves = 4;
 constexpr uint32_t kTilePad = 4;   // spare entries after each staged density array (walk loads past a range)
 
-// Common head of the tiled passes: claim a block (next() runs on thread 0), decide LDS or run
-// table, load the halo table.  skip_to is a halo size above the LDS capacity up to which a block is
-// left to the wide launch (0: none).
+// Head of a tiled pass's block: decide LDS or run table, load the halo table (visible after the
+// caller's barrier).  skip_to is a halo size above the LDS capacity up to which a block is left to
+// the wide launch (0: none).  b is the same for the whole workgroup.
 struct TileState {
     uint32_t blk;
     uint32_t p0, p1;
     bool lds, skip;
+    bool fluid_only;  // the block's scene
+    bool complete;    // every particle of the block has a complete candidate list
     int bx, by, bz;
 };
 
-template <class Next>
-__device__ __forceinline__ bool tile_begin(Next &&next, uint32_t *s_blk, uint32_t *hoff, uint32_t *hstart,
-                                           TileState &ts, uint32_t skip_to, const FluidArgs &a,
-                                           const SubstepConsts &c)
+__device__ __forceinline__ void tile_load(TileState &ts, uint32_t b, uint32_t *hoff, uint32_t *hstart,
+                                          uint32_t skip_to, const FluidArgs &a, const SubstepConsts &c)
 {
     const uint32_t tid = threadIdx.x;
-    if (tid == 0) *s_blk = next();
-    __syncthreads();
-    const uint32_t b = *s_blk;
-    if (b == kInvalid) return false;
+    b = __builtin_amdgcn_readfirstlane(b);
     ts.blk = b;
     ts.lds = false;
     ts.skip = false;
     if (b < c.blk_cap) {
         const uint32_t *hd = a.blk_halo + (size_t)b * kHaloStride;
+        // the tables are loaded beside the header, whatever it says
+        for (uint32_t t = tid; t <= kHalo; t += blockDim.x) {
+            hoff[t] = hd[kHdOff + t];
+            if (t < kHalo) hstart[t] = hd[kHdStart + t];
+        }
         ts.p0 = hd[kHdP0];
         ts.p1 = hd[kHdP1];
-        if (!a.active[hd[kHdScene]] || hd[kHdFlags] == kHdNoFluid) {  // untouched this step, or no fluid
-            ts.skip = true;
-            __syncthreads();
-            return true;
-        }
-        const uint32_t total = hd[kHdOff + kHalo];
-        const bool pure = hd[kHdFlags] != 0u;
-        ts.lds = pure && total <= a.tile;
-        ts.skip = pure && !ts.lds && total <= skip_to;
-        if (ts.lds) {
-            for (uint32_t t = tid; t < kHalo; t += blockDim.x) {
-                hstart[t] = hd[kHdStart + t];
-                hoff[t] = hd[kHdOff + t];
-            }
-            if (tid == 0) hoff[kHalo] = hd[kHdOff + kHalo];
-            ts.bx = (int)hd[kHdBase];
-            ts.by = (int)hd[kHdBase + 1];
-            ts.bz = (int)hd[kHdBase + 2];
-        }
+        ts.bx = (int)hd[kHdBase];
+        ts.by = (int)hd[kHdBase + 1];
+        ts.bz = (int)hd[kHdBase + 2];
+        const uint32_t total = hd[kHdOff + kHalo], flags = hd[kHdFlags];
+        const uint32_t scene = hd[kHdScene];
+        ts.fluid_only = hd[kHdFluidOnly] != 0u;
+        ts.complete = hd[kHdSuper] != 0u;
+        ts.skip = flags == kHdNoFluid || (!c.all_active && !a.active[scene]);  // no fluid, or untouched this step
+        const bool pure = flags != 0u;
+        ts.lds = !ts.skip && pure && total <= a.tile;
+        ts.skip |= pure && !ts.lds && total <= skip_to;
     } else {
         ts.p0 = a.run_start[a.blk_first_run[b]];
         ts.p1 = a.run_start[a.blk_first_run[b + 1]];
         const uint32_t scene = a.classes[a.cls[ts.p0]].scene;
         ts.skip = !a.active[scene] || !a.scenes[scene].has_fluid;
+        ts.fluid_only = ts.complete = false;
     }
-    __syncthreads();
-    return true;
+}
+
+// Stages the halo: eight lanes per cell, so a cell's records are read as one 128-byte line and each
+// thread knows its cells without a search; load(u, slot) issues the loads of four cells' records
+// before put(u, staged index, slot) stores any.  (A thread per staged record found its cell by an
+// eight-step binary search of LDS per record, about 1 us of a block's latency.)
+constexpr uint32_t kStageCells = 4;
+template <class Load, class Put>
+__device__ __forceinline__ void stage_halo(const uint32_t *hoff, const uint32_t *hstart, Load &&load, Put &&put)
+{
+    const uint32_t ln = threadIdx.x & 7u, grp = threadIdx.x >> 3, ngrp = blockDim.x >> 3;
+    for (uint32_t c0 = grp; c0 < kHalo; c0 += kStageCells * ngrp) {
+        uint32_t o[kStageCells], n[kStageCells], s[kStageCells], most = 0;
+#pragma unroll
+        for (uint32_t u = 0; u < kStageCells; ++u) {
+            const uint32_t hc = c0 + u * ngrp, h = min(hc, kHalo - 1u);
+            o[u] = hoff[h];
+            n[u] = hc < kHalo ? hoff[h + 1] - o[u] : 0u;
+            s[u] = hstart[h];
+            most = max(most, n[u]);
+        }
+        for (uint32_t k = ln; k < most; k += 8) {
+            // past a cell's end its last record is loaded (of an empty cell slot 0), and not stored
+#pragma unroll
+            for (uint32_t u = 0; u < kStageCells; ++u) load(u, s[u] + min(k, n[u] - min(n[u], 1u)));
+#pragma unroll
+            for (uint32_t u = 0; u < kStageCells; ++u)
+                if (k < n[u]) put(u, o[u] + k, s[u] + k);
+        }
+    }
 }
 
 __device__ __forceinline__ int halo_cell(const TileState &ts, const int4 ci)
@@ -848,8 +918,7 @@ __device__ __forceinline__ int halo_cell(const TileState &ts, const int4 ci)
 
 // The density walk over the staged halo: tests every candidate in walk order and compacts those
 // within the radius (squared distance below thr2: the neighbor threshold t2, or ts2 for the
-// candidate list of a substep) as halo offsets into a list, four candidates per step with their
-// LDS loads issued first.  Returns the untruncated count.  Staged particles with zero inverse mass
+// candidate list of a substep) as halo offsets into a list.  Staged particles with zero inverse mass
 // carry an unreachable position, so the distance test also rejects them.
 //
 // Cells that no candidate inside can reach are left out of the walk (the order of the others is
@@ -881,29 +950,29 @@ __device__ __forceinline__ RowCull row_cull(const float4 s, const int4 ci, float
 __device__ __forceinline__ float gap_below(float u, int c) { return fmaxd(u - (float)c, 0.0f); }
 __device__ __forceinline__ float gap_above(float u, int c) { return fmaxd((float)(c + 1) - u, 0.0f); }
 
-// A particle's list in a grouped list buffer (list_entry_base): the buffer (a kernel argument, so a
-// scalar base) and the byte offset of entry 0; entry k sits 2 * kListGroup * k bytes further.  The
-// offsets are 32-bit (list buffers stay below 4 GiB), so an address is one 32-bit add from the base.
-constexpr uint32_t kEntryStride = 2u * kListGroup;
-struct ListRef {
-    char *base;
-    uint32_t off;
-    __device__ __forceinline__ uint16_t &entry(uint32_t k) const
-    {
-        return *reinterpret_cast<uint16_t *>(base + (off + k * kEntryStride));
-    }
-};
-
-__device__ __forceinline__ ListRef list_ref(uint16_t *buf, uint32_t i, uint32_t rows)
+// A particle's list in a grouped list buffer: words of four entries, word w kWordStride words after
+// word 0, so a wave reads or writes 512 consecutive bytes per word.  (Single 16-bit entries took
+// four loads per step of the term loops; their stores, one per push, made every wait for a load a
+// wait for the stores before it too.)
+constexpr uint32_t kWordStride = kListGroup;
+__device__ __forceinline__ uint2 *list_words(uint16_t *buf, uint32_t i, uint32_t rows)
 {
-    return ListRef{reinterpret_cast<char *>(buf), (uint32_t)list_entry_base(i, rows)};
+    return reinterpret_cast<uint2 *>(reinterpret_cast<char *>(buf) + list_word_base(i, rows));
 }
 
+// What a pass keeps per particle about its list: the staged entry of the particle itself, where the
+// entries are (kInList: the neighbor list, else the candidate list), and the words (kSuperNone: the
+// candidates did not fit).
+constexpr uint32_t kInList = 0x8000u, kSuperNone = 0x7fffu, kWordsMask = 0x7fffu;
+__device__ __forceinline__ uint32_t list_word(uint32_t entry, uint32_t words) { return (entry << 16) | words; }
+
 // List entries are byte offsets into a staged array of 16-byte records (halo index x 16; the tile
-// holds at most 4,096 halo particles, so they fit 16 bits), so the LDS address of a listed
-// neighbor's record needs no scaling; staged arrays of 4-byte items take the entry / 4.
+// holds at most kTileMost halo particles, so they fit 16 bits), so the LDS address of a listed
+// neighbor's record needs no scaling; staged arrays of 4-byte items take the entry / 4.  A list's
+// last word is filled up with the entry after the halo's last particle, which holds a record no
+// particle is within any radius of: a word's four entries need no test against the list's length.
 constexpr uint32_t kEntryScale = 16;
-static_assert(4096u * kEntryScale <= 65536u, "a byte-offset entry of the largest tile fits 16 bits");
+static_assert(kTileMost * kEntryScale <= 65535u, "the filling entry of the largest tile fits 16 bits");
 template <class T>
 __device__ __forceinline__ const T &at16(const T *base, uint32_t e)
 {
@@ -915,66 +984,105 @@ __device__ __forceinline__ uint32_t at4(const uint32_t *base, uint32_t e)
     return *reinterpret_cast<const uint32_t *>(reinterpret_cast<const char *>(base) + (e >> 2));
 }
 
-// Appends listed halo offsets to a particle's list, storing the first cap.  The write position is
-// the byte offset of the next entry and advances one entry stride per push, so a push is a compare,
-// a store and an add; n() is the untruncated count.  The position may run past entry cap by one
-// stride per walked candidate (at most the tile, 2^12 entries: 512 KiB), which the list buffer's
-// limit leaves room for below 4 GiB.
+// Appends halo offsets to a particle's list, keeping the first cap: four are collected in a register
+// pair, which is stored when full.  n counts all.
 struct ListOut {
-    char *base;
-    uint32_t a0, a, lim;  // byte offsets of entry 0, the next entry and entry cap
-    __device__ __forceinline__ ListOut(const ListRef &r, uint32_t cap)
-        : base(r.base), a0(r.off), a(r.off), lim(r.off + cap * kEntryStride)
+    uint2 *p;
+    uint32_t cap, n, lo, hi;
+    __device__ __forceinline__ ListOut(uint2 *words, uint32_t cap_) : p(words), cap(cap_), n(0), lo(0), hi(0) {}
+    __device__ __forceinline__ void shift_in(uint32_t e)
     {
+        lo = __builtin_amdgcn_alignbit(hi, lo, 16);
+        hi = __builtin_amdgcn_alignbit(e, hi, 16);
     }
-    __device__ __forceinline__ void push(uint32_t f)
+    __device__ __forceinline__ void push(uint32_t e)
     {
-        if (a < lim) *reinterpret_cast<uint16_t *>(base + a) = (uint16_t)f;
-        a += kEntryStride;
+        if (n < cap) {
+            shift_in(e);
+            if ((n & 3u) == 3u) {
+                *p = make_uint2(lo, hi);
+                p += kWordStride;
+            }
+        }
+        ++n;
     }
-    __device__ __forceinline__ uint32_t n() const { return (a - a0) / kEntryStride; }
+    // fills the last word; returns the words
+    __device__ __forceinline__ uint32_t finish(uint32_t fill)
+    {
+        const uint32_t m = min(n, cap), r = m & 3u;
+        if (r) {
+            for (uint32_t u = r; u < 4u; ++u) shift_in(fill);
+            *p = make_uint2(lo, hi);
+        }
+        return (m + 3u) >> 2;
+    }
 };
 
-// One contiguous range [k, f1) of the walk, four candidates per step: the loads read through a
-// pointer with immediate offsets and may run up to three entries past f1 (the staged arrays carry
-// kTilePad spare entries), which the u < f1 - k test then drops.
+// f(word) for each of a list's words (>= 1), two words ahead of use.  Past the end it reads up to
+// two words that belong to the slot group's next rows or to the buffer's spare rows.
+template <class F>
+__device__ __forceinline__ void each_word(const uint2 *p, uint32_t words, F &&f)
+{
+    uint2 w0 = p[0], w1 = p[kWordStride];
+    for (; words; --words) {
+        const uint2 e = w0;
+        w0 = w1;
+        w1 = p[2 * kWordStride];
+        p += kWordStride;
+        f(e);
+    }
+}
+__device__ __forceinline__ void word_entries(uint2 w, uint32_t (&e)[4])
+{
+    e[0] = w.x & 0xffffu;
+    e[1] = w.x >> 16;
+    e[2] = w.y & 0xffffu;
+    e[3] = w.y >> 16;
+}
+
+// Up to 32 candidates [k, f1) of a walked row: first every candidate's squared distance is tested and
+// the outcome shifted into a bit mask, without a branch (four candidates per step; the loads may run
+// up to three entries past f1, for which the staged arrays carry kTilePad spare entries), then the
+// few that passed are pushed in order.  skip is the staged index of a candidate to leave out (the
+// particle itself; any index outside the range leaves none out).  (Testing and pushing candidate by
+// candidate spent some 40 cycles of a lone wave's latency on each of the three branches of a push,
+// whether or not it happened: 21 us of a 34 us launch over the dam break's 64,000 particles.)
 template <bool UNIFORM>
-__device__ __forceinline__ void scan_range(uint32_t k, uint32_t f1, const float4 *lpos, const uint32_t *lcls,
-                                           const DensitySelf &x, float thr2, const FluidArgs &a, ListOut &lo)
+__device__ __forceinline__ void scan_range(uint32_t k, uint32_t f1, uint32_t skip, const float4 *lpos,
+                                           const uint32_t *lcls, const DensitySelf &x, float thr2, const FluidArgs &a,
+                                           ListOut &lo)
 {
     const float4 *pp = lpos + k;
-    const uint32_t *pc = lcls + k;
-    uint32_t kb = k * kEntryScale;  // the entry of candidate k
-    for (; k < f1; k += 4, kb += 4 * kEntryScale, pp += 4, pc += 4) {
+    const uint32_t n = f1 - k;  // 1 .. 32
+    uint32_t mask = 0, done = 0;
+    for (; done < n; done += 4, pp += 4) {
         float4 pj[4];
-        uint32_t qc[4];
 #pragma unroll
-        for (uint32_t u = 0; u < 4; ++u) {
-            pj[u] = pp[u];
-            qc[u] = UNIFORM ? 0u : pc[u];
-        }
-        const uint32_t rem = f1 - k;  // >= 1
+        for (uint32_t u = 0; u < 4; ++u) pj[u] = pp[u];
 #pragma unroll
         for (uint32_t u = 0; u < 4; ++u) {
             const float dx = x.s.x - pj[u].x, dy = x.s.y - pj[u].y, dz = x.s.z - pj[u].z;
-            const float d2 = dot3(dx, dy, dz, dx, dy, dz);
-            bool cand = (d2 < thr2) & (u == 0 || u < rem);
-            if (!UNIFORM) cand = cand && neighbor_ok(x.pc, a.classes[qc[u]]);
-            if (cand) lo.push(kb + u * kEntryScale);
+            mask = (mask << 1) | (dot3(dx, dy, dz, dx, dy, dz) < thr2 ? 1u : 0u);
         }
+    }
+    mask <<= 32u - done;           // bit 31: the first candidate
+    mask &= 0xffffffffu << (32u - n);
+    if (skip - k < n) mask &= ~(0x80000000u >> (skip - k));
+    while (mask) {
+        const uint32_t j = (uint32_t)__builtin_clz(mask);
+        mask &= ~(0x80000000u >> j);
+        if (!UNIFORM && !neighbor_ok(x.pc, a.classes[lcls[k + j]])) continue;
+        lo.push((k + j) * kEntryScale);
     }
 }
 
 template <bool UNIFORM>
-__device__ __forceinline__ uint32_t scan_rows(const uint32_t *hoff, int hc, uint32_t fs, const float4 *lpos,
-                                              const uint32_t *lcls, const DensitySelf &x, float thr2,
-                                              const ListRef &li, uint32_t cap, const FluidArgs &a,
-                                              const RowCull &rc)
+__device__ __forceinline__ void scan_rows(const uint32_t *hoff, int hc, uint32_t fs, const float4 *lpos,
+                                          const uint32_t *lcls, const DensitySelf &x, float thr2,
+                                          ListOut &lo, const FluidArgs &a, const RowCull &rc)
 {
-    ListOut lo(li, cap);
     const float gxl = gap_below(rc.ux, rc.cx), gxr = gap_above(rc.ux, rc.cx);
-    // rows of three cells along x, z outer, y inner; the centre row (r = 4) is walked as the
-    // ranges before and after the particle itself
+    // rows of three cells along x, z outer, y inner
 #pragma unroll 1
     for (int r = 0; r < 9; ++r) {
         const int ry = r % 3 - 1, rz = r / 3 - 1;
@@ -984,84 +1092,124 @@ __device__ __forceinline__ uint32_t scan_rows(const uint32_t *hoff, int hc, uint
         if (!(perp < rc.lim2)) continue;
         const int h0 = hc - 1 + 6 * ry + 36 * rz;
         const uint32_t f1 = hoff[h0 + (gxr * gxr + perp < rc.lim2 ? 3 : 2)];
-        const uint32_t k0 = hoff[h0 + (gxl * gxl + perp < rc.lim2 ? 0 : 1)];
-        if (r == 4) {
-            scan_range<UNIFORM>(k0, fs, lpos, lcls, x, thr2, a, lo);
-            scan_range<UNIFORM>(fs + 1, f1, lpos, lcls, x, thr2, a, lo);
-        } else {
-            scan_range<UNIFORM>(k0, f1, lpos, lcls, x, thr2, a, lo);
-        }
+        for (uint32_t k = hoff[h0 + (gxl * gxl + perp < rc.lim2 ? 0 : 1)]; k < f1; k += 32u)
+            scan_range<UNIFORM>(k, min(f1, k + 32u), fs, lpos, lcls, x, thr2, a, lo);
     }
-    return lo.n();
 }
 
-// List entries k .. k + kTermStep - 1 of a list of cnt >= 1 entries (the last one repeated past
-// the end, so the LDS reads they drive stay in range).
-template <uint32_t N>
-__device__ __forceinline__ void list_group(const ListRef &li, uint32_t k, uint32_t cnt, uint32_t (&e)[N])
+// The density terms of the listed particles within the neighbor radius at the current positions, in
+// list order; every lane evaluates each term before the test decides whether it is added.  d.req
+// counts the neighbors.
+template <bool TENSION, bool FAST>
+__device__ __forceinline__ void density_words(const uint2 *p, uint32_t words, const float4 *lpos, const DensitySelf &x,
+                                              DensitySum &d)
 {
+    if (!words) return;
+    each_word(p, words, [&](uint2 w) {
+        uint32_t e[4];
+        word_entries(w, e);
+        float4 pj[4];
 #pragma unroll
-    for (uint32_t u = 0; u < N; ++u) e[u] = li.entry(min(k + u, cnt - 1));
-}
-
-// The neighbors from the substep's candidate list (complete at iteration 0, and later while the
-// displacements stay under the skin, checked by the caller): the in-radius test at the current
-// positions, the listed neighbors written to the list in candidate order (= walk order), and the
-// density terms of the first cap summed in the same pass.  A step's four candidates are loaded first; each term is then
-// evaluated before the test decides whether it is added, so every lane runs the same instructions.
-// (Filtering first and summing over the written list afterwards measured slower.)  Returns the
-// untruncated neighbor count.
-template <bool TENSION>
-__device__ __forceinline__ uint32_t density_super(const ListRef &ls, uint32_t scount, const float4 *lpos,
-                                                  const DensitySelf &x, const ListRef &li, uint32_t cap,
-                                                  DensitySum &d)
-{
-    ListOut lo(li, cap);
-    uint32_t en[kTermStep];
-    list_group(ls, 0, scount, en);
-    for (uint32_t k = 0; k < scount; k += kTermStep) {
-        float4 pj[kTermStep];
-        uint32_t e[kTermStep];
+        for (uint32_t u = 0; u < 4; ++u) pj[u] = at16(lpos, e[u]);
 #pragma unroll
-        for (uint32_t u = 0; u < kTermStep; ++u) {
-            e[u] = en[u];
-            pj[u] = at16(lpos, e[u]);
+        for (uint32_t u = 0; u < 4; ++u) {
+            const DensityTerm t = density_term<TENSION, FAST>(x, pj[u]);
+            if (t.d2 < x.t2) {
+                ++d.req;
+                density_add<TENSION>(d, x, t);
+            }
         }
-        // the next step's entries while this step's terms are evaluated
-        list_group(ls, k + kTermStep, scount, en);
-#pragma unroll
-        for (uint32_t u = 0; u < kTermStep; ++u) {
-            const DensityTerm t = density_term<TENSION>(x, pj[u]);
-            const float dx = x.s.x - pj[u].x, dy = x.s.y - pj[u].y, dz = x.s.z - pj[u].z;
-            if ((k + u < scount) & (dot3(dx, dy, dz, dx, dy, dz) < x.t2)) {
-                if (lo.a < lo.lim) density_add<TENSION>(d, x, t);
+    });
+}
+
+__device__ __forceinline__ void density_sums(const uint2 *p, uint32_t words, const float4 *lpos, const DensitySelf &x,
+                                             DensitySum &d)
+{
+    // one vote per particle instead of a test per term
+    const bool fast = __all(x.fd);
+    if (x.tension) {
+        if (fast) density_words<true, true>(p, words, lpos, x, d);
+        else density_words<true, false>(p, words, lpos, x, d);
+    } else {
+        if (fast) density_words<false, true>(p, words, lpos, x, d);
+        else density_words<false, false>(p, words, lpos, x, d);
+    }
+}
+
+// The same over a candidate list that holds more neighbors than the cap: the first cap are summed
+// and written to the neighbor list.
+__device__ __forceinline__ uint32_t density_capped(const uint2 *p, uint32_t words, const float4 *lpos,
+                                                   const DensitySelf &x, uint2 *li, uint32_t cap, uint32_t fill,
+                                                   DensitySum &d)
+{
+    d = DensitySum{};
+    ListOut lo(li, cap);
+    each_word(p, words, [&](uint2 w) {
+        uint32_t e[4];
+        word_entries(w, e);
+        for (uint32_t u = 0; u < 4; ++u) {
+            const DensityTerm t = density_term<true, false>(x, at16(lpos, e[u]));
+            if (t.d2 < x.t2) {
+                if (lo.n < cap) density_add<true>(d, x, t);
                 lo.push(e[u]);
             }
         }
-    }
-    return lo.n();
+    });
+    d.req = lo.n;
+    return lo.finish(fill);
 }
 
-// Density sums over a compacted list, kTermStep entries per step (loads first, sums in list order).
-template <bool TENSION>
-__device__ __forceinline__ void density_list(const ListRef &li, uint32_t cnt, const float4 *lpos,
-                                             const DensitySelf &x, DensitySum &d)
+// The delta terms of a particle without cohesion, viscosity, CFL and tension terms: the pressure
+// term of every listed particle within the neighbor radius (delta_term's, restated for the one
+// term), in list order.
+template <bool FAST>
+__device__ __forceinline__ void delta_plain(const uint2 *p, uint32_t words, const float4 *lcs, const DeltaSelf &x,
+                                            DeltaSum &d)
 {
-    // the next group's entries are loaded while the current group's terms are evaluated
-    uint32_t en[kTermStep];
-    if (cnt > 0) list_group(li, 0, cnt, en);
-    for (uint32_t k = 0; k < cnt; k += kTermStep) {
-        uint32_t e[kTermStep];
+    const float k2 = __fmul_rn(2.0f, x.kw);
+    each_word(p, words, [&](uint2 w) {
+        uint32_t e[4];
+        word_entries(w, e);
+        // two at a time: four hold more registers than the pass has without spilling
 #pragma unroll
-        for (uint32_t u = 0; u < kTermStep; ++u) e[u] = en[u];
-        list_group(li, k + kTermStep, cnt, en);
-        DensityTerm t[kTermStep];
+        for (uint32_t v = 0; v < 4; v += 2) {
+            float4 q[2];
+            float d2[2], dist[2], y[2];
 #pragma unroll
-        for (uint32_t u = 0; u < kTermStep; ++u) t[u] = density_term<TENSION>(x, at16(lpos, e[u]));
+            for (uint32_t u = 0; u < 2; ++u) q[u] = at16(lcs, e[v + u]);
+            uint32_t sig = 0;
 #pragma unroll
-        for (uint32_t u = 0; u < kTermStep; ++u)
-            if (k + u < cnt) density_add<TENSION>(d, x, t[u]);
-    }
+            for (uint32_t u = 0; u < 2; ++u) {
+                q[u].x = x.sx - q[u].x;
+                q[u].y = x.sy - q[u].y;
+                q[u].z = x.sz - q[u].z;
+                d2[u] = dot3(q[u].x, q[u].y, q[u].z, q[u].x, q[u].y, q[u].z);
+                dist[u] = fsqrt_nearzero_free(d2[u]);
+                if (FAST) {
+                    y[u] = frcp_newton(dist[u]);
+                    sig = max(sig, __float_as_uint(dist[u]) & 0x7fffffu);
+                }
+            }
+            // one test for the two: the significand that the Newton steps do not reach (frcp_exact)
+            if (FAST && sig == 0x7fffffu) {
+                __asm__ volatile("");
+#pragma unroll
+                for (uint32_t u = 0; u < 2; ++u) y[u] = frcp_exact(dist[u]);
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < 2; ++u) {
+                PairQuot pq;
+                pair_quot_y<FAST, true>(pq, q[u].x, q[u].y, q[u].z, dist[u], x.h, x.ih, k2, y[u]);
+                const float msc = 0.5f * (x.Ci + q[u].w) * pq.der;
+                if (d2[u] < x.t2 && !(dist[u] <= kEps)) {
+                    d.x = d.x + msc * pq.nnx;
+                    d.y = d.y + msc * pq.nny;
+                    d.z = d.z + msc * pq.nnz;
+                    d.w = d.w + 1.0f;
+                }
+            }
+        }
+    });
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1076,7 +1224,7 @@ constexpr int kDensPlain = 0, kDensBuild = 1, kDensReuse = 2;
 // particle class 0, kClsBlock one class per scene with fluid, read from the block's first particle.
 constexpr int kClsMixed = 0, kClsOne = 1, kClsBlock = 2;
 template <int UCLS, int MODE>
-__global__ __launch_bounds__(kTileBlock) __attribute__((amdgpu_waves_per_eu(kTileWaves))) void k_fluid_density_tiled(
+__global__ __launch_bounds__(kTileBlock) __attribute__((amdgpu_waves_per_eu(kDensityWaves))) void k_fluid_density_tiled(
     FluidArgs a, SubstepConsts c)
 {
     constexpr bool UNIFORM = UCLS != kClsMixed;
@@ -1087,9 +1235,7 @@ __global__ __launch_bounds__(kTileBlock) __attribute__((amdgpu_waves_per_eu(kTil
     __shared__ uint32_t s_meta[kWgMetaWords];
     __shared__ uint32_t s_hmax;  // largest displacement bound in the staged halo (float bits)
     __shared__ uint32_t s_omax;  // the same over the block's own particles with mass (one class)
-    __shared__ uint32_t s_obad;  // one of those has no complete candidate list (one class)
-    constexpr bool SUP = MODE == kDensBuild || MODE == kDensReuse;  // candidate lists apply
-    constexpr bool REUSE = MODE == kDensReuse;
+    constexpr bool BUILD = MODE == kDensBuild, REUSE = MODE == kDensReuse;
     float4 *lpos = dyn;
     uint32_t *lcls = reinterpret_cast<uint32_t *>(dyn + a.tile + kTilePad);
     const uint32_t tid = threadIdx.x;
@@ -1100,12 +1246,16 @@ __global__ __launch_bounds__(kTileBlock) __attribute__((amdgpu_waves_per_eu(kTil
     if (blockIdx.x == 0 && tid == 0) a.iter_state[kStateMaxDisp + a.it] = 0u;
     const uint32_t nblk = a.nblk[1];  // the blocks of scenes with fluid
     uint32_t *queue = a.iter_state + kStateDensity + a.it * kXcds * kQueueStride;
-    if (tid < kWgMetaWords) s_meta[tid] = 0u;  // ordered before any use by tile_begin's barrier
-    if (tid == 0) s_hmax = s_omax = s_obad = 0u;
+    if (tid < kWgMetaWords) s_meta[tid] = 0u;  // ordered before any use by the first block's barrier
+    if (tid == 0) s_hmax = s_omax = 0u;
     BlockQueue bq(blockIdx.x);
     TileState ts;
-    auto next = [&]() -> uint32_t { return bq.next(queue, nblk); };
-    while (tile_begin(next, &s_blk, hoff, hstart, ts, 0u, a, c)) {
+    uint32_t after;
+    for (uint32_t blk = BlockQueue::first(blockIdx.x, nblk); blk != kInvalid; blk = after) {
+        tile_load(ts, blk, hoff, hstart, 0u, a, c);
+        if (tid == 0) s_blk = bq.next(queue, nblk);  // the next block, while this one's tables arrive
+        __syncthreads();
+        after = s_blk;
         if (ts.skip) {
             __syncthreads();
             continue;
@@ -1115,89 +1265,86 @@ __global__ __launch_bounds__(kTileBlock) __attribute__((amdgpu_waves_per_eu(kTil
         // registers)
         const uint32_t bcls = UCLS == kClsBlock ? __builtin_amdgcn_readfirstlane(a.cls[ts.p0]) : 0u;
         if (ts.lds) {
-            const uint32_t total = hoff[kHalo];
+            const uint32_t total = hoff[kHalo], fill = total * kEntryScale;
             // a halo of one particle class (the common case in a pool of single-material scenes)
             // takes the class filter out of the walk, as a pool of one class does
             const uint32_t ref = UNIFORM ? bcls : a.cls[ts.p0];
-            bool mixed = false, obad = false;
+            bool mixed = false;
             uint32_t dmb = 0, dmo = 0;  // displacement bounds are non-negative floats: their bits order them
-            for (uint32_t f = tid; f < total; f += kTileBlock) {
-                const uint32_t hc = halo_cell_of(hoff, f);
-                const uint32_t q = hstart[hc] + (f - hoff[hc]);
-                float4 v = a.cur[q];
-                const bool mass = v.w > kEps;
-                if (!mass) v.x = v.y = v.z = kFarAway;
-                lpos[f] = v;
-                if (REUSE) {
-                    const uint32_t dq = __float_as_uint(a.disp[q]);
-                    dmb = max(dmb, dq);
-                    // one class: the block's own particles' part of the reuse check rides along
-                    if (UNIFORM && mass && q >= ts.p0 && q < ts.p1) {
-                        dmo = max(dmo, dq);
-                        obad |= a.scnt[q] == kSuperNone;
+            float4 lv[kStageCells];
+            uint32_t lq[kStageCells];
+            stage_halo(
+                hoff, hstart,
+                [&](uint32_t u, uint32_t q) {
+                    lv[u] = a.cur[q];
+                    if (!UNIFORM) lq[u] = a.cls[q];
+                },
+                [&](uint32_t u, uint32_t f, uint32_t q) {
+                    float4 v = lv[u];
+                    if (v.w < 0.0f) {
+                        v.x = v.y = v.z = kFarAway;
+                    } else if (REUSE) {
+                        dmb = max(dmb, __float_as_uint(v.w));
+                        // one class: the block's own particles' part of the reuse check rides along
+                        if (UNIFORM && q >= ts.p0 && q < ts.p1) dmo = max(dmo, __float_as_uint(v.w));
                     }
-                }
-                if (!UNIFORM) {
-                    const uint32_t qc = a.cls[q];
-                    lcls[f] = qc;
-                    mixed |= qc != ref;
-                }
-            }
+                    lpos[f] = v;
+                    if (!UNIFORM) {
+                        lcls[f] = lq[u];
+                        mixed |= lq[u] != ref;
+                    }
+                });
+            if (tid == 0) lpos[total] = make_float4(kFarAway, kFarAway, kFarAway, kNoMass);
             if (REUSE) {
                 dmb = wave_max(dmb);
                 if ((tid & 63u) == 0u) atomicMax(&s_hmax, dmb);
                 if (UNIFORM) {
                     dmo = wave_max(dmo);
                     if ((tid & 63u) == 0u) atomicMax(&s_omax, dmo);
-                    if (obad) s_obad = 1u;
                 }
             }
             const int any_mixed = __syncthreads_or(mixed ? 1 : 0);  // also the barrier after staging
             const bool bu = UNIFORM || !any_mixed;
+            // candidate lists apply to fluid-only scenes (only the fluid passes move their particles
+            // within a substep, and they record every displacement)
+            const bool sup = (BUILD || REUSE) && ts.fluid_only;
+            // The candidates of iteration 0 (within h + skin of x*) hold particle i's list while
+            // D_i + D_j < skin for every j in its 27 cells: a pair within h now was within
+            // h + D_i + D_j then (D: displacement since iteration 0, x* to x* + delta).  D_j is
+            // bounded by the halo's largest; the margins in FluidConst cover the rounding of the
+            // squared distances (a few ulps) and of the recorded displacements.  A block where some
+            // particle fails, or has no complete candidate list, is walked whole (one decision per
+            // block keeps the walk out of the waves of the others).
             bool reuse = false;
-            if (REUSE && UNIFORM) {
-                // One class: the check below for every particle at once, from the staging loop.
-                // D_i + hmax < allow holds for every particle with mass exactly when it holds for
-                // their largest D_i (rounded addition is monotone).
-                const ParticleClass pc = a.classes[bcls];
-                const float h = fmaxd(a.fm[pc.fluid_mat].smoothing_radius, 1.0e-4f);
-                reuse = pc.kind != CN_PARTICLE_KIND_FLUID || c.cap == 0u ||
-                        (a.scenes[pc.scene].fluid_only && s_obad == 0u &&
-                         __uint_as_float(s_omax) + __uint_as_float(s_hmax) < 0.98f * (kSkinFrac * h));
-            } else if (REUSE) {
-                // The candidates of iteration 0 (within h + skin of x*) hold particle i's list while
-                // D_i + D_j < skin for every j in its 27 cells (D: displacement since iteration 0);
-                // D_j is bounded by the halo's largest.  A block where some particle fails, or has
-                // no complete candidate list, is walked whole (one decision per block keeps the
-                // walk out of the waves of the others).
+            if (REUSE && sup && ts.complete) {
                 const float hmax = __uint_as_float(s_hmax);
-                bool bad = false;
-                for (uint32_t i = ts.p0 + tid; i < ts.p1; i += kTileBlock) {
-                    const int hc = halo_cell(ts, a.cellc[i]);
-                    const uint32_t fs = hoff[hc] + (i - hstart[hc]);
-                    const ParticleClass pc = a.classes[UNIFORM ? bcls : lcls[fs]];
-                    if (pc.kind != CN_PARTICLE_KIND_FLUID || !(lpos[fs].w > kEps) || c.cap == 0u) continue;
-                    const float h = fmaxd(a.fm[pc.fluid_mat].smoothing_radius, 1.0e-4f);
-                    bad |= !a.scenes[pc.scene].fluid_only || a.scnt[i] == kSuperNone ||
-                           !(a.disp[i] + hmax < 0.98f * (kSkinFrac * h));
+                if (UNIFORM) {
+                    // D_i + hmax < allow holds for every particle with mass exactly when it holds for
+                    // their largest D_i (rounded addition is monotone)
+                    const ParticleClass pc = a.classes[bcls];
+                    reuse = pc.kind != CN_PARTICLE_KIND_FLUID ||
+                            __uint_as_float(s_omax) + hmax < a.fc[pc.fluid_mat].allow;
+                } else {
+                    bool bad = false;
+                    for (uint32_t i = ts.p0 + tid; i < ts.p1; i += kTileBlock) {
+                        const uint32_t e = a.scnt[i] >> 16;
+                        const ParticleClass pc = a.classes[at4(lcls, e)];
+                        const float D = at16(lpos, e).w;
+                        if (pc.kind == CN_PARTICLE_KIND_FLUID && D >= 0.0f) bad |= !(D + hmax < a.fc[pc.fluid_mat].allow);
+                    }
+                    reuse = !__syncthreads_or(bad ? 1 : 0);
                 }
-                reuse = !__syncthreads_or(bad ? 1 : 0);
             }
-            // the walk at the neighbor radius (thr2 = t2, radius h) or the candidate radius (ts2) into l
+            // the walk at the neighbor radius (thr2 = t2, radius h) or the candidate radius (ts2)
             auto scan = [&](auto bu_tag, const DensitySelf &x, int4 ci, int hc, uint32_t fs, float thr2,
-                            float radius, const ListRef &l, uint32_t cap) {
+                            float radius, ListOut &lo) {
                 constexpr bool BU = decltype(bu_tag)::value;
                 const float inv = c.inv_cell > 0.0f ? c.inv_cell : a.scenes[x.pc.scene].inv_cell;
                 // displacement since the cells were assigned: none at iteration 0; later the largest
                 // |delta| of the previous iteration, where only the fluid passes move fluid particles
-                const float dmax = a.it == 0 ? 0.0f : (a.scenes[x.pc.scene].fluid_only ? fsqrt(md2) : 3.4e38f);
+                const float dmax = a.it == 0 ? 0.0f : (ts.fluid_only ? fsqrt(md2) : 3.4e38f);
                 const RowCull rc = row_cull(x.s, ci, inv, radius, dmax);
-                return scan_rows<BU>(hoff, hc, fs, lpos, lcls, x, thr2, l, cap, a, rc);
-            };
-            auto super = [&](const DensitySelf &x, const ListRef &ls, uint32_t scount, const ListRef &li,
-                             DensitySum &d) {
-                return x.tension ? density_super<true>(ls, scount, lpos, x, li, c.cap, d)
-                                 : density_super<false>(ls, scount, lpos, x, li, c.cap, d);
+                scan_rows<BU>(hoff, hc, fs, lpos, lcls, x, thr2, lo, a, rc);
             };
             // BLK: the block's halo holds one particle class (bref, wave-uniform), so the class and
             // everything the particle derives from it (material, radius, thresholds) load into
@@ -1207,50 +1354,63 @@ __global__ __launch_bounds__(kTileBlock) __attribute__((amdgpu_waves_per_eu(kTil
             auto particles = [&](auto blk_tag) {
                 constexpr bool BLK = decltype(blk_tag)::value;
                 for (uint32_t i = ts.p0 + tid; i < ts.p1; i += kTileBlock) {
-                    const int4 ci = a.cellc[i];
-                    const uint32_t bw = a.bnd[i];  // loaded beside the cell, long before its use
-                    const int hc = halo_cell(ts, ci);
-                    const uint32_t fs = hoff[hc] + (i - hstart[hc]);
+                    const uint32_t bw = a.bnd[i];  // loaded first, long before its use
+                    int4 ci = make_int4(0, 0, 0, 0);
+                    int hc = 0;
+                    uint32_t entry, words = 0;
+                    if (REUSE && reuse) {
+                        const uint32_t sw = a.scnt[i];
+                        entry = sw >> 16;
+                        words = sw & kWordsMask;
+                    } else {
+                        ci = a.cellc[i];
+                        hc = halo_cell(ts, ci);
+                        entry = (hoff[hc] + (i - hstart[hc])) * kEntryScale;
+                    }
                     DensitySelf x;
-                    uint32_t cnt = 0;
-                    if (density_begin(x, i, lpos[fs], UNIFORM ? bcls : (BLK ? bref : lcls[fs]), a, SUP)) {
+                    uint32_t lw = 0, sw = 0;
+                    if (density_begin(x, i, at16(lpos, entry),
+                                      UNIFORM ? bcls : (BLK ? bref : at4(lcls, entry)), a)) {
                         DensitySum d;
-                        const ListRef li = list_ref(a.list, i, c.cap);
                         if (density_walks(x, BLK || bu, c)) {
-                            bool done = false;
-                            if (REUSE && reuse) {
-                                ++ma.reuse;
-                                d.req = super(x, list_ref(a.slist, i, kSuperSlots), a.scnt[i], li, d);
-                                done = true;
-                            } else if (MODE == kDensBuild && x.sup) {
+                            uint2 *li = list_words(a.list, i, list_rows(c.cap));
+                            uint2 *ls = list_words(a.slist, i, kSuperSlots);
+                            bool done = REUSE && reuse;
+                            if (REUSE && reuse) ++ma.reuse;
+                            if (BUILD && sup) {
                                 // the candidates within h + skin, then the neighbors among them; a
                                 // particle with more candidates than the list holds walks for its
-                                // neighbors (and never reuses: its count is marked)
-                                const ListRef ls = list_ref(a.slist, i, kSuperSlots);
-                                const float rs = fsqrt(x.ts2);
-                                const uint32_t sreq = BLK || bu ? scan(std::true_type{}, x, ci, hc, fs, x.ts2, rs, ls, kSuperSlots)
-                                                                : scan(std::false_type{}, x, ci, hc, fs, x.ts2, rs, ls, kSuperSlots);
-                                a.scnt[i] = sreq <= kSuperSlots ? (uint16_t)sreq : kSuperNone;
-                                if (sreq <= kSuperSlots) {
-                                    d.req = super(x, ls, sreq, li, d);
-                                    done = true;
-                                }
+                                // neighbors (and its block never reuses)
+                                const FluidConst fc = a.fc[x.pc.fluid_mat];
+                                ListOut lo(ls, kSuperSlots);
+                                if (BLK || bu) scan(std::true_type{}, x, ci, hc, entry / kEntryScale, fc.ts2, fc.rs, lo);
+                                else scan(std::false_type{}, x, ci, hc, entry / kEntryScale, fc.ts2, fc.rs, lo);
+                                done = lo.n <= kSuperSlots;
+                                words = lo.finish(fill);
+                                sw = done ? words : kSuperNone;
+                                if (!done) a.blk_halo[(size_t)ts.blk * kHaloStride + kHdSuper] = 0u;
                             }
-                            if (!done) {
-                                d.req = BLK || bu ? scan(std::true_type{}, x, ci, hc, fs, x.t2, x.h, li, c.cap)
-                                                  : scan(std::false_type{}, x, ci, hc, fs, x.t2, x.h, li, c.cap);
-                                d.inr = min(d.req, c.cap);
-                                if (x.tension)
-                                    density_list<true>(li, d.inr, lpos, x, d);
-                                else
-                                    density_list<false>(li, d.inr, lpos, x, d);
+                            if (done) {
+                                density_sums(ls, words, lpos, x, d);
+                                lw = words;
+                                if (d.req > c.cap)
+                                    lw = kInList | density_capped(ls, words, lpos, x, li, c.cap, fill, d);
+                            } else {
+                                ListOut lo(li, c.cap);
+                                if (BLK || bu) scan(std::true_type{}, x, ci, hc, entry / kEntryScale, x.t2, x.h, lo);
+                                else scan(std::false_type{}, x, ci, hc, entry / kEntryScale, x.t2, x.h, lo);
+                                const uint32_t req = lo.n;
+                                words = lo.finish(fill);
+                                density_sums(li, words, lpos, x, d);
+                                d.req = req;
+                                lw = kInList | words;
                             }
                             d.inr = min(d.req, c.cap);
                         }
-                        cnt = d.inr;
                         density_end(i, bw, d, x, ma, a, c);
                     }
-                    a.lcnt[i] = cnt;
+                    a.lcnt[i] = list_word(entry, lw);
+                    if (BUILD && sup) a.scnt[i] = list_word(entry, sw);
                 }
             };
             if (!UNIFORM && bu)
@@ -1259,12 +1419,13 @@ __global__ __launch_bounds__(kTileBlock) __attribute__((amdgpu_waves_per_eu(kTil
                 particles(std::false_type{});
             if (tid == 0) ++ma.lds;
         } else {
-            for (uint32_t i = ts.p0 + tid; i < ts.p1; i += kTileBlock) density_global<UNIFORM>(i, ma, a, c, bcls);
+            for (uint32_t i = ts.p0 + tid; i < ts.p1; i += kTileBlock)
+                density_global<UNIFORM>(i, ma, a, c, bcls);
             if (tid == 0) ++ma.runs;
         }
         meta_to_wg(ma, s_meta);
         __syncthreads();
-        if (tid == 0) s_hmax = s_omax = s_obad = 0u;  // read again only after the next block's staging barrier
+        if (tid == 0) s_hmax = s_omax = 0u;  // read again only after the next block's staging barrier
     }
     flush_wg_meta(s_meta, a);
 }
@@ -1273,9 +1434,10 @@ __global__ __launch_bounds__(kTileBlock) __attribute__((amdgpu_waves_per_eu(kTil
 // only fits without it are skipped and left to the WIDE = true launch, which takes the listed wide
 // blocks and reads the previous delta from HBM through a staged slot map.
 template <int UCLS, bool WIDE>
-__global__ __launch_bounds__(kTileBlock) __attribute__((amdgpu_waves_per_eu(kTileWaves))) void k_fluid_delta_tiled(
+__global__ __launch_bounds__(kTileBlock) __attribute__((amdgpu_waves_per_eu(kDeltaWaves))) void k_fluid_delta_tiled(
     FluidArgs a, SubstepConsts c)
 {
+    const bool listed = WIDE && a.wide_only;  // the listed wide blocks, else every block
     constexpr bool UNIFORM = UCLS != kClsMixed;
     extern __shared__ float4 dyn[];
     __shared__ uint32_t hoff[kHalo + 1];
@@ -1283,39 +1445,69 @@ __global__ __launch_bounds__(kTileBlock) __attribute__((amdgpu_waves_per_eu(kTil
     __shared__ uint32_t s_blk;
     const bool use_d = a.it > 0;
     const bool tension = c.tension != 0u;
+    const uint32_t room = a.tile + 1u;  // the halo and the filling entry's record
     float4 *lcs = dyn;
-    float4 *ldin = lcs + a.tile;
-    float4 *lnc = ldin + (use_d && !WIDE ? a.tile : 0u);
-    uint32_t *lcls = reinterpret_cast<uint32_t *>(lnc + (tension ? a.tile : 0u));
-    uint32_t *lslot = lcls + (UNIFORM ? 0u : a.tile);
+    float4 *ldin = lcs + room;
+    float4 *lnc = ldin + (use_d && !WIDE ? room : 0u);
+    uint32_t *lcls = reinterpret_cast<uint32_t *>(lnc + (tension ? room : 0u));
+    uint32_t *lslot = lcls + (UNIFORM ? 0u : room);
     const uint32_t tid = threadIdx.x;
     const uint32_t nblk = a.nblk[1];
     uint32_t *queue = a.iter_state + kStateDelta + a.it * kXcds * kQueueStride;
     uint32_t *wqueue = a.iter_state + kStateWideQueue + a.it;
-    const uint32_t nwide = WIDE ? a.iter_state[kStateWideCount] : 0u;
+    const uint32_t nwide = listed ? a.iter_state[kStateWideCount] : 0u;
     BlockQueue bq(blockIdx.x);
     TileState ts;
-    const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     float d2max = 0.0f;
+    bool rel_one = false;  // one class in the launch: see rel
+    if (UCLS == kClsOne && use_d) {
+        const ParticleClass pc0 = a.classes[0];
+        rel_one = pc0.kind == CN_PARTICLE_KIND_FLUID &&
+                  (cfl_term_on(a.fm[pc0.fluid_mat], a, c) || visc_term_on(a.fm[pc0.fluid_mat], a, c));
+    }
     auto next = [&]() -> uint32_t {
-        if (!WIDE) return bq.next(queue, nblk);
-        const uint32_t t = atomicAdd(wqueue, 1u);
+        if (!listed) return bq.next(queue, nblk);
+        if (nwide <= gridDim.x) return kInvalid;
+        const uint32_t t = gridDim.x + atomicAdd(wqueue, 1u);
         return t < nwide ? a.wide_blk[t] : kInvalid;
     };
-    while (tile_begin(next, &s_blk, hoff, hstart, ts, WIDE || !use_d ? 0u : c.tile_wide, a, c)) {
+    const uint32_t first = !listed ? BlockQueue::first(blockIdx.x, nblk)
+                                   : (blockIdx.x < nwide ? a.wide_blk[blockIdx.x] : kInvalid);
+    uint32_t after;
+    for (uint32_t blk = first; blk != kInvalid; blk = after) {
+        tile_load(ts, blk, hoff, hstart, WIDE || !use_d ? 0u : c.tile_wide, a, c);
+        if (tid == 0) s_blk = next();  // the next block, while this one's tables arrive
+        __syncthreads();
+        after = s_blk;
         if (ts.skip) {
             __syncthreads();
             continue;
         }
         // the block's class
         const uint32_t bcls = UCLS == kClsBlock ? __builtin_amdgcn_readfirstlane(a.cls[ts.p0]) : 0u;
+        const uint32_t ref = UNIFORM ? bcls : a.cls[ts.p0];
+        bool bu = UNIFORM;  // one particle class in the halo: every listed neighbor has the particle's material
         if (ts.lds) {
-            const uint32_t total = hoff[kHalo];
-            const uint32_t ref = UNIFORM ? bcls : a.cls[ts.p0];
+            bool mixed = false;
+            float4 lv[kStageCells];
+            uint32_t lq[kStageCells];
+            stage_halo(
+                hoff, hstart,
+                [&](uint32_t u, uint32_t q) {
+                    lv[u] = a.cs[q];
+                    if (!UNIFORM) lq[u] = a.cls[q];
+                },
+                [&](uint32_t u, uint32_t f, uint32_t q) {
+                    lcs[f] = make_float4(lv[u].x, lv[u].y, lv[u].z, lv[u].w);
+                    if (!UNIFORM) {
+                        lcls[f] = lq[u];
+                        mixed |= lq[u] != ref;
+                    }
+                });
             // the neighbors' previous deltas are read only by the viscosity and CFL terms: staged
-            // only when one of the block's fluid particles has one of them on
-            bool rel = false;
-            if (!WIDE && use_d) {
+            // (the wide layout: their slots) only when one of the block's fluid particles has one on
+            bool rel = rel_one;
+            if (use_d && UCLS != kClsOne) {
                 if (UNIFORM) {
                     const ParticleClass pc0 = a.classes[bcls];
                     rel = pc0.kind == CN_PARTICLE_KIND_FLUID &&
@@ -1330,78 +1522,91 @@ __global__ __launch_bounds__(kTileBlock) __attribute__((amdgpu_waves_per_eu(kTil
                     rel = __syncthreads_or(mine ? 1 : 0) != 0;
                 }
             }
-            bool mixed = false;
-            for (uint32_t f = tid; f < total; f += kTileBlock) {
-                const uint32_t hc = halo_cell_of(hoff, f);
-                const uint32_t q = hstart[hc] + (f - hoff[hc]);
-                lcs[f] = a.cs[q];
-                if (rel) ldin[f] = a.din[q];
-                if (WIDE) lslot[f] = q;
-                if (tension) lnc[f] = a.nc[q];
-                if (!UNIFORM) {
-                    const uint32_t qc = a.cls[q];
-                    lcls[f] = qc;
-                    mixed |= qc != ref;
-                }
+            if (WIDE && rel)
+                stage_halo(
+                    hoff, hstart, [&](uint32_t, uint32_t) {}, [&](uint32_t, uint32_t f, uint32_t q) { lslot[f] = q; });
+            if (!WIDE && rel) {
+                float4 dv[kStageCells];
+                stage_halo(
+                    hoff, hstart, [&](uint32_t u, uint32_t q) { dv[u] = a.din[q]; },
+                    [&](uint32_t u, uint32_t f, uint32_t) { ldin[f] = make_float4(dv[u].x, dv[u].y, dv[u].z, 0.0f); });
             }
-            // one particle class in the halo: every listed neighbor has the particle's material
+            if (tension) {
+                float4 nv[kStageCells];
+                stage_halo(
+                    hoff, hstart, [&](uint32_t u, uint32_t q) { nv[u] = a.nc[q]; },
+                    [&](uint32_t u, uint32_t f, uint32_t) { lnc[f] = make_float4(nv[u].x, nv[u].y, nv[u].z, nv[u].w); });
+            }
+            if (tid == 0) {  // what the filling entry names
+                const uint32_t total = hoff[kHalo];
+                lcs[total] = make_float4(kFarAway, kFarAway, kFarAway, 0.0f);
+                if (!WIDE && rel) ldin[total] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                if (tension) lnc[total] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                if (!UNIFORM) lcls[total] = ref;
+                if (WIDE && rel) lslot[total] = ts.p0;
+            }
             const int any_mixed = __syncthreads_or(mixed ? 1 : 0);  // also the barrier after staging
-            const bool bu = UNIFORM || !any_mixed;
-            // BLK: one particle class in the halo (bref, wave-uniform): the class-derived values of
-            // each particle load into scalar registers (the general instantiation in a pool of
-            // single-material scenes)
-            const uint32_t bref = __builtin_amdgcn_readfirstlane(ref);
-            auto particles = [&](auto blk_tag) {
-                constexpr bool BLK = decltype(blk_tag)::value;
-                for (uint32_t i = ts.p0 + tid; i < ts.p1; i += kTileBlock) {
-                    const int4 ci = a.cellc[i];
-                    const DeltaPre pre = delta_pre<UNIFORM || BLK>(i, a, UNIFORM ? bcls : bref);
-                    const uint32_t cnt = a.lcnt[i];
-                    const int hc = halo_cell(ts, ci);
-                    const uint32_t fs = hoff[hc] + (i - hstart[hc]);
-                    const ListRef li = list_ref(a.list, i, c.cap);
-                    const float d2 = delta_particle<UNIFORM>(
-                        i, fs, pre,
-                        [&](const DeltaSelf &x, DeltaSum &d) {
-                            // the listed neighbors, kDeltaStep per step: loads first (the next group's
-                            // entries while this group's terms are evaluated), terms independent, sums
-                            // in list order
-                            uint32_t en[kDeltaStep];
-                            if (cnt > 0) list_group(li, 0, cnt, en);
-                            for (uint32_t k = 0; k < cnt; k += kDeltaStep) {
-                                uint32_t e[kDeltaStep];
-    #pragma unroll
-                                for (uint32_t u = 0; u < kDeltaStep; ++u) e[u] = en[u];
-                                list_group(li, k + kDeltaStep, cnt, en);
-                                float4 dq[kDeltaStep];
-    #pragma unroll
-                                for (uint32_t u = 0; u < kDeltaStep; ++u)
-                                    dq[u] = !x.need_rel ? zero : (WIDE ? a.din[at4(lslot, e[u])] : at16(ldin, e[u]));
-                                DeltaTerm t[kDeltaStep];
-    #pragma unroll
-                                for (uint32_t u = 0; u < kDeltaStep; ++u)
-                                    t[u] = BLK || bu
-                                               ? delta_term<true>(x, at16(lcs, e[u]), dq[u],
-                                                                  x.tension ? at16(lnc, e[u]) : zero, 0u, a)
-                                               : delta_term<false>(x, at16(lcs, e[u]), dq[u],
-                                                                   x.tension ? at16(lnc, e[u]) : zero, at4(lcls, e[u]), a);
-    #pragma unroll
-                                for (uint32_t u = 0; u < kDeltaStep; ++u)
-                                    if (k + u < cnt) delta_add(d, t[u]);
-                            }
-                        },
-                        lcs, lnc, a, c);
-                    d2max = fmaxd(d2max, d2);
-                }
-            };
-            if (!UNIFORM && bu)
-                particles(std::true_type{});
-            else
-                particles(std::false_type{});
-        } else {
-            for (uint32_t i = ts.p0 + tid; i < ts.p1; i += kTileBlock)
-                d2max = fmaxd(d2max, delta_global<UNIFORM>(i, a, c, bcls));
+            bu = UNIFORM || !any_mixed;
         }
+        // BLK: one particle class in the halo (bref, wave-uniform): the class-derived values of
+        // each particle load into scalar registers (the general instantiation in a pool of
+        // single-material scenes)
+        const uint32_t bref = __builtin_amdgcn_readfirstlane(ref);
+        auto particles = [&](auto blk_tag) {
+            constexpr bool BLK = decltype(blk_tag)::value;
+            for (uint32_t i = ts.p0 + tid; i < ts.p1; i += kTileBlock) {
+                // a block that is not staged walks the run table
+                const uint32_t lw = ts.lds ? a.lcnt[i] : 0u;
+                const DeltaPre pre = delta_pre<UNIFORM || BLK>(i, a, UNIFORM ? bcls : bref);
+                const uint2 *p = lw & kInList ? list_words(a.list, i, list_rows(c.cap))
+                                              : list_words(a.slist, i, kSuperSlots);
+                const float d2 = delta_particle<UNIFORM>(
+                    i, pre,
+                    [&](const DeltaSelf &x, DeltaSum &d) {
+                        if (!ts.lds) {
+                            delta_walk<UNIFORM || BLK>(i, x, d, a, c);
+                            return;
+                        }
+                        const uint32_t words = lw & kWordsMask;
+                        if (!words) return;
+                        const bool fast = __all(x.fd);
+                        if (x.plain) {
+                            if (fast) delta_plain<true>(p, words, lcs, x, d);
+                            else delta_plain<false>(p, words, lcs, x, d);
+                            return;
+                        }
+                        // the general terms, two listed particles at a time
+                        each_word(p, words, [&](uint2 w) {
+#pragma unroll 2
+                            for (uint32_t u = 0; u < 4; ++u) {
+                                const uint32_t e = (u & 2u ? w.y : w.x) >> ((u & 1u) * 16u) & 0xffffu;
+                                const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                                const float4 dq = !x.need_rel ? zero : (WIDE ? a.din[at4(lslot, e)] : at16(ldin, e));
+                                const float4 ncq = x.tension ? at16(lnc, e) : zero;
+                                delta_add(d, BLK || bu ? delta_term<true>(x, at16(lcs, e), dq, ncq, 0u, a)
+                                                       : delta_term<false>(x, at16(lcs, e), dq, ncq, at4(lcls, e), a));
+                            }
+                        });
+                    },
+                    [&](bool nc) {
+                        float4 r;
+                        if (ts.lds) {
+                            const float4 &v = at16(nc ? lnc : lcs, lw >> 16);
+                            r = make_float4(v.x, v.y, v.z, v.w);
+                        } else {
+                            const float4 &v = (nc ? a.nc : a.cs)[i];
+                            r = make_float4(v.x, v.y, v.z, v.w);
+                        }
+                        return r;
+                    },
+                    a, c);
+                d2max = fmaxd(d2max, d2);
+            }
+        };
+        if (!UNIFORM && bu)
+            particles(std::true_type{});
+        else
+            particles(std::false_type{});
         __syncthreads();
     }
     flush_disp(d2max, a);
@@ -1437,13 +1642,13 @@ __global__ __launch_bounds__(kBlock) void k_fluid_lists(FluidArgs a, SubstepCons
     const ParticleClass pc = a.classes[UNIFORM ? 0u : a.cls[i]];
     const float4 s = a.cur[i];
     uint32_t cnt = 0;
-    if (pc.kind == CN_PARTICLE_KIND_FLUID && s.w > kEps && c.cap > 0 && (!UNIFORM || neighbor_ok(pc, pc))) {
-        const float t2 = a.t2[pc.fluid_mat];
+    if (pc.kind == CN_PARTICLE_KIND_FLUID && s.w >= 0.0f && c.cap > 0 && (!UNIFORM || neighbor_ok(pc, pc))) {
+        const float t2 = a.fc[pc.fluid_mat].t2;
         walk_runs(a.cellc[i], run_table(a), c, [&](uint32_t q) {
             if (q == i) return true;
             if (!UNIFORM && !neighbor_ok(pc, a.classes[a.cls[q]])) return true;
             const float4 pj = a.cur[q];
-            if (pj.w <= kEps) return true;
+            if (pj.w < 0.0f) return true;
             const float dx = s.x - pj.x, dy = s.y - pj.y, dz = s.z - pj.z;
             if (!(dot3(dx, dy, dz, dx, dy, dz) < t2)) return true;
             a.nbr[(size_t)cnt * c.n + i] = q;
@@ -1484,7 +1689,7 @@ __global__ __launch_bounds__(kBlock) void k_fluid_vorticity(FluidArgs a, Substep
     float4 self = APPLY ? vort[i] : vel[i];
     if (APPLY && self.w <= kEps) return;
     const float h = fmaxd(m.smoothing_radius, 1.0e-4f);
-    const float t2 = a.t2[pc.fluid_mat];
+    const float t2 = a.fc[pc.fluid_mat].t2;
     float ax = 0.0f, ay = 0.0f, az = 0.0f;
     // one listed neighbor's term (same material, inside the kernel's support)
     auto term = [&](uint32_t q, uint32_t qmat, float dx, float dy, float dz) {
@@ -1622,7 +1827,7 @@ __global__ __launch_bounds__(kBlock) void k_fluid_render_aniso(FluidArgs a, Subs
         const float inv = fdiv(1.0f, support);
         const float iso = fmaxd(1.0f * radius, radius);
         const float4 s = a.pos[i];
-        const float t2 = a.t2[pc.fluid_mat];
+        const float t2 = a.fc[pc.fluid_mat].t2;
         const bool walk = s.w > kEps && c.cap > 0 && (!UNIFORM || neighbor_ok(pc, pc));
         // f(neighbor position, weight) per contributing entry of the list
         auto weigh = [&](const float4 &pj, float d2, auto &&f) {
@@ -1759,7 +1964,6 @@ static FluidArgs fluid_args(const SceneBuffers &s, const SubstepConsts &c, uint3
     a.lcnt = s.lcnt;
     a.slist = s.slist;
     a.scnt = s.scnt;
-    a.disp = c.superset ? s.disp : nullptr;
     a.run_key = s.run_key;
     a.run_start = s.run_start;
     a.run_info = s.run_info;
@@ -1772,21 +1976,29 @@ static FluidArgs fluid_args(const SceneBuffers &s, const SubstepConsts &c, uint3
     a.iter_state = s.iter_state;
     a.classes = s.classes;
     a.fm = s.fluid_mats;
-    a.t2 = s.fluid_t2;
+    a.fc = s.fluid_consts;
     a.col = s.colliders;
     a.scenes = s.scenes;
     a.active = s.scene_active;
     a.meta = s.meta;
     a.it = it;
     a.tile = 0;
+    a.wide_only = 0;
     return a;
 }
 
 static uint32_t grid_of(uint32_t n) { return (n + kBlock - 1) / kBlock; }
 
-// LDS budget of one tiled workgroup: the dynamic tile plus the static halo table stays under a third
-// of the CU's 160 KiB, so three workgroups share a CU
-constexpr uint32_t kDynLdsBytes = 50u * 1024u;
+// LDS budget of one tiled workgroup (the static halo table and counters take some 2 KiB more).  In a
+// large scene three workgroups of the density pass and two of the delta pass share a CU's 160 KiB; a
+// scene whose cell blocks (some 400 particles each, fewer at its surface) leave a CU one or two
+// workgroups lets each have what the others would not use, so that fewer blocks need the wide layout
+// or the run table.
+static uint32_t lds_budget(const SubstepConsts &c, uint32_t share)
+{
+    const uint32_t fits = c.n <= 96u * 1024u ? 1u : (c.n <= 192u * 1024u ? 2u : 3u);
+    return 156u * 1024u / std::min(share, fits) - 2u * 1024u;
+}
 
 static bool tiled(const SubstepConsts &c, uint32_t it) { return c.key_mode == CN_KEY_MORTON && it < kIterStateWords; }
 
@@ -1802,10 +2014,11 @@ static uint32_t persistent_grid(const SubstepConsts &c)
 // passes stage was staged (and listed in halo offsets) by the density pass.
 void fluid_tiles(SubstepConsts &c)
 {
-    const uint32_t cls = c.fluid_uniform ? 0u : 4u, nc = c.tension ? 16u : 0u;
-    c.tile_dens = std::min<uint32_t>(c.tile_max, kDynLdsBytes / (16u + cls) - kTilePad);
-    c.tile_delta = std::min<uint32_t>(c.tile_max, kDynLdsBytes / (32u + nc + cls));
-    c.tile_wide = std::min<uint32_t>(c.tile_max, kDynLdsBytes / (20u + nc + cls));
+    const uint32_t cls = c.fluid_uniform ? 0u : 4u, nc = c.tension ? 16u : 0u, dens = lds_budget(c, 3), lds = lds_budget(c, 2);
+    const uint32_t most = std::min<uint32_t>(c.tile_max, kTileMost);
+    c.tile_dens = std::min<uint32_t>(most, dens / (16u + cls) - kTilePad);
+    c.tile_wide = std::min<uint32_t>(c.tile_dens, lds / (20u + nc + cls) - 1u);
+    c.tile_delta = c.viscous ? std::min<uint32_t>(c.tile_wide, lds / (32u + nc + cls) - 1u) : c.tile_wide;
 }
 
 void launch_blk_halo(const SceneBuffers &s, const SubstepConsts &c, hipStream_t st)
@@ -1860,18 +2073,27 @@ void launch_fluid_delta(const SceneBuffers &s, const SubstepConsts &c, uint32_t 
     FluidArgs a = fluid_args(s, c, it, din);
     if (tiled(c, it)) {
         const uint32_t cls = c.fluid_uniform ? 0u : 4u, nc = c.tension ? 16u : 0u;
+        const dim3 grid(persistent_grid(c)), block(kTileBlock);
+        // The neighbors' previous deltas are read by the viscosity and CFL terms.  Without a viscous
+        // material only the CFL term can want them, which it does in the rare iteration that moved a
+        // particle by half its CFL radius: every block takes the wide layout in one launch.
+        if (it > 0 && !c.viscous) {
+            a.tile = c.tile_wide;
+            launch_tiled<k_fluid_delta_tiled<kClsOne, true>, k_fluid_delta_tiled<kClsBlock, true>,
+                         k_fluid_delta_tiled<kClsMixed, true>>(c, grid, block, (size_t)(a.tile + 1u) * (20u + nc + cls), st, a);
+            return;
+        }
         // first iteration: no previous delta, so the delta pass stages as much as the wide one
         a.tile = it > 0 ? c.tile_delta : c.tile_wide;
-        size_t lds = (size_t)a.tile * (16u + (it > 0 ? 16u : 0u) + nc + cls);
-        const dim3 grid(persistent_grid(c)), block(kTileBlock);
+        size_t lds = (size_t)(a.tile + 1u) * (16u + (it > 0 ? 16u : 0u) + nc + cls);
         launch_tiled<k_fluid_delta_tiled<kClsOne, false>, k_fluid_delta_tiled<kClsBlock, false>,
                      k_fluid_delta_tiled<kClsMixed, false>>(c, grid, block, lds, st, a);
         if (it > 0 && c.tile_wide > c.tile_delta) {
             a.tile = c.tile_wide;
-            lds = (size_t)a.tile * (20u + nc + cls);
-            const dim3 wgrid(persistent_grid(c));
+            a.wide_only = 1;
+            lds = (size_t)(a.tile + 1u) * (20u + nc + cls);
             launch_tiled<k_fluid_delta_tiled<kClsOne, true>, k_fluid_delta_tiled<kClsBlock, true>,
-                         k_fluid_delta_tiled<kClsMixed, true>>(c, wgrid, block, lds, st, a);
+                         k_fluid_delta_tiled<kClsMixed, true>>(c, grid, block, lds, st, a);
         }
     } else {
         if (c.uniform_class)

@@ -36,7 +36,10 @@ constexpr uint32_t kHdP1 = kHdFlags + 2;
 constexpr uint32_t kHdBase = kHdFlags + 3;      // 3 words
 constexpr uint32_t kHdScene = kHdFlags + 6;
 constexpr uint32_t kHdPairs = kHdFlags + 7;     // 1: a contact pair can exist between particles of the halo
+constexpr uint32_t kHdSuper = kHdFlags + 8;     // 1: every particle of the block has its candidate list
+constexpr uint32_t kHdFluidOnly = kHdFlags + 9;  // the scene's fluid_only
 constexpr uint32_t kHaloStride = 448;
+static_assert(kHdFluidOnly < kHaloStride, "the descriptor's words fit its stride");
 // kHdFlags value of a block in a scene without fluid particles or contact pairs (no halo written)
 constexpr uint32_t kHdNoFluid = 2u;
 // candidate contact partners a particle keeps per substep; more are counted as overflows
@@ -47,21 +50,44 @@ constexpr uint32_t kMetaWords = 16;  // device diagnostics words
 // iteration 0 plus the largest one in its block's halo stays below the skin
 constexpr uint32_t kSuperSlots = 96;
 constexpr float kSkinFrac = 0.05f;
-constexpr uint16_t kSuperNone = 0xffffu;  // count marker: the candidates did not fit, walk instead
-// Per-slot lists of 16-bit entries are stored in groups of kListGroup consecutive slots: entry k
-// of slot i sits at (i / kListGroup) * kListGroup * rows + k * kListGroup + i % kListGroup, so one
-// wave's row is one 128-byte line and a group's rows are contiguous (few pages per wave).
+// Per-slot lists of 16-bit entries are stored four to a word, in groups of kListGroup consecutive
+// slots: word w of slot i sits (i / kListGroup) * kListGroup * rows entries into the buffer, then
+// w * kListGroup + i % kListGroup words on, so one wave's words are 512 consecutive bytes.
 constexpr uint32_t kListGroup = 64;
-// byte offset of entry 0 of slot i
-__host__ __device__ inline size_t list_entry_base(uint32_t i, uint32_t rows)
+__host__ __device__ inline uint32_t list_rows(uint32_t entries) { return (entries + 3u) & ~3u; }
+// byte offset of word 0 of slot i; rows is a multiple of four
+__host__ __device__ inline size_t list_word_base(uint32_t i, uint32_t rows)
 {
-    return ((size_t)(i / kListGroup) * kListGroup * rows + (i % kListGroup)) * sizeof(uint16_t);
+    return (size_t)(i / kListGroup) * kListGroup * rows * sizeof(uint16_t) + (i % kListGroup) * (4 * sizeof(uint16_t));
 }
 __host__ __device__ inline size_t list_slots(size_t n) { return (n + kListGroup - 1) / kListGroup * kListGroup; }
-// A list buffer is addressed with 32-bit byte offsets from its base (one 32-bit add per entry on the
-// device), so it stays within 4 GiB less 1 MiB: a list's write position may run up to 512 KiB past
-// its particle's last entry without wrapping.
+// entries of a list buffer: the slots' rows, and two words per lane that a list's reader may load
+// past the last one
+inline size_t list_entries(size_t n, uint32_t entries)
+{
+    return list_slots(n) * list_rows(entries ? entries : 1u) + 2 * 4 * kListGroup;
+}
+// Bytes of the entries themselves (slots x entries) that cn_scene_reserve and the candidate lists
+// allow.
 constexpr uint64_t kListBytesMax = 0xffffffffull - 0x100000ull;
+// halo particles a list entry can name (a byte offset of 16-byte records), less the filling entry
+constexpr uint32_t kTileMost = 4095;
+// w of a fluid solver position (SceneBuffers::curpos) that no neighbor list takes: zero inverse mass.
+// Otherwise w is D, the bound on the particle's displacement since the substep's first iteration.
+constexpr float kNoMass = -1.0f;
+
+// What follows from a fluid material's smoothing radius, computed on the host with the operations
+// the kernels would use.
+struct FluidConst {
+    float t2;     // smallest d^2 whose correctly rounded root is >= h: d2 < t2 <=> sqrt(d2) < h
+    float h;      // max(smoothing radius, 1e-4)
+    float kw;     // spiky_coef(h)
+    float ih;     // 1 / h
+    float ts2;    // squared candidate radius, h + skin
+    float rs;     // its root
+    float allow;  // bound on D_i + D_j under which the candidate lists stay complete
+    float pad;
+};
 
 // ---- radix sort (cn_sort.hip) ----
 size_t sort_scratch_words(uint32_t n);
@@ -127,7 +153,7 @@ struct SceneBuffers {
     uint32_t *perm = nullptr;
     // fluid solve
     float4 *dacc[2] = {nullptr, nullptr};
-    float4 *curpos = nullptr;       // (x* + delta, inverse mass): neighbor positions of the walk
+    float4 *curpos = nullptr;       // (x* + delta, D or kNoMass): neighbor positions of the walk
     float4 *cs = nullptr;           // (x* + delta, density constraint): neighbor records of the delta pass
     float4 *nc = nullptr;           // surface normal * tension (only with surface tension)
     uint32_t *blk_first_run = nullptr;  // first run of each Morton 4x4x4 block, then the run count
@@ -136,17 +162,16 @@ struct SceneBuffers {
     uint32_t blk_cap = 0;
     uint32_t *wide_blk = nullptr;   // blocks whose halo fits the wide delta tile only (blk_cap)
     uint32_t *iter_state = nullptr; // kStateWords: block-queue counters and max |delta|^2 per iteration
-    float *fluid_t2 = nullptr;      // per fluid material: smallest d^2 whose correctly rounded sqrt >= h
-    uint16_t *list = nullptr;       // fluid neighbor lists as halo offsets, in slot groups (list_row)
+    FluidConst *fluid_consts = nullptr;  // per fluid material
+    uint16_t *list = nullptr;       // fluid neighbor lists as halo offsets, in slot groups
     uint16_t *slist = nullptr;      // candidate lists of iteration 0 as halo offsets, in slot groups
-    uint16_t *scnt = nullptr;       // candidate count per slot, or kSuperNone
-    float *disp = nullptr;          // per slot: bound on |x* + delta - x*| after the last delta pass
+    uint32_t *scnt = nullptr;       // per slot: its staged entry and the words of its candidate list
     // constraint adjacency in particle-index order (pool indices): particle i's adjacent
     // particles are adj_idx[adj_off[i] .. adj_off[i] + adj_cnt[i]); null when no scene has any
     uint32_t *adj_off = nullptr;
     uint32_t *adj_cnt = nullptr;
     uint32_t *adj_idx = nullptr;
-    uint32_t *lcnt = nullptr;       // fluid neighbor count per slot
+    uint32_t *lcnt = nullptr;       // per slot: its staged entry, the list the delta pass walks and its words
     uint32_t *nbr = nullptr;        // neighbor lists of the pass entry, k-major: nbr[k * n + i]
     uint32_t *nbr_cnt = nullptr;
     size_t nbr_alloc = 0;

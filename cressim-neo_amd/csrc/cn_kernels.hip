@@ -303,7 +303,8 @@ __global__ __launch_bounds__(kBlock) void k_reorder(
     if (active[pc.scene]) predict(p, v, pv, gravity_scale(pc, fm), c);
     else pv = prev_o[o];
     pos_n[t] = p;
-    cur[t] = p;  // solver position x* + delta with delta = 0 at the first iteration
+    // solver position x* + delta with delta = 0 at the first iteration
+    cur[t] = make_float4(p.x, p.y, p.z, p.w > kEps ? 0.0f : kNoMass);
     vel_n[t] = v;
     prev[t] = pv;
     cls_n[t] = k;
