@@ -26,7 +26,7 @@ using namespace cn;
 // host code `scratch` is only a stand-in for the symbol: its device address on the current GPU
 // comes from hipGetSymbolAddress (noalloc_scratch below), and only that address reaches a kernel.
 constexpr size_t kNoAllocPairBytes = (size_t)CN_NOALLOC_MAX_PAIRS * sizeof(uint2);
-constexpr size_t kNoAllocCountWords = 256u * (CN_NOALLOC_MAX_PAIRS / 4096u) + 256u;
+constexpr size_t kNoAllocCountWords = 256u * (CN_NOALLOC_MAX_PAIRS / 2048u) + 256u;  // sort_scratch_words(CN_NOALLOC_MAX_PAIRS)
 constexpr size_t kNoAllocScratchBytes = 2 * kNoAllocPairBytes + kNoAllocCountWords * sizeof(uint32_t);
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
@@ -201,9 +201,9 @@ void free_scene(SceneBuffers &s)
     dfree(s.run_start);
     dfree(s.run_info);
     dfree(s.bucket);
-    dfree(s.block_runs);
-    dfree(s.run_count);
+    dfree(s.tile_counts);
     dfree(s.perm);
+    dfree(s.run_count);
     dfree(s.nc);
     dfree(s.curpos);
     dfree(s.cs);
@@ -651,27 +651,27 @@ SubstepConsts make_consts(const cn_ctx *ctx, const SceneBuffers &s, const cn_ste
 // predict + keys + sort + runs + reorder for one substep; returns the sorted (key, old slot) pairs
 uint2 *broadphase(cn_ctx *ctx, SceneBuffers &s, const SubstepConsts &c, uint32_t key_bits)
 {
+    bool counted;
     {
         ProfScope ps(ctx, "keys");
-        launch_keys(s, c, ctx->stream);
+        counted = launch_keys(s, c, ctx->stream);
     }
     uint2 *sorted;
     {
         ProfScope ps(ctx, "sort");
-        sorted = radix_sort_pairs(s.kv[0], s.kv[1], c.n, key_bits, s.sort_scratch, ctx->stream);
+        sorted = radix_sort_pairs(s.kv[0], s.kv[1], c.n, key_bits, s.sort_scratch, counted, ctx->stream);
     }
     {
         ProfScope ps(ctx, "runs");
-        launch_runs(s, c, sorted, key_bits, ctx->stream);
+        launch_runs(s, c, sorted, key_bits, ctx->has_fluid || ctx->any_pairs, ctx->stream);
     }
     {
         ProfScope ps(ctx, "reorder");
-        launch_reorder(s, c, ctx->stream);
+        launch_reorder(s, c, sorted, ctx->stream);
     }
-    if (c.key_mode == CN_KEY_MORTON) {
+    if (c.key_mode == CN_KEY_MORTON && (ctx->has_fluid || ctx->any_pairs)) {
         ProfScope ps(ctx, "blocks");
-        launch_blocks(s, c, ctx->stream);
-        if (ctx->has_fluid || ctx->any_pairs) launch_blk_halo(s, c, ctx->stream);
+        launch_blk_halo(s, c, ctx->stream);
     }
     return sorted;
 }
@@ -862,9 +862,9 @@ cn_status cn_scene_reserve(cn_ctx *ctx, uint32_t n, uint32_t cap)
     s.bucket_bits = std::min<uint32_t>(bb, 30u);
     ctx->bucket_bits_alloc = s.bucket_bits;
     CN_HIP(ctx, dalloc(&s.bucket, (size_t(1) << s.bucket_bits) + 1));
-    CN_HIP(ctx, dalloc(&s.block_runs, (N + 1023) / 1024 + 1));
-    CN_HIP(ctx, dalloc(&s.run_count, 1));
     CN_HIP(ctx, dalloc(&s.perm, N));
+    CN_HIP(ctx, dalloc(&s.tile_counts, (N + 1023) / 1024 + 1));
+    CN_HIP(ctx, dalloc(&s.run_count, kRunWords));
     CN_HIP(ctx, dalloc(&s.nc, N));
     CN_HIP(ctx, dalloc(&s.curpos, N));
     CN_HIP(ctx, dalloc(&s.cs, N));
@@ -1220,7 +1220,12 @@ cn_status upload_pool(cn_ctx *ctx, uint32_t count, const cn_scene_desc *descs)
                 lo[a] = std::min(lo[a], c.aabb_min[a]);
                 hi[a] = std::max(hi[a], c.aabb_max[a]);
             }
-        for (int a = 0; a < 3; ++a) max_span = std::max(max_span, (double)(hi[a] - lo[a]) / (double)cell + 3.0);
+        for (int a = 0; a < 3; ++a) {
+            max_span = std::max(max_span, (double)(hi[a] - lo[a]) / (double)cell + 3.0);
+            // the window starts a cell below the scene (its width is known once every scene's span is)
+            const double w = std::floor((double)lo[a] * (double)sinfo[k].inv_cell) - 1.0;
+            sinfo[k].win[a] = (int32_t)std::min(std::max(w, -1.0e9), 1.0e9);
+        }
         ctx->scene_first[k] = base;
         base += m;
     }
@@ -1708,9 +1713,9 @@ cn_status ensure_tick(cn_ctx *ctx, uint32_t m)
     CN_HIP(ctx, dalloc(&t.run_info, N));
     t.bucket_bits = std::min<uint32_t>(std::max<uint32_t>(4u, ceil_log2(N) > 1 ? ceil_log2(N) - 1 : 1), 30u);
     CN_HIP(ctx, dalloc(&t.bucket, (size_t(1) << t.bucket_bits) + 1));
-    CN_HIP(ctx, dalloc(&t.block_runs, (N + 1023) / 1024 + 1));
-    CN_HIP(ctx, dalloc(&t.run_count, 1));
     CN_HIP(ctx, dalloc(&t.perm, N));
+    CN_HIP(ctx, dalloc(&t.tile_counts, (N + 1023) / 1024 + 1));
+    CN_HIP(ctx, dalloc(&t.run_count, kRunWords));
     CN_HIP(ctx, dalloc(&t.nc, N));
     CN_HIP(ctx, dalloc(&t.curpos, N));
     CN_HIP(ctx, dalloc(&t.cs, N));
@@ -1767,9 +1772,9 @@ SceneBuffers tick_view(const cn_ctx *ctx, uint32_t m, const cn_step_params *p)
     v.bucket = t.bucket;
     const uint32_t bb = std::max<uint32_t>(4u, ceil_log2(m) > 1 ? ceil_log2(m) - 1 : 1);
     v.bucket_bits = std::min<uint32_t>(std::min<uint32_t>(bb, key_bits_of(ctx, p)), t.bucket_bits);
-    v.block_runs = t.block_runs;
-    v.run_count = t.run_count;
+    v.tile_counts = t.tile_counts;
     v.perm = t.perm;
+    v.run_count = t.run_count;
     v.nc = t.nc;
     v.curpos = t.curpos;
     v.cs = t.cs;
@@ -2476,7 +2481,7 @@ cn_status cn_pass_sort_pairs(cn_ctx *ctx, uint32_t n, uint32_t *keys, uint32_t *
     CN_HIP(ctx, dalloc(&b, n));
     CN_HIP(ctx, dalloc(&scr, sort_scratch_words(n)));
     CN_HIP(ctx, hipMemcpy(a, h.data(), n * sizeof(uint2), hipMemcpyHostToDevice));
-    uint2 *res = radix_sort_pairs(a, b, n, 32u, scr, ctx->stream);
+    uint2 *res = radix_sort_pairs(a, b, n, 32u, scr, false, ctx->stream);
     CN_HIP(ctx, hipStreamSynchronize(ctx->stream));
     CN_HIP(ctx, hipMemcpy(h.data(), res, n * sizeof(uint2), hipMemcpyDeviceToHost));
     for (uint32_t i = 0; i < n; ++i) {
@@ -2504,9 +2509,7 @@ cn_status cn_pass_sort_pairs_noalloc(cn_ctx *ctx, uint32_t n, uint32_t *keys, ui
     uint2 *b = reinterpret_cast<uint2 *>(base + kNoAllocPairBytes);
     uint32_t *counts = reinterpret_cast<uint32_t *>(base + 2 * kNoAllocPairBytes);
     // the sort writes every count and total it reads, so nothing left by an earlier call is read
-    launch_pack_pairs(keys, indices, n, a, ctx->stream);
-    const uint2 *res = radix_sort_pairs(a, b, n, 32u, counts, ctx->stream);
-    launch_unpack_pairs(res, n, keys, indices, ctx->stream);
+    radix_sort_arrays(keys, indices, a, b, n, 32u, counts, ctx->stream);
     CN_HIP(ctx, hipGetLastError());
     return CN_OK;
 }

@@ -68,6 +68,8 @@ struct SceneInfo {
                           // phase group)
     uint32_t rigid;       // 1: particle-rigid contacts can exist (a solid particle and a static
                           // collider slot), solved in the slot-order contact pass
+    int32_t win[3];       // lowest cell of the scene's window of 2^morton_bits cells per axis: inside it
+                          // no two cells share a Morton code
     uint32_t rigid_pid;   // 1: the same, for a scene without particle-particle pairs whose every
                           // particle is constrained: solved in particle-index order in the soft phase
 };
@@ -497,22 +499,35 @@ __device__ __forceinline__ float cephes_acosf(float x)
     return kCephesPio2 - cephes_asinf(x);
 }
 
-// Exclusive scan over a kBlock-thread workgroup (sh holds kBlock words); total receives the sum.
+// Exclusive scan over a workgroup of THREADS threads: a shuffle scan per wave, then the waves' totals
+// (sh holds one word per wave).  total receives the sum.
+template <int THREADS>
+__device__ __forceinline__ uint32_t block_exclusive_scan_wide(uint32_t v, uint32_t *sh, uint32_t &total)
+{
+    constexpr int W = THREADS / 64;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    uint32_t incl = v;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t o = (uint32_t)__shfl_up((int)incl, off);
+        incl += lane >= (uint32_t)off ? o : 0u;
+    }
+    if (lane == 63u) sh[wave] = incl;
+    __syncthreads();
+    uint32_t before = 0, sum = 0;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+        const uint32_t x = sh[w];
+        before += (uint32_t)w < wave ? x : 0u;
+        sum += x;
+    }
+    total = sum;
+    __syncthreads();
+    return before + incl - v;
+}
 __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t *sh, uint32_t &total)
 {
-    const uint32_t t = threadIdx.x;
-    sh[t] = v;
-    __syncthreads();
-    for (uint32_t off = 1; off < (uint32_t)kBlock; off <<= 1) {
-        const uint32_t add = t >= off ? sh[t - off] : 0u;
-        __syncthreads();
-        sh[t] += add;
-        __syncthreads();
-    }
-    total = sh[kBlock - 1];
-    const uint32_t ex = sh[t] - v;
-    __syncthreads();
-    return ex;
+    return block_exclusive_scan_wide<kBlock>(v, sh, total);
 }
 
 // XCD-aware tile index: consecutive logical tiles land on the same XCD (and its L2), since the

@@ -55,6 +55,8 @@ struct FluidArgs {
     const uint32_t *run_key;
     const uint32_t *run_start;
     const int4 *run_info;
+    int4 *run_info_out;
+    const uint32_t *run_count;
     const uint32_t *bucket;
     uint32_t bucket_shift;
     const uint32_t *blk_first_run;
@@ -720,12 +722,19 @@ __device__ __forceinline__ void flush_disp(float d2, const FluidArgs &a)
 // ---------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(kBlock) void k_blk_halo(FluidArgs a, SubstepConsts c)
 {
-    __shared__ uint32_t scan[kBlock];
+    __shared__ uint32_t scan[kBlock / 64];
     __shared__ uint32_t s_kinds, s_gmin, s_gmax;  // what the halo holds: kHas* bits, solid phase groups
     constexpr uint32_t kHasFluid = 1, kHasSolid = 2, kHasOther = 4;
     // blocks of scenes with fluid are a prefix; contact pairs can exist in any scene
     const uint32_t nb = min(a.nblk[c.pairs ? 0 : 1], c.blk_cap);
     const uint32_t tid = threadIdx.x;
+    // some particle lies outside its scene's window: wrapped cells may share runs, so every run's
+    // record is taken from its members, here and (for the later walks) in run_info
+    const bool wrapped = a.run_count[1] != 0u;
+    const uint32_t *rcls = c.pairs ? a.cls : nullptr;
+    if (wrapped)
+        for (uint32_t r = blockIdx.x * kBlock + tid; r < a.run_count[0]; r += gridDim.x * kBlock)
+            a.run_info_out[r] = run_record(a.run_start[r], a.run_start[r + 1], a.cellc, rcls);
     for (uint32_t b = blockIdx.x; b < nb; b += gridDim.x) {
         const uint32_t p0 = a.run_start[a.blk_first_run[b]], p1 = a.run_start[a.blk_first_run[b + 1]];
         const uint32_t scene = a.classes[a.cls[p0]].scene;
@@ -764,7 +773,7 @@ __global__ __launch_bounds__(kBlock) void k_blk_halo(FluidArgs a, SubstepConsts 
             if (cell_hash(tx, ty, tz) != kInvalid) {
                 const int r = find_run(cell_key(tx, ty, tz, (uint32_t)c0.w, c.key_mode, c.morton_bits), run_table(a));
                 if (r >= 0) {
-                    const int4 info = a.run_info[r];
+                    const int4 info = wrapped ? run_record(a.run_start[r], a.run_start[r + 1], a.cellc, rcls) : a.run_info[r];
                     if (!(info.w & kRunPure)) bad = true;
                     else if (info.x == tx && info.y == ty && info.z == tz) {
                         st = a.run_start[r];
@@ -1967,6 +1976,8 @@ static FluidArgs fluid_args(const SceneBuffers &s, const SubstepConsts &c, uint3
     a.run_key = s.run_key;
     a.run_start = s.run_start;
     a.run_info = s.run_info;
+    a.run_info_out = s.run_info;
+    a.run_count = s.run_count;
     a.bucket = s.bucket;
     a.bucket_shift = c.bucket_shift;
     a.blk_first_run = s.blk_first_run;

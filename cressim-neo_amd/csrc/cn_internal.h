@@ -90,11 +90,14 @@ struct FluidConst {
 };
 
 // ---- radix sort (cn_sort.hip) ----
+constexpr uint32_t kDirectTiles = 128;  // tiles whose counts a scatter workgroup sums itself
 size_t sort_scratch_words(uint32_t n);
-uint2 *radix_sort_pairs(uint2 *buf_a, uint2 *buf_b, uint32_t n, uint32_t key_bits, uint32_t *scratch,
+uint32_t sort_rounds(uint32_t n);   // a tile holds 256 x rounds pairs
+bool sort_one_group(uint32_t n);    // sorted in one launch, without counts
+uint2 *radix_sort_pairs(uint2 *buf_a, uint2 *buf_b, uint32_t n, uint32_t key_bits, uint32_t *scratch, bool counted,
                         hipStream_t stream);
-void launch_pack_pairs(const uint32_t *keys, const uint32_t *vals, uint32_t n, uint2 *out, hipStream_t stream);
-void launch_unpack_pairs(const uint2 *in, uint32_t n, uint32_t *keys, uint32_t *vals, hipStream_t stream);
+void radix_sort_arrays(uint32_t *keys, uint32_t *vals, uint2 *buf_a, uint2 *buf_b, uint32_t n, uint32_t key_bits,
+                       uint32_t *scratch, hipStream_t stream);
 
 // Device pointers of one resident scene (single scene or one slot pool).
 // Device forms of the soft constraints: the caller's records (cn_soft_edge, cn_soft_bend,
@@ -148,9 +151,9 @@ struct SceneBuffers {
     int4 *run_info = nullptr;       // (cx, cy, cz, pure)
     uint32_t *bucket = nullptr;     // (1 << bucket_bits) + 1
     uint32_t bucket_bits = 0;
-    uint32_t *block_runs = nullptr; // per 1024-element block, then scanned
-    uint32_t *run_count = nullptr;  // device scalar
-    uint32_t *perm = nullptr;
+    uint2 *tile_counts = nullptr;   // runs and blocks per 1024-key tile (scanned when there are many)
+    uint32_t *perm = nullptr;       // slot -> old slot (large scenes)
+    uint32_t *run_count = nullptr;  // [0] runs, [1] some cell lies outside its scene's window (kRunWords)
     // fluid solve
     float4 *dacc[2] = {nullptr, nullptr};
     float4 *curpos = nullptr;       // (x* + delta, D or kNoMass): neighbor positions of the walk
@@ -228,10 +231,13 @@ struct SceneBuffers {
 };
 
 // ---- broadphase + fluid launches (cn_kernels.hip) ----
-void launch_keys(const SceneBuffers &s, const SubstepConsts &c, hipStream_t st);
-void launch_runs(SceneBuffers &s, const SubstepConsts &c, const uint2 *sorted, uint32_t key_bits, hipStream_t st);
-void launch_reorder(SceneBuffers &s, const SubstepConsts &c, hipStream_t st);
-void launch_blocks(SceneBuffers &s, const SubstepConsts &c, hipStream_t st);
+constexpr uint32_t kRunWords = 2;
+// returns whether the lowest digit's sort counts were taken too
+bool launch_keys(const SceneBuffers &s, const SubstepConsts &c, hipStream_t st);
+// lookups: the run table will be searched (fluid, or contact candidates)
+void launch_runs(SceneBuffers &s, const SubstepConsts &c, const uint2 *sorted, uint32_t key_bits, bool lookups,
+                 hipStream_t st);
+void launch_reorder(SceneBuffers &s, const SubstepConsts &c, const uint2 *sorted, hipStream_t st);
 void fluid_tiles(SubstepConsts &c);
 void launch_blk_halo(const SceneBuffers &s, const SubstepConsts &c, hipStream_t st);
 void launch_fluid_density(const SceneBuffers &s, const SubstepConsts &c, uint32_t it, int din, hipStream_t st);

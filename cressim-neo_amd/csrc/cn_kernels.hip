@@ -55,110 +55,228 @@ __device__ __forceinline__ float scene_inv_cell(const SceneInfo &sc, const Subst
     return c.inv_cell > 0.0f ? c.inv_cell : sc.inv_cell;
 }
 
+// R > 0: a workgroup takes a sort tile of R rounds and counts its keys' lowest digit on the way
+// (the first histogram of the sort, laid out as k_radix_hist would).
+template <int R>
 __global__ __launch_bounds__(kBlock) void k_keys(const float4 *__restrict__ pos, const float4 *__restrict__ vel,
                                                  const uint32_t *__restrict__ cls,
                                                  const ParticleClass *__restrict__ classes,
                                                  const cn_fluid_material *__restrict__ fm,
                                                  const SceneInfo *__restrict__ scenes,
                                                  const uint32_t *__restrict__ active, SubstepConsts c,
-                                                 uint2 *__restrict__ kv)
+                                                 uint2 *__restrict__ kv, uint32_t *__restrict__ counts, uint32_t direct)
 {
-    const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
-    if (s >= c.n) return;
-    float4 p = pos[s], v = vel[s], pv;
-    const ParticleClass pc = classes[c.uniform_class ? 0u : cls[s]];
-    if (active[pc.scene]) predict(p, v, pv, gravity_scale(pc, fm), c);
-    const SceneInfo sc = scenes[pc.scene];
-    const int3 g = cell_of(p.x, p.y, p.z, scene_inv_cell(sc, c));
-    kv[s] = make_uint2(cell_key(g.x, g.y, g.z, sc.key_prefix, c.key_mode, c.morton_bits), s);
+    __shared__ uint32_t hist[256];
+    static_assert(kBlock == 256, "one thread per digit");
+    if (R > 0) {
+        hist[threadIdx.x] = 0;
+        __syncthreads();
+    }
+    constexpr int N = R > 0 ? R : 1, B = N < 4 ? N : 4;  // loads of B rounds in flight
+#pragma unroll 1
+    for (int r0 = 0; r0 < N; r0 += B) {
+        const uint32_t s0 = blockIdx.x * (kBlock * N) + r0 * kBlock + threadIdx.x;
+        float4 p[B], v[B];
+        uint32_t k[B];
+#pragma unroll
+        for (int u = 0; u < B; ++u) {
+            const uint32_t s = min(s0 + u * kBlock, c.n - 1u);
+            p[u] = pos[s];
+            v[u] = vel[s];
+            k[u] = c.uniform_class ? 0u : cls[s];
+        }
+#pragma unroll
+        for (int u = 0; u < B; ++u) {
+            const uint32_t s = s0 + u * kBlock;
+            if (s >= c.n) continue;
+            float4 pv;
+            const ParticleClass pc = classes[k[u]];
+            if (c.all_active || active[pc.scene]) predict(p[u], v[u], pv, gravity_scale(pc, fm), c);
+            const SceneInfo sc = scenes[pc.scene];
+            const int3 g = cell_of(p[u].x, p[u].y, p[u].z, scene_inv_cell(sc, c));
+            const uint32_t key = cell_key(g.x, g.y, g.z, sc.key_prefix, c.key_mode, c.morton_bits);
+            kv[s] = make_uint2(key, s);
+            if (R > 0) atomicAdd(&hist[key & 0xffu], 1u);
+        }
+    }
+    if (R > 0) {
+        __syncthreads();
+        counts[direct ? blockIdx.x * 256u + threadIdx.x : threadIdx.x * gridDim.x + blockIdx.x] = hist[threadIdx.x];
+    }
 }
 
-void launch_keys(const SceneBuffers &s, const SubstepConsts &c, hipStream_t st)
+bool launch_keys(const SceneBuffers &s, const SubstepConsts &c, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_keys, dim3(grid1(c.n)), dim3(kBlock), 0, st, s.pos[s.cur], s.vel[s.cur], s.cls[s.cur],
-                       s.classes, s.fluid_mats, s.scenes, s.scene_active, c, s.kv[0]);
+    const uint32_t rounds = sort_one_group(c.n) ? 0u : sort_rounds(c.n), per = kBlock * std::max(rounds, 1u);
+    const dim3 grid((c.n + per - 1) / per), block(kBlock);
+    const uint32_t direct = grid.x <= kDirectTiles ? 1u : 0u;
+    auto *k = rounds == 0u ? k_keys<0> : (rounds == 4u ? k_keys<4> : (rounds == 8u ? k_keys<8> : k_keys<16>));
+    hipLaunchKernelGGL(k, grid, block, 0, st, s.pos[s.cur], s.vel[s.cur], s.cls[s.cur], s.classes, s.fluid_mats,
+                       s.scenes, s.scene_active, c, s.kv[0], s.sort_scratch, direct);
+    return rounds > 0u;
 }
 
 // ---------------------------------------------------------------------------------------------
-// runs of equal keys: flags -> block counts -> scan -> run table, bucket index, rank fix-up
+// runs of equal keys and Morton blocks: flags -> tile counts -> (scan) -> run table, bucket index
 // ---------------------------------------------------------------------------------------------
+// Runs of equal keys and Morton blocks (runs grouped by key >> 6, aligned 4x4x4 cells: the tiles of
+// the LDS walk) come from one pass over the sorted keys: starts counted per tile of kRunTile keys,
+// then emitted.  A count holds runs in its low half and blocks in its high half.
 constexpr int kRunItems = 4;
 constexpr int kRunTile = kBlock * kRunItems;
 
-__device__ __forceinline__ bool run_flag(const uint2 *kv, uint32_t i, uint32_t n)
+// Bit 0: key i starts a run; bit 16: it starts a block too.
+__device__ __forceinline__ uint32_t start_flags(const uint2 *kv, uint32_t i, uint32_t n)
 {
-    return i < n && (i == 0 || kv[i].x != kv[i - 1].x);
+    if (i >= n) return 0u;
+    if (i == 0) return 0x10001u;
+    const uint32_t d = kv[i].x ^ kv[i - 1].x;
+    return (d ? 1u : 0u) | ((d >> 6) ? 0x10000u : 0u);
 }
 
 __global__ __launch_bounds__(kBlock) void k_run_count(const uint2 *__restrict__ kv, uint32_t n,
-                                                      uint32_t *__restrict__ block_runs)
+                                                      uint2 *__restrict__ tile_counts, uint32_t *__restrict__ nblk)
 {
-    __shared__ uint32_t sh[kBlock];
+    __shared__ uint32_t sh[kBlock / 64];
     const uint32_t base = blockIdx.x * kRunTile + threadIdx.x * kRunItems;
     uint32_t cnt = 0;
 #pragma unroll
-    for (int k = 0; k < kRunItems; ++k) cnt += run_flag(kv, base + k, n) ? 1u : 0u;
+    for (int k = 0; k < kRunItems; ++k) cnt += start_flags(kv, base + k, n);
     uint32_t total;
     block_exclusive_scan(cnt, sh, total);
-    if (threadIdx.x == 0) block_runs[blockIdx.x] = total;
+    if (threadIdx.x == 0) tile_counts[blockIdx.x] = make_uint2(total & 0xffffu, total >> 16);
+    if (blockIdx.x == 0 && threadIdx.x == 0) nblk[1] = 0u;  // set by the emit pass in a pool with fluid
 }
 
-// single workgroup: exclusive scan of the per-block run counts; total -> *run_count
-__global__ __launch_bounds__(1024) void k_scan_block_runs(uint32_t *__restrict__ v, uint32_t nb,
-                                                          uint32_t *__restrict__ run_count)
+// single workgroup: exclusive scan of the tiles' counts (more than kOwnPrefix tiles)
+__global__ __launch_bounds__(1024) void k_scan_tiles(uint2 *__restrict__ v, uint32_t nb)
 {
-    __shared__ uint32_t sh[1024];
+    __shared__ uint32_t sh[1024 / 64];
     const uint32_t t = threadIdx.x;
     const uint32_t per = (nb + 1023u) / 1024u;
     const uint32_t b0 = t * per;
-    uint32_t local = 0;
-    for (uint32_t k = 0; k < per; ++k)
-        if (b0 + k < nb) local += v[b0 + k];
-    sh[t] = local;
-    __syncthreads();
-    for (uint32_t off = 1; off < 1024; off <<= 1) {
-        const uint32_t add = t >= off ? sh[t - off] : 0u;
-        __syncthreads();
-        sh[t] += add;
-        __syncthreads();
-    }
-    uint32_t run = sh[t] - local;
+    uint2 local = make_uint2(0u, 0u);
     for (uint32_t k = 0; k < per; ++k)
         if (b0 + k < nb) {
-            const uint32_t x = v[b0 + k];
-            v[b0 + k] = run;
-            run += x;
+            local.x += v[b0 + k].x;
+            local.y += v[b0 + k].y;
         }
-    if (t == 1023) *run_count = sh[1023];
+    uint32_t total;
+    uint2 run;
+    run.x = block_exclusive_scan_wide<1024>(local.x, sh, total);
+    run.y = block_exclusive_scan_wide<1024>(local.y, sh, total);
+    for (uint32_t k = 0; k < per; ++k)
+        if (b0 + k < nb) {
+            const uint2 x = v[b0 + k];
+            v[b0 + k] = run;
+            run.x += x.x;
+            run.y += x.y;
+        }
 }
 
-__global__ __launch_bounds__(kBlock) void k_run_emit(const uint2 *__restrict__ kv, uint32_t n,
-                                                     const uint32_t *__restrict__ block_off,
-                                                     uint32_t *__restrict__ elem_run, uint32_t *__restrict__ run_key,
-                                                     uint32_t *__restrict__ run_start)
+// Up to kOwnPrefix tiles each emit workgroup sums the counts before it, which saves the scan's launch
+// (4 us of a small scene's substep); of more they are scanned first.
+constexpr uint32_t kOwnPrefix = 1024;
+struct EmitArgs {
+    const uint2 *kv;
+    uint32_t n;
+    const uint2 *tile_counts;
+    uint32_t scanned;
+    uint32_t *elem_run, *run_key, *run_start, *run_count;
+    uint32_t *blk_first_run, *nblk;
+    uint32_t prefix_shift, fluid_scenes;
+    uint32_t *work;  // the substep's queue counters (the max-displacement words past nwork are kept)
+    uint32_t nwork, last_word, prev_word;
+    uint32_t *meta;
+};
+
+// The end of the run of keys that holds position s, searched from the position `from` on.
+__device__ __forceinline__ uint32_t run_end(const uint2 *__restrict__ kv, uint32_t n, uint32_t s, uint32_t from)
 {
-    __shared__ uint32_t sh[kBlock];
+    const uint32_t key = kv[s].x;
+    if (from >= n || kv[from].x != key) return min(from, n);
+    uint32_t step = 1;
+    while (from + step < n && kv[from + step].x == key) step <<= 1;
+    uint32_t lo = from + (step >> 1), hi = min(from + step, n);  // kv[lo] is in the run, hi is past it
+    while (hi - lo > 1u) {
+        const uint32_t mid = lo + ((hi - lo) >> 1);
+        if (kv[mid].x == key) lo = mid;
+        else hi = mid;
+    }
+    return hi;
+}
+
+__global__ __launch_bounds__(kBlock) void k_run_emit(EmitArgs a)
+{
+    __shared__ uint32_t sh[kBlock / 64];
+    __shared__ uint32_t starts[kRunTile];  // of the tile's runs
+    const uint32_t n = a.n;
     const uint32_t base = blockIdx.x * kRunTile + threadIdx.x * kRunItems;
-    bool f[kRunItems];
+    uint32_t f[kRunItems];
     uint32_t cnt = 0;
 #pragma unroll
     for (int k = 0; k < kRunItems; ++k) {
-        f[k] = run_flag(kv, base + k, n);
-        cnt += f[k] ? 1u : 0u;
+        f[k] = start_flags(a.kv, base + k, n);
+        cnt += f[k];
     }
     uint32_t total;
-    uint32_t incl = block_off[blockIdx.x] + block_exclusive_scan(cnt, sh, total);
+    uint2 before;
+    if (a.scanned) {
+        before = a.tile_counts[blockIdx.x];
+    } else {
+        uint2 x = make_uint2(0u, 0u);
+        for (uint32_t k = threadIdx.x; k < blockIdx.x; k += kBlock) {
+            x.x += a.tile_counts[k].x;
+            x.y += a.tile_counts[k].y;
+        }
+        block_exclusive_scan(x.x, sh, before.x);
+        block_exclusive_scan(x.y, sh, before.y);
+    }
+    const uint32_t in_tile = block_exclusive_scan(cnt, sh, total);
+    uint32_t run = before.x + (in_tile & 0xffffu), blk = before.y + (in_tile >> 16);
+    if (blockIdx.x == 0 && threadIdx.x == 0) a.run_count[1] = 0u;  // raised by the reorder pass
 #pragma unroll
     for (int k = 0; k < kRunItems; ++k) {
         const uint32_t i = base + k;
         if (i >= n) break;
-        if (f[k]) {
-            run_key[incl] = kv[i].x;
-            run_start[incl] = i;
-            ++incl;
+        const uint32_t key = a.kv[i].x;
+        if (f[k] & 0x10000u) a.blk_first_run[blk++] = run;
+        if (f[k] & 1u) {
+            a.run_key[run] = key;
+            a.run_start[run] = i;
+            starts[run - before.x] = i;
+            ++run;
         }
-        elem_run[i] = incl - 1u;
-        if (i == n - 1) run_start[incl] = n;
+        a.elem_run[i] = run - 1u;
+        // scenes with fluid hold the lowest key prefixes, so their blocks come first: the last key of
+        // theirs tells their number
+        if ((uint32_t)((uint64_t)key >> a.prefix_shift) < a.fluid_scenes &&
+            (i == n - 1 || (uint32_t)((uint64_t)a.kv[i + 1].x >> a.prefix_shift) >= a.fluid_scenes))
+            a.nblk[1] = blk;
+        if (i == n - 1) {
+            a.run_start[run] = n;
+            a.run_count[0] = run;
+            a.blk_first_run[blk] = run;
+            a.nblk[0] = blk;
+        }
+    }
+    // the queue counters, cleared by every workgroup's share
+    for (uint32_t w = blockIdx.x * kBlock + threadIdx.x; w < a.nwork; w += gridDim.x * kBlock) a.work[w] = 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) a.work[a.prev_word] = a.work[a.last_word];
+    // the longest run: the tile's largest, and an atomic only when it beats the value already stored
+    // (one look at that word per tile: one per wave of particles cost 105 us of a launch at 4,194,304)
+    __syncthreads();
+    const uint32_t runs = total & 0xffffu;
+    uint32_t occ = 0;
+    for (uint32_t k = threadIdx.x; k < runs; k += kBlock)
+        occ = max(occ, (k + 1u < runs ? starts[k + 1u] : run_end(a.kv, n, starts[k], (blockIdx.x + 1u) * kRunTile)) - starts[k]);
+    for (int w = 32; w > 0; w >>= 1) occ = max(occ, (uint32_t)__shfl_xor((int)occ, w));
+    if ((threadIdx.x & 63u) == 0) sh[threadIdx.x >> 6] = occ;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int w = 1; w < kBlock / 64; ++w) occ = max(occ, sh[w]);
+        if (occ > __builtin_nontemporal_load(a.meta + 8)) atomicMax(a.meta + 8, occ);
     }
 }
 
@@ -180,41 +298,36 @@ __global__ __launch_bounds__(kBlock) void k_bucket_fill(const uint32_t *__restri
     bucket[b] = lo;
 }
 
-// Stable order inside a run is by particle index: rank = #run members with a smaller id.
-__global__ __launch_bounds__(kBlock) void k_rank_fix(const uint2 *__restrict__ kv, uint32_t n,
-                                                     const uint32_t *__restrict__ elem_run,
-                                                     const uint32_t *__restrict__ run_start,
-                                                     const uint32_t *__restrict__ id_old, uint32_t *__restrict__ perm)
+void launch_runs(SceneBuffers &s, const SubstepConsts &c, const uint2 *sorted, uint32_t key_bits, bool lookups,
+                 hipStream_t st)
 {
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t r = elem_run[i];
-    const uint32_t s = run_start[r], e = run_start[r + 1];
-    const uint32_t o = min(kv[i].y, n - 1u);
-    if (e - s == 1u) {
-        perm[i] = o;
-        return;
-    }
-    const uint32_t me = id_old[o];
-    uint32_t rank = 0;
-    for (uint32_t q = s; q < e; ++q) rank += id_old[min(kv[q].y, n - 1u)] < me ? 1u : 0u;
-    perm[s + rank] = o;
-}
-
-void launch_runs(SceneBuffers &s, const SubstepConsts &c, const uint2 *sorted, uint32_t key_bits, hipStream_t st)
-{
-    const uint32_t n = c.n;
-    const uint32_t nb = (n + kRunTile - 1) / kRunTile;
-    hipLaunchKernelGGL(k_run_count, dim3(nb), dim3(kBlock), 0, st, sorted, n, s.block_runs);
-    hipLaunchKernelGGL(k_scan_block_runs, dim3(1), dim3(1024), 0, st, s.block_runs, nb, s.run_count);
-    hipLaunchKernelGGL(k_run_emit, dim3(nb), dim3(kBlock), 0, st, sorted, n, s.block_runs, s.elem_run, s.run_key,
-                       s.run_start);
+    const uint32_t nb = (c.n + kRunTile - 1) / kRunTile;
+    EmitArgs a;
+    a.kv = sorted;
+    a.n = c.n;
+    a.tile_counts = s.tile_counts;
+    a.scanned = nb > kOwnPrefix ? 1u : 0u;
+    a.elem_run = s.elem_run;
+    a.run_key = s.run_key;
+    a.run_start = s.run_start;
+    a.run_count = s.run_count;
+    a.blk_first_run = s.blk_first_run;
+    a.nblk = s.nblk;
+    a.prefix_shift = 3u * c.morton_bits;
+    a.fluid_scenes = c.key_mode == CN_KEY_MORTON ? c.fluid_scenes : 0u;
+    a.work = s.iter_state;
+    a.nwork = kStateMaxDisp;
+    a.last_word = kStateMaxDisp + std::min<uint32_t>(std::max<uint32_t>(c.fluid_iters, 1u), kIterStateWords) - 1;
+    a.prev_word = kStatePrevDisp;
+    a.meta = s.meta;
+    hipLaunchKernelGGL(k_run_count, dim3(nb), dim3(kBlock), 0, st, sorted, c.n, s.tile_counts, s.nblk);
+    if (a.scanned) hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(1024), 0, st, s.tile_counts, nb);
+    hipLaunchKernelGGL(k_run_emit, dim3(nb), dim3(kBlock), 0, st, a);
+    if (!lookups) return;
     const uint32_t nbuckets = 1u << s.bucket_bits;
     const uint32_t shift = key_bits - s.bucket_bits;
     hipLaunchKernelGGL(k_bucket_fill, dim3((nbuckets + 1 + kBlock - 1) / kBlock), dim3(kBlock), 0, st, s.run_key,
                        s.run_count, shift, nbuckets, s.bucket);
-    hipLaunchKernelGGL(k_rank_fix, dim3(grid1(n)), dim3(kBlock), 0, st, sorted, n, s.elem_run, s.run_start,
-                       s.id[s.cur], s.perm);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -282,8 +395,46 @@ __device__ __forceinline__ uint32_t boundary_candidates(const ParticleClass &pc,
     return n ? kBndList | min(n, kBndListCap) : 0u;
 }
 
+// Stable order inside a run is by particle index: a particle's slot is the run's start plus the number
+// of its members with a smaller index (four of them compared per round trip).
+__device__ __forceinline__ uint32_t run_slot(const uint2 *__restrict__ kv, const uint32_t *__restrict__ id_o,
+                                             uint32_t rs, uint32_t re, uint32_t pid, uint32_t n)
+{
+    uint32_t t = rs;
+    for (uint32_t q = rs; q < re; q += 4) {
+        uint32_t other[4];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) other[u] = id_o[min(kv[min(q + u, re - 1u)].y, n - 1u)];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) t += q + u < re && other[u] < pid ? 1u : 0u;
+    }
+    return t;
+}
+
+// perm[slot] = old slot.  From kRankApart particles the ranks are taken in a pass of their own: at
+// 4,194,304 it and the gather take 185 us, the pass that does both 308 (its registers leave too few
+// waves to hide the ranks' dependent loads); below, one launch is the shorter.
+constexpr uint32_t kRankApart = 512u * 1024u;
+__global__ __launch_bounds__(kBlock) void k_rank(const uint2 *__restrict__ kv, uint32_t n,
+                                                 const uint32_t *__restrict__ elem_run,
+                                                 const uint32_t *__restrict__ run_start,
+                                                 const uint32_t *__restrict__ id_o, uint32_t *__restrict__ perm)
+{
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t r = elem_run[i], o = min(kv[i].y, n - 1u);
+    const uint32_t rs = run_start[r], re = run_start[r + 1];
+    perm[re - rs > 1u ? run_slot(kv, id_o, rs, re, id_o[o], n) : rs] = o;
+}
+
+// RANKED: one thread per slot, its particle from perm; otherwise one thread per sorted pair, which
+// finds its particle's slot itself.  The run's record is written by the member that comes first:
+// pure, as every cell of the scene's window is; a particle outside it raises run_count[1], and the
+// runs are then looked over one by one.
+template <bool RANKED>
 __global__ __launch_bounds__(kBlock) void k_reorder(
-    const uint32_t *__restrict__ perm, const float4 *__restrict__ pos_o, const float4 *__restrict__ vel_o,
+    const uint2 *__restrict__ kv, const uint32_t *__restrict__ perm, const uint32_t *__restrict__ elem_run, const uint32_t *__restrict__ run_start,
+    int4 *__restrict__ run_info, uint32_t *__restrict__ run_count, const float4 *__restrict__ pos_o, const float4 *__restrict__ vel_o,
     const uint32_t *__restrict__ cls_o, const uint32_t *__restrict__ id_o, float4 *__restrict__ pos_n,
     float4 *__restrict__ vel_n, uint32_t *__restrict__ cls_n, uint32_t *__restrict__ id_n,
     const float4 *__restrict__ prev_o, float4 *__restrict__ prev, float4 *__restrict__ cur,
@@ -293,158 +444,69 @@ __global__ __launch_bounds__(kBlock) void k_reorder(
     const SceneInfo *__restrict__ scenes, const uint32_t *__restrict__ active, uint32_t *__restrict__ meta,
     SubstepConsts c)
 {
-    const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
-    if (t >= c.n) return;
-    const uint32_t o = min(perm[t], c.n - 1u);  // perm is a permutation; the clamp only bounds reads
-    float4 p = pos_o[o], v = vel_o[o], pv;
-    const uint32_t k = cls_o[o];
-    const ParticleClass pc = classes[c.uniform_class ? 0u : k];
-    // a scene this step leaves untouched keeps its state; its particles only change slot
-    if (active[pc.scene]) predict(p, v, pv, gravity_scale(pc, fm), c);
-    else pv = prev_o[o];
-    pos_n[t] = p;
-    // solver position x* + delta with delta = 0 at the first iteration
-    cur[t] = make_float4(p.x, p.y, p.z, p.w > kEps ? 0.0f : kNoMass);
-    vel_n[t] = v;
-    prev[t] = pv;
-    cls_n[t] = k;
-    const uint32_t pid = id_o[o];
-    id_n[t] = pid;
-    if (slot_of) slot_of[min(pid, c.npid - 1u)] = t;
-    const SceneInfo sc = scenes[pc.scene];
-    const int3 g = cell_of(p.x, p.y, p.z, scene_inv_cell(sc, c));
-    // w: the scene's key prefix, from which neighbor-cell keys are formed
-    cellc[t] = make_int4(g.x, g.y, g.z, (int)sc.key_prefix);
-    // a scene with more than kMaskColliders colliders has groups, and the pool a list per slot
-    bnd[t] = boundary_candidates(pc, fm, col + sc.col0, bndl ? sc.ncol : min(sc.ncol, kMaskColliders),
-                                 grp + sc.grp0, bndl + (size_t)t * kBndListCap, meta, p.x, p.y, p.z);
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < c.n) {
+        const uint32_t r = elem_run[i];
+        const uint32_t o = min(RANKED ? perm[i] : kv[i].y, c.n - 1u);  // a permutation; the clamp only bounds reads
+        const uint32_t rs = run_start[r], re = run_start[r + 1];
+        float4 p = pos_o[o], v = vel_o[o], pv;
+        const uint32_t pid = id_o[o];
+        const uint32_t t = RANKED ? i : (re - rs > 1u ? run_slot(kv, id_o, rs, re, pid, c.n) : rs);
+        const uint32_t k = cls_o[o];
+        const ParticleClass pc = classes[c.uniform_class ? 0u : k];
+        // a scene this step leaves untouched keeps its state; its particles only change slot
+        if (active[pc.scene]) predict(p, v, pv, gravity_scale(pc, fm), c);
+        else pv = prev_o[o];
+        pos_n[t] = p;
+        // solver position x* + delta with delta = 0 at the first iteration
+        cur[t] = make_float4(p.x, p.y, p.z, p.w > kEps ? 0.0f : kNoMass);
+        vel_n[t] = v;
+        prev[t] = pv;
+        cls_n[t] = k;
+        id_n[t] = pid;
+        if (slot_of) slot_of[min(pid, c.npid - 1u)] = t;
+        const SceneInfo sc = scenes[pc.scene];
+        const int3 g = cell_of(p.x, p.y, p.z, scene_inv_cell(sc, c));
+        // w: the scene's key prefix, from which neighbor-cell keys are formed
+        cellc[t] = make_int4(g.x, g.y, g.z, (int)sc.key_prefix);
+        // a scene with more than kMaskColliders colliders has groups, and the pool a list per slot
+        bnd[t] = boundary_candidates(pc, fm, col + sc.col0, bndl ? sc.ncol : min(sc.ncol, kMaskColliders),
+                                     grp + sc.grp0, bndl + (size_t)t * kBndListCap, meta, p.x, p.y, p.z);
+        const uint32_t width = 1u << c.morton_bits;
+        if ((uint32_t)g.x - (uint32_t)sc.win[0] >= width || (uint32_t)g.y - (uint32_t)sc.win[1] >= width ||
+            (uint32_t)g.z - (uint32_t)sc.win[2] >= width)
+            run_count[1] = 1u;
+        if (t == rs) run_info[r] = make_int4(g.x, g.y, g.z, kRunPure);
+    }
 }
 
-// (cx, cy, cz, w): pure runs hold a single cell; mixed runs (hash collisions or wrapped
-// Morton coordinates) are filtered per particle like the reference (:94-98).  cls: the slots'
-// classes when the contact candidates want each run's one class (null otherwise).  The members are
-// read four at a time, so a run of a few particles costs one round trip.
+// Every run's record: hash keys, whose runs may hold several cells, and the contact candidates, which
+// want the runs' classes.
 __global__ __launch_bounds__(kBlock) void k_run_info(const uint32_t *__restrict__ run_start,
                                                      const uint32_t *__restrict__ run_count,
                                                      const int4 *__restrict__ cellc, const uint32_t *__restrict__ cls,
-                                                     int4 *__restrict__ run_info, uint32_t *__restrict__ meta)
+                                                     int4 *__restrict__ run_info)
 {
     const uint32_t r = blockIdx.x * kBlock + threadIdx.x;
-    uint32_t occ = 0;
-    if (r < *run_count) {
-        const uint32_t s = run_start[r], e = run_start[r + 1];
-        occ = e - s;
-        const int4 c0 = cellc[s];
-        const uint32_t k0 = cls ? cls[s] : 0u;
-        bool pure = true, one = cls != nullptr;
-        for (uint32_t q = s + 1; q < e && (pure || one); q += 4) {
-            int4 cq[4];
-            uint32_t kq[4];
-#pragma unroll
-            for (uint32_t u = 0; u < 4; ++u) {
-                const uint32_t i = min(q + u, e - 1u);
-                cq[u] = cellc[i];
-                kq[u] = cls ? cls[i] : 0u;
-            }
-#pragma unroll
-            for (uint32_t u = 0; u < 4; ++u) {
-                pure &= cq[u].x == c0.x && cq[u].y == c0.y && cq[u].z == c0.z;
-                one &= kq[u] == k0;
-            }
-        }
-        run_info[r] = make_int4(c0.x, c0.y, c0.z, (pure ? kRunPure : 0) | (one ? run_class_word(k0) : 0));
-    }
-    // longest run: wave maximum, and an atomic only when it beats the value already stored
-    for (int o = 32; o > 0; o >>= 1) occ = max(occ, (uint32_t)__shfl_xor((int)occ, o));
-    if ((threadIdx.x & 63u) == 0 && occ > __builtin_nontemporal_load(meta + 8)) atomicMax(meta + 8, occ);
+    if (r < *run_count) run_info[r] = run_record(run_start[r], run_start[r + 1], cellc, cls);
 }
 
-void launch_reorder(SceneBuffers &s, const SubstepConsts &c, hipStream_t st)
+void launch_reorder(SceneBuffers &s, const SubstepConsts &c, const uint2 *sorted, hipStream_t st)
 {
     const int o = s.cur, nw = 1 - s.cur;
-    hipLaunchKernelGGL(k_reorder, dim3(grid1(c.n)), dim3(kBlock), 0, st, s.perm, s.pos[o], s.vel[o], s.cls[o],
-                       s.id[o], s.pos[nw], s.vel[nw], s.cls[nw], s.id[nw], s.prev[o], s.prev[nw], s.curpos, s.cellc,
-                       s.bnd, s.bndl,
+    const bool apart = c.n >= kRankApart;
+    if (apart)
+        hipLaunchKernelGGL(k_rank, dim3(grid1(c.n)), dim3(kBlock), 0, st, sorted, c.n, s.elem_run, s.run_start, s.id[o],
+                           s.perm);
+    hipLaunchKernelGGL(apart ? k_reorder<true> : k_reorder<false>, dim3(grid1(c.n)), dim3(kBlock), 0, st, sorted, s.perm,
+                       s.elem_run, s.run_start, s.run_info, s.run_count, s.pos[o], s.vel[o], s.cls[o], s.id[o], s.pos[nw],
+                       s.vel[nw], s.cls[nw], s.id[nw], s.prev[o], s.prev[nw], s.curpos, s.cellc, s.bnd, s.bndl,
                        s.ne + s.nb + s.nd + s.nt ? s.slot_of : nullptr, s.classes, s.fluid_mats, s.colliders,
                        s.col_groups, s.scenes, s.scene_active, s.meta, c);
-    hipLaunchKernelGGL(k_run_info, dim3(grid1(c.n)), dim3(kBlock), 0, st, s.run_start, s.run_count, s.cellc,
-                       c.pairs ? s.cls[nw] : nullptr, s.run_info, s.meta);
+    if (c.key_mode == CN_KEY_HASH || c.pairs)
+        hipLaunchKernelGGL(k_run_info, dim3(grid1(c.n)), dim3(kBlock), 0, st, s.run_start, s.run_count, s.cellc,
+                           c.pairs ? s.cls[nw] : nullptr, s.run_info);
     s.cur = nw;
-}
-
-// ---------------------------------------------------------------------------------------------
-// Morton blocks: runs grouped by key >> 6 (aligned 4x4x4 cells), the tiles of the LDS walk
-// ---------------------------------------------------------------------------------------------
-__device__ __forceinline__ bool block_flag(const uint32_t *run_key, uint32_t r, uint32_t R)
-{
-    return r < R && (r == 0 || (run_key[r] >> 6) != (run_key[r - 1] >> 6));
-}
-
-__global__ __launch_bounds__(kBlock) void k_blk_count(const uint32_t *__restrict__ run_key,
-                                                      const uint32_t *__restrict__ run_count,
-                                                      uint32_t *__restrict__ block_cnt, uint32_t *__restrict__ nfluid)
-{
-    __shared__ uint32_t sh[kBlock];
-    if (blockIdx.x == 0 && threadIdx.x == 0) *nfluid = 0u;
-    const uint32_t R = *run_count;
-    const uint32_t base = blockIdx.x * kRunTile + threadIdx.x * kRunItems;
-    uint32_t cnt = 0;
-#pragma unroll
-    for (int k = 0; k < kRunItems; ++k) cnt += block_flag(run_key, base + k, R) ? 1u : 0u;
-    uint32_t total;
-    block_exclusive_scan(cnt, sh, total);
-    if (threadIdx.x == 0) block_cnt[blockIdx.x] = total;
-}
-
-__global__ __launch_bounds__(kBlock) void k_blk_emit(const uint32_t *__restrict__ run_key,
-                                                     const uint32_t *__restrict__ run_count,
-                                                     const uint32_t *__restrict__ block_off,
-                                                     uint32_t *__restrict__ blk_first_run,
-                                                     uint32_t *__restrict__ nblk, uint32_t *__restrict__ work,
-                                                     uint32_t nwork, uint32_t last_word, uint32_t prev_word,
-                                                     uint32_t prefix_shift, uint32_t fluid_scenes)
-{
-    __shared__ uint32_t sh[kBlock];
-    const uint32_t R = *run_count;
-    const uint32_t base = blockIdx.x * kRunTile + threadIdx.x * kRunItems;
-    bool f[kRunItems];
-    uint32_t cnt = 0;
-#pragma unroll
-    for (int k = 0; k < kRunItems; ++k) {
-        f[k] = block_flag(run_key, base + k, R);
-        cnt += f[k] ? 1u : 0u;
-    }
-    uint32_t total;
-    uint32_t idx = block_off[blockIdx.x] + block_exclusive_scan(cnt, sh, total);
-#pragma unroll
-    for (int k = 0; k < kRunItems; ++k) {
-        const uint32_t r = base + k;
-        if (r >= R) break;
-        if (f[k]) {
-            // scenes with fluid hold the lowest key prefixes, so their blocks come first
-            if ((uint32_t)((uint64_t)run_key[r] >> prefix_shift) < fluid_scenes) atomicMax(nblk + 1, idx + 1);
-            blk_first_run[idx++] = r;
-        }
-        if (r == R - 1) {
-            blk_first_run[idx] = R;
-            *nblk = idx;
-        }
-    }
-    // the substep's queue counters, cleared by every workgroup's share (the max-displacement words
-    // past nwork are kept)
-    for (uint32_t w = blockIdx.x * kBlock + threadIdx.x; w < nwork; w += gridDim.x * kBlock) work[w] = 0;
-    if (blockIdx.x == 0 && threadIdx.x == 0) work[prev_word] = work[last_word];
-}
-
-void launch_blocks(SceneBuffers &s, const SubstepConsts &c, hipStream_t st)
-{
-    const uint32_t nb = (c.n + kRunTile - 1) / kRunTile;
-    hipLaunchKernelGGL(k_blk_count, dim3(nb), dim3(kBlock), 0, st, s.run_key, s.run_count, s.block_runs, s.nblk + 1);
-    hipLaunchKernelGGL(k_scan_block_runs, dim3(1), dim3(1024), 0, st, s.block_runs, nb, s.nblk);
-    const uint32_t last = kStateMaxDisp + std::min<uint32_t>(std::max<uint32_t>(c.fluid_iters, 1u), kIterStateWords) - 1;
-    hipLaunchKernelGGL(k_blk_emit, dim3(nb), dim3(kBlock), 0, st, s.run_key, s.run_count, s.block_runs,
-                       s.blk_first_run, s.nblk, s.iter_state, kStateMaxDisp, last, kStatePrevDisp, 3u * c.morton_bits,
-                       c.fluid_scenes);
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -22,6 +22,34 @@ constexpr int kRunPure = 1;
 __device__ __forceinline__ int run_class_word(uint32_t cls) { return (int)((cls + 1u) << 1); }
 __device__ __forceinline__ uint32_t run_class(int w) { return ((uint32_t)w >> 1) - 1u; }  // kInvalid: differ
 
+// The record of run r from its members: (cx, cy, cz, w).  Pure runs hold a single cell; mixed runs
+// (hash collisions or wrapped Morton coordinates) are filtered per particle like the reference
+// (:94-98).  cls: the slots' classes when the contact candidates want each run's one class (null
+// otherwise).  The members are read four at a time, so a run of a few particles costs one round trip.
+__device__ __forceinline__ int4 run_record(uint32_t s, uint32_t e, const int4 *__restrict__ cellc,
+                                           const uint32_t *__restrict__ cls)
+{
+    const int4 c0 = cellc[s];
+    const uint32_t k0 = cls ? cls[s] : 0u;
+    bool pure = true, one = cls != nullptr;
+    for (uint32_t q = s + 1; q < e && (pure || one); q += 4) {
+        int4 cq[4];
+        uint32_t kq[4];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+            const uint32_t i = min(q + u, e - 1u);
+            cq[u] = cellc[i];
+            kq[u] = cls ? cls[i] : 0u;
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+            pure &= cq[u].x == c0.x && cq[u].y == c0.y && cq[u].z == c0.z;
+            one &= kq[u] == k0;
+        }
+    }
+    return make_int4(c0.x, c0.y, c0.z, (pure ? kRunPure : 0) | (one ? run_class_word(k0) : 0));
+}
+
 // The run of a key: a binary search of its bucket's runs.  A bucket is a range of keys, so where a
 // scene fills a corner of its key range (a pool whose key holds the scene, a small body in a large
 // box) one bucket holds hundreds of runs: the linear scan it replaces made the 48-scene pool's halo
