@@ -217,11 +217,53 @@ def hip_runtimes_mapped() -> list:
     return sorted(seen)
 
 
+class _PhdrInfo(C.Structure):
+    _fields_ = [("addr", C.c_void_p), ("name", C.c_char_p), ("phdr", C.c_void_p), ("phnum", C.c_uint16),
+                ("adds", C.c_ulonglong), ("subs", C.c_ulonglong)]
+
+
+_phdr_adds = C.c_ulonglong()
+
+
+@C.CFUNCTYPE(C.c_int, C.POINTER(_PhdrInfo), C.c_size_t, C.c_void_p)
+def _first_phdr(info, size, _):
+    _phdr_adds.value = info.contents.adds if size >= C.sizeof(_PhdrInfo) else 0
+    return 1  # the counter is the same in every record
+
+
+try:
+    _iterate_phdr = C.CDLL(None).dl_iterate_phdr
+except (AttributeError, OSError):  # pragma: no cover - another libc
+    _iterate_phdr = None
+
+
+def objects_loaded() -> int | None:
+    """How many shared objects this process has loaded since it started (the dynamic linker's own
+    counter), or None where the linker does not tell."""
+    if _iterate_phdr is None:
+        return None
+    _iterate_phdr(_first_phdr, None)
+    return _phdr_adds.value or None
+
+
+_single_at = None  # objects_loaded() when one runtime was last found mapped
+
+
 def require_single_hip_runtime(what: str):
     """Raises CnLibraryError when two HIP runtimes are mapped: device pointers and streams of one
-    are not valid in the other, so handing the library's buffers to torch would be undefined."""
+    are not valid in the other, so handing the library's buffers to torch would be undefined.
+
+    Reading /proc/self/maps takes about a millisecond in a process that has torch loaded (it was most
+    of a small scene's frame); a call that finds the linker's count of loaded objects where the last
+    passed check found it looks no further, since a second runtime can only come with a load."""
+    global _single_at
+    loaded = objects_loaded()
+    if loaded is not None and loaded == _single_at:
+        return
     rts = hip_runtimes_mapped()
-    if len(rts) > 1:
+    if len(rts) <= 1:
+        _single_at = loaded
+    else:
         raise CnLibraryError(
             f"{what}: two HIP runtimes are mapped ({', '.join(rts)}); load libcn_hip.so through "
             "cnhip.load_library() (which maps torch's runtime first) or import torch before loading it")

@@ -78,3 +78,24 @@ def test_uploads_refused_while_views_alive(call):
     args = {"upload": (None,), "upload_batch": ([],), "reserve": (100, 64)}[call]
     with pytest.raises(RuntimeError, match="release the exported tensor views"):
         getattr(s, call)(*args)
+
+
+@needs_lib
+def test_single_runtime_check_notices_a_later_load(tmp_path):
+    """The check skips the maps while no object has been loaded since it last passed, and looks again
+    after one has: a second runtime (here any shared object under a runtime's name) is refused."""
+    import _ctypes
+    fake = tmp_path / "libamdhip64.so.9"
+    fake.write_bytes(open(_ctypes.__file__, "rb").read())
+    body = ("import cnhip, ctypes\ncnhip.load_library()\nimport torch\n"
+            "from cnhip import abi\n"
+            "abi.require_single_hip_runtime('x')\nreads = []\nreal = abi.hip_runtimes_mapped\n"
+            "abi.hip_runtimes_mapped = lambda: reads.append(1) or real()\n"
+            "abi.require_single_hip_runtime('x')\nassert not reads, 'looked again without a load'\n"
+            f"ctypes.CDLL({str(fake)!r})\n"
+            "for _ in range(2):\n"
+            "    try:\n        abi.require_single_hip_runtime('x')\n        print('NOT_REFUSED')\n"
+            "    except abi.CnLibraryError:\n        print('REFUSED')\n")
+    out = subprocess.run([sys.executable, "-c", MAPPED.format(pkg=PKG, body=body)], capture_output=True, text=True,
+                         timeout=300, check=True).stdout
+    assert out.count("REFUSED") == 2 and "NOT_REFUSED" not in out
