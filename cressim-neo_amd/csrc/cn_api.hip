@@ -177,6 +177,44 @@ uint32_t ceil_log2(uint64_t v)
     return b;
 }
 
+void free_constraints(SceneBuffers &s)
+{
+    dfree(s.edges);
+    dfree(s.bends);
+    dfree(s.dihedrals);
+    dfree(s.tets);
+    dfree(s.lam);
+    dfree(s.corr);
+    dfree(s.inc);
+    dfree(s.posi);
+    dfree(s.soft_ids);
+    dfree(s.rigid_pick);
+    dfree(s.soft_tiles);
+    dfree(s.soft_own);
+    dfree(s.soft_halo);
+    dfree(s.soft_starts);
+    dfree(s.soft_ent);
+    dfree(s.soft_prm);
+    dfree(s.lam2);
+    s.soft_tiles = nullptr;
+    s.soft_own = s.soft_halo = s.soft_ent = nullptr;
+    s.soft_starts = nullptr;
+    s.soft_prm = nullptr;
+    s.lam2 = nullptr;
+    s.posi = nullptr;
+    s.soft_ids = nullptr;
+    s.rigid_pick = nullptr;
+    s.nsoft = 0;
+    s.edges = nullptr;
+    s.bends = nullptr;
+    s.dihedrals = nullptr;
+    s.tets = nullptr;
+    s.lam = nullptr;
+    s.corr = nullptr;
+    s.inc = nullptr;
+    s.ne = s.nb = s.nd = s.nt = 0;
+}
+
 void free_scene(SceneBuffers &s)
 {
     for (int k = 0; k < 2; ++k) {
@@ -239,16 +277,7 @@ void free_scene(SceneBuffers &s)
     dfree(s.scenes);
     dfree(s.meta);
     dfree(s.slot_of);
-    dfree(s.posi);
-    dfree(s.soft_ids);
-    dfree(s.rigid_pick);
-    dfree(s.edges);
-    dfree(s.bends);
-    dfree(s.dihedrals);
-    dfree(s.tets);
-    dfree(s.lam);
-    dfree(s.corr);
-    dfree(s.inc);
+    free_constraints(s);
     s = SceneBuffers{};
 }
 
@@ -259,32 +288,6 @@ void clear_graphs(cn_ctx *ctx)
         if (g.graph) (void)hipGraphDestroy(g.graph);
     }
     ctx->graphs.clear();
-}
-
-void free_constraints(SceneBuffers &s)
-{
-    dfree(s.edges);
-    dfree(s.bends);
-    dfree(s.dihedrals);
-    dfree(s.tets);
-    dfree(s.lam);
-    dfree(s.corr);
-    dfree(s.inc);
-    dfree(s.posi);
-    dfree(s.soft_ids);
-    dfree(s.rigid_pick);
-    s.posi = nullptr;
-    s.soft_ids = nullptr;
-    s.rigid_pick = nullptr;
-    s.nsoft = 0;
-    s.edges = nullptr;
-    s.bends = nullptr;
-    s.dihedrals = nullptr;
-    s.tets = nullptr;
-    s.lam = nullptr;
-    s.corr = nullptr;
-    s.inc = nullptr;
-    s.ne = s.nb = s.nd = s.nt = 0;
 }
 
 // Particle -> incident constraints, ascending constraint order (physics_scene_gpu_state.cpp:3273-3360);
@@ -980,6 +983,86 @@ cn_status check_scene(cn_ctx *ctx, const cn_scene_desc &d)
     return CN_OK;
 }
 
+// (rest value, compliance) of constraints [first, first + count) of group g, from the host copies of
+// their device forms.
+void soft_params(const cn_ctx *ctx, int g, uint32_t first, uint32_t count, std::vector<float2> &out)
+{
+    const uint32_t nb = (uint32_t)ctx->bends_host.size();
+    out.resize(count);
+    for (uint32_t k = 0; k < count; ++k) {
+        const uint32_t c = first + k;
+        if (g == 0) out[k] = make_float2(ctx->edges_host[c].rest_length, ctx->edges_host[c].compliance);
+        else if (g == 2) out[k] = make_float2(ctx->tets_host[c].rest_volume, ctx->tets_host[c].compliance);
+        else if (c < nb) out[k] = make_float2(ctx->bends_host[c].rest_angle, ctx->bends_host[c].compliance);
+        else out[k] = make_float2(ctx->dih_host[c - nb].rest_angle, ctx->dih_host[c - nb].compliance);
+    }
+}
+
+// Uploads the tiles of the soft-constraint passes.
+cn_status upload_tiles(cn_ctx *ctx, uint32_t n, const SoftTopology &topo, SoftTilesHost &h)
+{
+    SceneBuffers &s = ctx->s;
+    // the groups' tables one after another
+    size_t ntile = 0, nhalo = 0, nstart = 0, nent = 0;
+    for (int g = 0; g < 3; ++g) {
+        SoftTilesHost::Group &G = h.group[g];
+        for (SoftTile &t : G.tiles) {
+            t.halo0 += (uint32_t)nhalo;
+            t.start0 += (uint32_t)nstart;
+        }
+        s.soft_ntiles[g] = (uint32_t)G.tiles.size();
+        s.soft_lds[g] = G.lds;
+        const size_t part[3] = {G.con.size(), G.verts.size(), G.slots.size()};
+        for (int k = 0; k < 3; ++k) {
+            s.soft_ent_off[g][k] = nent;
+            nent += part[k];
+        }
+        ntile += G.tiles.size();
+        nhalo += G.halo.size();
+        nstart += G.starts.size();
+    }
+    auto put = [](auto *dst, const auto &v) {
+        return v.empty() ? hipSuccess : hipMemcpy(dst, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice);
+    };
+    CN_HIP(ctx, dalloc(&s.soft_own, h.own.size()));
+    CN_HIP(ctx, dalloc(&s.soft_halo, nhalo));
+    CN_HIP(ctx, dalloc(&s.soft_starts, nstart));
+    CN_HIP(ctx, dalloc(&s.soft_ent, nent));
+    CN_HIP(ctx, put(s.soft_own, h.own));
+    nhalo = nstart = 0;
+    for (int g = 0; g < 3; ++g) {
+        const SoftTilesHost::Group &G = h.group[g];
+        CN_HIP(ctx, put(s.soft_halo + nhalo, G.halo));
+        CN_HIP(ctx, put(s.soft_starts + nstart, G.starts));
+        CN_HIP(ctx, put(s.soft_ent + s.soft_ent_off[g][0], G.con));
+        CN_HIP(ctx, put(s.soft_ent + s.soft_ent_off[g][1], G.verts));
+        CN_HIP(ctx, put(s.soft_ent + s.soft_ent_off[g][2], G.slots));
+        nhalo += G.halo.size();
+        nstart += G.starts.size();
+    }
+    std::vector<float2> prm, part;
+    prm.reserve((size_t)topo.count[0] + topo.count[1] + topo.count[2]);
+    for (int g = 0; g < 3; ++g) {
+        soft_params(ctx, g, 0, topo.count[g], part);
+        prm.insert(prm.end(), part.begin(), part.end());
+    }
+    CN_HIP(ctx, dalloc(&s.soft_prm, prm.size()));
+    CN_HIP(ctx, put(s.soft_prm, prm));
+    CN_HIP(ctx, dalloc(&s.lam2, prm.size()));
+    CN_HIP(ctx, dalloc(&s.posi, 2 * (size_t)n));
+    CN_HIP(ctx, dalloc(&s.corr, 4 * (size_t)s.nt));
+    if (s.nt) CN_HIP(ctx, hipMemset(s.corr, 0, 4 * (size_t)s.nt * sizeof(CorrRec)));
+    for (uint32_t k = 0; k < ctx->nscenes; ++k) ctx->scene_info[k].soft_stages = h.stages[k];
+    CN_HIP(ctx, hipMemcpy(s.scenes, ctx->scene_info.data(), ctx->nscenes * sizeof(SceneInfo), hipMemcpyHostToDevice));
+    CN_HIP(ctx, dalloc(&s.soft_tiles, ntile));
+    ntile = 0;
+    for (int g = 0; g < 3; ++g) {
+        CN_HIP(ctx, put(s.soft_tiles + ntile, h.group[g].tiles));
+        ntile += h.group[g].tiles.size();
+    }
+    return CN_OK;
+}
+
 // Uploads a pool of independent scenes: particles, classes, materials and constraints are
 // concatenated with index offsets, colliders are visit-ordered per scene, and each scene gets its
 // own cell size and key range.  One scene is the plain path.
@@ -1022,10 +1105,16 @@ cn_status upload_pool(cn_ctx *ctx, uint32_t count, const cn_scene_desc *descs)
     std::vector<Collider> col;
     std::vector<ColGroup> groups;  // candidate groups of the scenes of more than kMaskColliders colliders
     std::vector<SceneInfo> sinfo(count);
-    std::vector<cn_soft_edge> edges;
-    std::vector<cn_soft_bend> bends;
-    std::vector<cn_cloth_dihedral> dih;
-    std::vector<cn_soft_tet> tets;
+    // device forms of the constraints: padding dropped, max(compliance, 0) and max(rest volume, 0) taken
+    // here, a disabled edge carried as a NaN compliance
+    std::vector<EdgeDev> edges;
+    std::vector<BendDev> bends;
+    std::vector<DihedralDev> dih;
+    std::vector<TetDev> tets;
+    edges.reserve(ne);
+    bends.reserve(nb);
+    dih.reserve(nd);
+    tets.reserve(nt);
     std::map<std::array<uint32_t, 9>, uint32_t> cmap;
     std::vector<ParticleClass> classes;
     std::vector<uint32_t> cls(n);
@@ -1177,32 +1266,10 @@ cn_status upload_pool(cn_ctx *ctx, uint32_t count, const cn_scene_desc *descs)
         ctx->scene_con[4 * k + 2] = (uint32_t)dih.size();
         ctx->scene_con[4 * k + 3] = (uint32_t)tets.size();
         if (cv) {
-            for (uint32_t e = 0; e < cv->edge_count; ++e) {
-                cn_soft_edge E = cv->edges[e];
-                E.a += base;
-                E.b += base;
-                edges.push_back(E);
-            }
-            for (uint32_t q = 0; q < cv->bend_count; ++q) {
-                cn_soft_bend B = cv->bends[q];
-                B.p0 += base;
-                B.p1 += base;
-                B.p2 += base;
-                bends.push_back(B);
-            }
-            for (uint32_t q = 0; q < cv->dihedral_count; ++q) {
-                cn_cloth_dihedral D = cv->dihedrals[q];
-                D.e0 += base;
-                D.e1 += base;
-                D.o0 += base;
-                D.o1 += base;
-                dih.push_back(D);
-            }
-            for (uint32_t t = 0; t < cv->tet_count; ++t) {
-                cn_soft_tet T = cv->tets[t];
-                for (int j = 0; j < 4; ++j) T.p[j] += base;
-                tets.push_back(T);
-            }
+            for (uint32_t e = 0; e < cv->edge_count; ++e) edges.push_back(edge_dev(cv->edges[e], base));
+            for (uint32_t q = 0; q < cv->bend_count; ++q) bends.push_back(bend_dev(cv->bends[q], base));
+            for (uint32_t q = 0; q < cv->dihedral_count; ++q) dih.push_back(dihedral_dev(cv->dihedrals[q], base));
+            for (uint32_t t = 0; t < cv->tet_count; ++t) tets.push_back(tet_dev(cv->tets[t], base));
         }
         // grid cell size of the scene (recomputeParticleGridCellSize) and its extent in cells
         const float cell = cn_particle_grid_cell_size(m, pv->radii, pv->fluid_material_indices,
@@ -1396,87 +1463,92 @@ cn_status upload_pool(cn_ctx *ctx, uint32_t count, const cn_scene_desc *descs)
         s.nb = (uint32_t)bends.size();
         s.nd = (uint32_t)dih.size();
         s.nt = (uint32_t)tets.size();
-        CN_HIP(ctx, dalloc(&s.edges, s.ne));
-        CN_HIP(ctx, dalloc(&s.bends, s.nb));
-        CN_HIP(ctx, dalloc(&s.dihedrals, s.nd));
-        CN_HIP(ctx, dalloc(&s.tets, s.nt));
+        ctx->edges_host = std::move(edges);
+        ctx->bends_host = std::move(bends);
+        ctx->dih_host = std::move(dih);
+        ctx->tets_host = std::move(tets);
+        // the constrained particles
+        const SoftTopology topo{ctx->edges_host.data(), ctx->bends_host.data(), ctx->dih_host.data(),
+                                ctx->tets_host.data(), s.nb, {s.ne, s.nb + s.nd, s.nt}};
+        std::vector<uint32_t> soft, scene_of(n);
         {
-            // device forms: padding dropped, max(compliance, 0) and max(rest volume, 0) taken here,
-            // a disabled edge carried as a NaN compliance
-            std::vector<EdgeDev> de(s.ne);
-            for (uint32_t e = 0; e < s.ne; ++e) de[e] = edge_dev(edges[e], 0);
-            std::vector<BendDev> db(s.nb);
-            for (uint32_t q = 0; q < s.nb; ++q) db[q] = bend_dev(bends[q], 0);
-            std::vector<DihedralDev> dd(s.nd);
-            for (uint32_t q = 0; q < s.nd; ++q) dd[q] = dihedral_dev(dih[q], 0);
-            std::vector<TetDev> dt(s.nt);
-            for (uint32_t t = 0; t < s.nt; ++t) dt[t] = tet_dev(tets[t], 0);
-            if (s.ne) CN_HIP(ctx, hipMemcpy(s.edges, de.data(), s.ne * sizeof(EdgeDev), hipMemcpyHostToDevice));
-            if (s.nb) CN_HIP(ctx, hipMemcpy(s.bends, db.data(), s.nb * sizeof(BendDev), hipMemcpyHostToDevice));
-            if (s.nd) CN_HIP(ctx, hipMemcpy(s.dihedrals, dd.data(), s.nd * sizeof(DihedralDev), hipMemcpyHostToDevice));
-            if (s.nt) CN_HIP(ctx, hipMemcpy(s.tets, dt.data(), s.nt * sizeof(TetDev), hipMemcpyHostToDevice));
-            ctx->edges_host = std::move(de);
-            ctx->bends_host = std::move(db);
-            ctx->dih_host = std::move(dd);
-            ctx->tets_host = std::move(dt);
+            std::vector<uint8_t> held[3];
+            auto mark = [&](int g) {
+                held[g].assign(n, 0);
+                for (uint32_t c = 0; c < topo.count[g]; ++c)
+                    for (uint32_t k = 0; k < (g == 0 ? 2u : 4u); ++k) {
+                        const uint32_t p = topo.vertex(g, c, k);
+                        if (p < n) held[g][p] = 1;
+                    }
+            };
+            std::future<void> edges_held = run_aside([&] { mark(0); }), tets_held = run_aside([&] { mark(2); });
+            mark(1);
+            edges_held.get();
+            tets_held.get();
+            for (uint32_t k = 0; k < ctx->nscenes; ++k)
+                for (uint32_t i = ctx->scene_first[k]; i < ctx->scene_first[k + 1]; ++i) {
+                    scene_of[i] = k;
+                    if (held[0][i] | held[1][i] | held[2][i]) soft.push_back(i);
+                }
         }
+        SoftTilesHost tiles;
         const size_t nlam = (size_t)s.ne + s.nb + s.nd + s.nt;
         CN_HIP(ctx, dalloc(&s.lam, nlam));
-        std::vector<uint32_t> inc, map_e, map_b, map_t;
-        size_t refs[3] = {0, 0, 0};
-        {
-            const uint32_t cnt[1] = {s.ne}, ar[1] = {2}, off[1] = {0};
-            build_incidence(n, 1, cnt, ar, off, [&](uint32_t, uint32_t c, uint32_t k) { return k == 0 ? edges[c].a : edges[c].b; },
-                            inc, s.inc_off[0], s.inc_off[1], map_e, 2u, refs[0]);
-        }
-        {
-            const uint32_t cnt[2] = {s.nb, s.nd}, ar[2] = {3, 4}, off[2] = {0, s.nb};
-            build_incidence(n, 2, cnt, ar, off,
-                            [&](uint32_t g, uint32_t c, uint32_t k) {
-                                if (g == 0) {
-                                    const cn_soft_bend &B = bends[c];
-                                    return k == 0 ? B.p0 : (k == 1 ? B.p1 : B.p2);
-                                }
-                                const cn_cloth_dihedral &D = dih[c];
-                                return k == 0 ? D.e0 : (k == 1 ? D.e1 : (k == 2 ? D.o0 : D.o1));
-                            },
-                            inc, s.inc_off[2], s.inc_off[3], map_b, 4u, refs[1]);
-        }
-        {
-            const uint32_t cnt[1] = {s.nt}, ar[1] = {4}, off[1] = {0};
-            build_incidence(n, 1, cnt, ar, off, [&](uint32_t, uint32_t c, uint32_t k) { return tets[c].p[k]; }, inc,
-                            s.inc_off[4], s.inc_off[5], map_t, 4u, refs[2]);
-        }
-        // record maps after the incidence structures; records of each group in CSR order + a spare
-        s.inc_off[6] = inc.size();
-        inc.insert(inc.end(), map_e.begin(), map_e.end());
-        s.inc_off[7] = inc.size();
-        inc.insert(inc.end(), map_b.begin(), map_b.end());
-        s.inc_off[8] = inc.size();
-        inc.insert(inc.end(), map_t.begin(), map_t.end());
-        s.corr_off[0] = 0;
-        s.corr_off[1] = refs[0] + 1;
-        s.corr_off[2] = s.corr_off[1] + refs[1] + 1;
-        const size_t ncorr = s.corr_off[2] + refs[2] + 1;
-        CN_HIP(ctx, dalloc(&s.corr, ncorr));
-        CN_HIP(ctx, hipMemset(s.corr, 0, ncorr * sizeof(CorrRec)));
-        // constrained particles: any incidence in the three structures
-        {
-            std::vector<uint32_t> soft;
-            for (uint32_t i = 0; i < n; ++i) {
-                bool any = false;
-                for (int g = 0; g < 3; ++g) any |= inc[s.inc_off[2 * g] + i + 1] != inc[s.inc_off[2 * g] + i];
-                if (any) soft.push_back(i);
-            }
-            s.nsoft = (uint32_t)soft.size();
-            CN_HIP(ctx, dalloc(&s.soft_ids, soft.size()));
-            CN_HIP(ctx, dalloc(&s.rigid_pick, soft.size()));
-            if (!soft.empty())
-                CN_HIP(ctx, hipMemcpy(s.soft_ids, soft.data(), soft.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+        s.nsoft = (uint32_t)soft.size();
+        CN_HIP(ctx, dalloc(&s.soft_ids, soft.size()));
+        CN_HIP(ctx, dalloc(&s.rigid_pick, soft.size()));
+        if (!soft.empty())
+            CN_HIP(ctx, hipMemcpy(s.soft_ids, soft.data(), soft.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+        if (build_soft_tiles(n, pos.data(), soft, scene_of.data(), ctx->nscenes, topo, tiles)) {
+            const cn_status st = upload_tiles(ctx, n, topo, tiles);
+            if (st != CN_OK) return st;
+        } else {
             CN_HIP(ctx, dalloc(&s.posi, n));
+            CN_HIP(ctx, dalloc(&s.edges, s.ne));
+            CN_HIP(ctx, dalloc(&s.bends, s.nb));
+            CN_HIP(ctx, dalloc(&s.dihedrals, s.nd));
+            CN_HIP(ctx, dalloc(&s.tets, s.nt));
+            auto put = [](auto *dst, const auto &v) {
+                return v.empty() ? hipSuccess : hipMemcpy(dst, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice);
+            };
+            CN_HIP(ctx, put(s.edges, ctx->edges_host));
+            CN_HIP(ctx, put(s.bends, ctx->bends_host));
+            CN_HIP(ctx, put(s.dihedrals, ctx->dih_host));
+            CN_HIP(ctx, put(s.tets, ctx->tets_host));
+            std::vector<uint32_t> inc, map_e, map_b, map_t;
+            size_t refs[3] = {0, 0, 0};
+            {
+                const uint32_t cnt[1] = {s.ne}, ar[1] = {2}, off[1] = {0};
+                build_incidence(n, 1, cnt, ar, off, [&](uint32_t, uint32_t c, uint32_t k) { return topo.vertex(0, c, k); },
+                                inc, s.inc_off[0], s.inc_off[1], map_e, 2u, refs[0]);
+            }
+            {
+                const uint32_t cnt[2] = {s.nb, s.nd}, ar[2] = {3, 4}, off[2] = {0, s.nb};
+                build_incidence(n, 2, cnt, ar, off,
+                                [&](uint32_t g, uint32_t c, uint32_t k) { return topo.vertex(1, c + off[g], k); }, inc,
+                                s.inc_off[2], s.inc_off[3], map_b, 4u, refs[1]);
+            }
+            {
+                const uint32_t cnt[1] = {s.nt}, ar[1] = {4}, off[1] = {0};
+                build_incidence(n, 1, cnt, ar, off, [&](uint32_t, uint32_t c, uint32_t k) { return topo.vertex(2, c, k); },
+                                inc, s.inc_off[4], s.inc_off[5], map_t, 4u, refs[2]);
+            }
+            // record maps after the incidence structures; records of each group in CSR order + a spare
+            s.inc_off[6] = inc.size();
+            inc.insert(inc.end(), map_e.begin(), map_e.end());
+            s.inc_off[7] = inc.size();
+            inc.insert(inc.end(), map_b.begin(), map_b.end());
+            s.inc_off[8] = inc.size();
+            inc.insert(inc.end(), map_t.begin(), map_t.end());
+            s.corr_off[0] = 0;
+            s.corr_off[1] = refs[0] + 1;
+            s.corr_off[2] = s.corr_off[1] + refs[1] + 1;
+            const size_t ncorr = s.corr_off[2] + refs[2] + 1;
+            CN_HIP(ctx, dalloc(&s.corr, ncorr));
+            CN_HIP(ctx, hipMemset(s.corr, 0, ncorr * sizeof(CorrRec)));
+            CN_HIP(ctx, dalloc(&s.inc, inc.size()));
+            CN_HIP(ctx, hipMemcpy(s.inc, inc.data(), inc.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
         }
-        CN_HIP(ctx, dalloc(&s.inc, inc.size()));
-        CN_HIP(ctx, hipMemcpy(s.inc, inc.data(), inc.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
         dfree(s.slot_of);
         s.slot_of = nullptr;
         CN_HIP(ctx, dalloc(&s.slot_of, std::max<uint32_t>(ctx->capacity, n)));
@@ -1559,32 +1631,54 @@ void record_step(cn_ctx *ctx, SceneBuffers &s, const cn_step_params *p)
         sa.n = s.npid;
         sa.dt = dt;
         sa.relax = p->solver_config[kCfgSoftRelax];
-        sa.edges = s.edges;
         sa.ne = s.ne;
-        sa.bends = s.bends;
         sa.nb = s.nb;
-        sa.dih = s.dihedrals;
         sa.nd = s.nd;
-        sa.tets = s.tets;
         sa.nt = s.nt;
-        sa.lam_e = s.lam;
-        sa.lam_b = s.lam + s.ne;
-        sa.lam_t = s.lam + s.ne + s.nb + s.nd;
         sa.posi = s.posi;
         sa.soft_ids = s.soft_ids;
         sa.nsoft = s.nsoft;
-        sa.corr_e = s.corr + s.corr_off[0];
-        sa.corr_b = s.corr + s.corr_off[1];
-        sa.corr_t = s.corr + s.corr_off[2];
-        sa.map_e = s.inc + s.inc_off[6];
-        sa.map_b = s.inc + s.inc_off[7];
-        sa.map_t = s.inc + s.inc_off[8];
-        sa.inc_e_start = s.inc + s.inc_off[0];
-        sa.inc_b_start = s.inc + s.inc_off[2];
-        sa.inc_t_start = s.inc + s.inc_off[4];
         sa.active = s.scene_active;
         sa.pid_scene = s.pid_scene;
         sa.all_live = all_active(ctx) ? 1u : 0u;
+        sa.scenes = s.scenes;
+        if (s.soft_tiles) {
+            sa.corr_t = s.corr;
+            sa.tiles = s.soft_tiles;
+            const uint32_t count[3] = {s.ne, s.nb + s.nd, s.nt};
+            size_t off = 0;
+            for (int g = 0; g < 3; ++g) {
+                sa.ntiles[g] = s.soft_ntiles[g];
+                sa.lds[g] = s.soft_lds[g];
+                sa.con[g] = s.soft_ent + s.soft_ent_off[g][0];
+                sa.verts[g] = s.soft_ent + s.soft_ent_off[g][1];
+                sa.slots[g] = s.soft_ent + s.soft_ent_off[g][2];
+                sa.prm[g] = s.soft_prm + off;
+                sa.lam_in[g] = s.lam + off;
+                sa.lam_out[g] = s.lam2 + off;
+                off += count[g];
+            }
+            sa.own = s.soft_own;
+            sa.halo = s.soft_halo;
+            sa.starts = s.soft_starts;
+        } else {
+            sa.edges = s.edges;
+            sa.bends = s.bends;
+            sa.dih = s.dihedrals;
+            sa.tets = s.tets;
+            sa.lam_e = s.lam;
+            sa.lam_b = s.lam + s.ne;
+            sa.lam_t = s.lam + s.ne + s.nb + s.nd;
+            sa.corr_e = s.corr + s.corr_off[0];
+            sa.corr_b = s.corr + s.corr_off[1];
+            sa.corr_t = s.corr + s.corr_off[2];
+            sa.map_e = s.inc + s.inc_off[6];
+            sa.map_b = s.inc + s.inc_off[7];
+            sa.map_t = s.inc + s.inc_off[8];
+            sa.inc_e_start = s.inc + s.inc_off[0];
+            sa.inc_b_start = s.inc + s.inc_off[2];
+            sa.inc_t_start = s.inc + s.inc_off[4];
+        }
     }
     for (uint32_t sub = 0; sub < substeps; ++sub) {
         broadphase(ctx, s, c, key_bits);
@@ -1619,9 +1713,10 @@ void record_step(cn_ctx *ctx, SceneBuffers &s, const cn_step_params *p)
                 ProfScope ps(ctx, "soft");
                 const bool gather = it == 0 || has_contacts, scatter = it + 1 == pid_iters || has_contacts;
                 sa.first = it == 0 ? 1u : 0u;
+                sa.keep_tets = sub + 1 == substeps && it + 1 == soft_iters ? 1u : 0u;
                 if (rigid_pid && it < contact_iters) {
                     launch_soft_iteration(sa, gather, false, it < soft_iters, soft_st);
-                    launch_rigid_pid(s, c, it == 0, soft_st);
+                    launch_rigid_pid(s, c, it == 0, sa.tiles ? sa.solved : 0u, soft_st);
                     if (scatter) launch_soft_iteration(sa, false, true, false, soft_st);
                 } else {
                     launch_soft_iteration(sa, gather, scatter, it < soft_iters, soft_st);
@@ -2336,6 +2431,7 @@ static cn_status set_records(cn_ctx *ctx, std::vector<Dev> &host, Dev *dev, uint
 {
     if (!count) return CN_OK;
     for (uint32_t q = 0; q < count; ++q) host[first + q] = conv(src[q], base);
+    if (!dev) return CN_OK;  // a pool in tiles has the parameters alone on the device
     CN_HIP(ctx, hipMemcpyAsync(dev + first, host.data() + first, count * sizeof(Dev), hipMemcpyHostToDevice,
                                ctx->stream));
     return CN_OK;
@@ -2384,6 +2480,19 @@ cn_status cn_scene_set_constraints(cn_ctx *ctx, uint32_t scene, const cn_constra
     if (st == CN_OK) st = set_records(ctx, ctx->bends_host, s.bends, c0[1], nb, cv->bends, base, bend_dev);
     if (st == CN_OK) st = set_records(ctx, ctx->dih_host, s.dihedrals, c0[2], nd, cv->dihedrals, base, dihedral_dev);
     if (st == CN_OK) st = set_records(ctx, ctx->tets_host, s.tets, c0[3], nt, cv->tets, base, tet_dev);
+    if (s.soft_tiles && st == CN_OK) {
+        const uint32_t first[4] = {c0[0], c0[1], s.nb + c0[2], c0[3]}, count[4] = {ne, nb, nd, nt};
+        const int group[4] = {0, 1, 1, 2};
+        const size_t off[3] = {0, s.ne, (size_t)s.ne + s.nb + s.nd};
+        std::vector<float2> prm;
+        for (int k = 0; k < 4; ++k) {
+            if (!count[k]) continue;
+            soft_params(ctx, group[k], first[k], count[k], prm);
+            CN_HIP(ctx, hipStreamSynchronize(ctx->stream));
+            CN_HIP(ctx, hipMemcpy(s.soft_prm + off[group[k]] + first[k], prm.data(), count[k] * sizeof(float2),
+                                  hipMemcpyHostToDevice));
+        }
+    }
     // the host sources may go as soon as the call returns
     CN_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return st;

@@ -615,6 +615,7 @@ struct RigidPidArgs {
     float4 *rgen;             // slot order
     uint32_t *pick;           // per constrained particle: kPickSkip, kPickNone or its slot
     uint32_t npid;
+    uint32_t solved;          // soft iterations since the gather, in the tiled passes' two position buffers
 };
 
 // What the iterations of a substep do for a constrained particle, fixed for the substep (slot,
@@ -644,13 +645,14 @@ __global__ __launch_bounds__(kBlock) void k_rigid_pid(RigidPidArgs a, SubstepCon
     const uint32_t v = a.pick[j];
     if (v == kPickSkip) return;
     const uint32_t pid = a.soft_ids[j];
-    float4 p = a.posi[pid];
+    const SceneInfo &sc = a.scenes[a.pid_scene[pid]];
+    float4 *posi = a.posi + ((a.solved * __popc(sc.soft_stages)) & 1u ? (size_t)a.npid : 0);
+    float4 p = posi[pid];
     if (p.w <= kEps) return;
     float sx = 0.0f, sy = 0.0f, sz = 0.0f;
     if (v != kPickNone) {
         const uint32_t t = v, rm = a.bnd[t];
         const ParticleClass &pc = a.classes[c.uniform_class ? 0u : a.cls[t]];
-        const SceneInfo &sc = a.scenes[a.pid_scene[pid]];
         a.rgen[t] = p;
         const float4 pv = a.prev[t];
         const float4 pm = a.part_mats[pc.part_mat];
@@ -668,7 +670,7 @@ __global__ __launch_bounds__(kBlock) void k_rigid_pid(RigidPidArgs a, SubstepCon
     p.x = p.x + sx;
     p.y = p.y + sy;
     p.z = p.z + sz;
-    a.posi[pid] = p;
+    posi[pid] = p;
 }
 
 static ContactArgs contact_args(const SceneBuffers &s, const SubstepConsts &c, int din)
@@ -734,7 +736,7 @@ void launch_contact_velocity(const SceneBuffers &s, const SubstepConsts &c, hipS
     hipLaunchKernelGGL(k_contact_velocity_apply, dim3(grid_c(c.n)), dim3(kBlock), 0, st, a);
 }
 
-void launch_rigid_pid(const SceneBuffers &s, const SubstepConsts &c, bool pick, hipStream_t st)
+void launch_rigid_pid(const SceneBuffers &s, const SubstepConsts &c, bool pick, uint32_t solved, hipStream_t st)
 {
     if (!s.nsoft) return;
     RigidPidArgs a;
@@ -755,6 +757,7 @@ void launch_rigid_pid(const SceneBuffers &s, const SubstepConsts &c, bool pick, 
     a.rgen = s.ct_gen;
     a.pick = s.rigid_pick;
     a.npid = s.npid;
+    a.solved = solved;
     if (pick) hipLaunchKernelGGL(k_rigid_pick, dim3(grid_c(s.nsoft)), dim3(kBlock), 0, st, a, c);
     hipLaunchKernelGGL(k_rigid_pid, dim3(grid_c(s.nsoft)), dim3(kBlock), 0, st, a, c);
 }

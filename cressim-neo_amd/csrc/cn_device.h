@@ -68,6 +68,7 @@ struct SceneInfo {
                           // phase group)
     uint32_t rigid;       // 1: particle-rigid contacts can exist (a solid particle and a static
                           // collider slot), solved in the slot-order contact pass
+    uint32_t soft_stages; // bit g: the scene has constraints of group g (edges; bends, dihedrals; tets)
     int32_t win[3];       // lowest cell of the scene's window of 2^morton_bits cells per axis: inside it
                           // no two cells share a Morton code
     uint32_t rigid_pid;   // 1: the same, for a scene without particle-particle pairs whose every

@@ -4,6 +4,10 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <future>
+#include <system_error>
+#include <vector>
+
 #include "cn_device.h"
 
 namespace cn {
@@ -127,6 +131,65 @@ struct CorrRec {
     float x, y, z;
 };
 
+// ---- tiled soft-constraint passes (cn_tiles.hip, cn_soft.hip) ----
+// A tile: up to kSoftTile constrained particles of one scene, close in space.  Per constraint group
+// (edges; bends and dihedrals; tets) a workgroup loads the tile's particles and those its constraints
+// reach (the halo), solves every constraint that touches one of its particles, and sums its own
+// particles' correction records, all in LDS.
+constexpr uint32_t kSoftTile = 256;
+constexpr uint32_t kSoftTileLds = 76u * 1024u;  // two workgroups per CU
+constexpr uint32_t kTileOwner = 0x80000000u;    // constraint word: this tile writes its lambda
+constexpr uint16_t kTileNoRec = 0xffffu;        // record slot of a vertex that is not the tile's own
+struct SoftTile {
+    uint32_t own0, nown;    // its particles: own[own0 ..), ascending
+    uint32_t halo0, nhalo;  // the others it reads: halo[halo0 ..)
+    uint32_t ent0, nent;    // its constraints: con / verts / slots
+    uint32_t start0, nrec;  // its particles' first records: starts[start0 .. start0 + nown]
+    uint32_t scene;
+};
+struct SoftTilesHost {
+    struct Group {
+        std::vector<SoftTile> tiles;
+        std::vector<uint32_t> con, verts, slots;  // per entry: constraint, arity / 2 words of 16-bit pairs
+        std::vector<uint32_t> halo;
+        std::vector<uint16_t> starts;
+        uint32_t lds = 0;                         // bytes of the largest tile
+    };
+    std::vector<uint32_t> own;
+    std::vector<uint32_t> stages;  // per scene: bit g: it has constraints of group g
+    Group group[3];
+};
+// The constraints of the three groups (bends before dihedrals) and their vertices.
+struct SoftTopology {
+    const EdgeDev *edges;
+    const BendDev *bends;
+    const DihedralDev *dihedrals;
+    const TetDev *tets;
+    uint32_t nb;
+    uint32_t count[3];
+    uint32_t vertex(int g, uint32_t c, uint32_t k) const
+    {
+        if (g == 0) return k == 0 ? edges[c].a : edges[c].b;
+        if (g == 2) return tets[c].p[k];
+        if (c < nb) return k == 0 ? bends[c].p0 : (k == 1 ? bends[c].p1 : (k == 2 ? bends[c].p2 : 0xffffffffu));
+        const DihedralDev &d = dihedrals[c - nb];
+        return k == 0 ? d.e0 : (k == 1 ? d.e1 : (k == 2 ? d.o0 : d.o1));
+    }
+};
+
+// f on a thread of its own; when none is to be had, at the time its result is asked for
+template <typename F>
+auto run_aside(F f) -> std::future<decltype(f())>
+{
+    try {
+        return std::async(std::launch::async, f);
+    } catch (const std::system_error &) {
+        return std::async(std::launch::deferred, f);
+    }
+}
+bool build_soft_tiles(uint32_t n, const float *pos, const std::vector<uint32_t> &soft, const uint32_t *pid_scene,
+                      uint32_t nscenes, const SoftTopology &topo, SoftTilesHost &out);
+
 struct SceneBuffers {
     uint32_t n = 0;                 // slots of the per-slot arrays in use
     uint32_t npid = 0;              // particles of the pool (particle-index arrays hold npid entries)
@@ -213,7 +276,7 @@ struct SceneBuffers {
     // soft constraints
     uint32_t *slot_of = nullptr;
     float4 *posi = nullptr;         // positions of the constrained particles in particle-index order
-                                    // during the soft phase of an iteration
+                                    // during the soft phase of an iteration: two buffers of npid
     uint32_t *soft_ids = nullptr;   // the constrained particles, ascending
     uint32_t *rigid_pick = nullptr; // per constrained particle: its particle-rigid work of the substep
     uint32_t nsoft = 0;
@@ -226,6 +289,15 @@ struct SceneBuffers {
     CorrRec *corr = nullptr;        // correction records of edges | bends + dihedrals | tets, each group
                                     // in its incidence (CSR) order, then one spare record
     size_t corr_off[3] = {0, 0, 0};
+    // tiled soft passes (null: some particle has too many constraints for a tile)
+    SoftTile *soft_tiles = nullptr;      // the groups' tiles back to back
+    uint32_t soft_ntiles[3] = {0, 0, 0}, soft_lds[3] = {0, 0, 0};
+    uint32_t *soft_own = nullptr, *soft_halo = nullptr;
+    uint16_t *soft_starts = nullptr;
+    uint32_t *soft_ent = nullptr;        // con, verts, slots of the three groups
+    size_t soft_ent_off[3][3] = {};
+    float2 *soft_prm = nullptr;          // (rest value, compliance) of edges | bends + dihedrals | tets
+    float *lam2 = nullptr;               // the other buffer of lam: a pass reads one and writes the other
     uint32_t *inc = nullptr;        // three CSR incidence structures back to back, then the record maps
     size_t inc_off[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
 };
@@ -260,7 +332,8 @@ void launch_contact_velocity(const SceneBuffers &s, const SubstepConsts &c, hipS
 void launch_rigid_velocity(const SceneBuffers &s, const SubstepConsts &c, uint32_t iters, hipStream_t st);
 // the particle-rigid contacts of scenes solved in particle-index order, on the soft phase's positions;
 // pick: first call of the substep (each particle's slot and candidates are looked up once)
-void launch_rigid_pid(const SceneBuffers &s, const SubstepConsts &c, bool pick, hipStream_t st);
+// solved: soft iterations since the gather (tiled passes; 0 otherwise)
+void launch_rigid_pid(const SceneBuffers &s, const SubstepConsts &c, bool pick, uint32_t solved, hipStream_t st);
 void launch_tick_gather(const SceneBuffers &pool, const SceneBuffers &tick, const uint4 *seg, uint32_t nseg,
                         hipStream_t st);
 void launch_tick_scatter(const SceneBuffers &pool, const SceneBuffers &tick, const uint4 *seg, uint32_t nseg,
@@ -298,6 +371,18 @@ struct SoftArgs {
     const uint32_t *inc_t_start;
     const uint32_t *active;    // per scene
     const uint32_t *pid_scene; // particle index -> scene
+    const SceneInfo *scenes;
+    // tiled passes: a scene's positions alternate between two buffers of n, one step per group it has
+    // constraints of; solved counts the iterations since the gather
+    const SoftTile *tiles;     // null: the passes over the whole pool
+    uint32_t ntiles[3], lds[3];
+    const uint32_t *own, *halo;
+    const uint16_t *starts;
+    const uint32_t *con[3], *verts[3], *slots[3];
+    const float2 *prm[3];
+    float *lam_in[3], *lam_out[3];
+    uint32_t keep_tets;        // the last iteration of a step: every tet's records go to corr_t
+    uint32_t solved;
     uint32_t all_live;         // every scene takes part in the step (no per-particle check)
     uint32_t first;            // first iteration of a substep: every lambda starts at zero (read as
                                // zero, and written by every constraint, also where it does nothing)
@@ -305,7 +390,7 @@ struct SoftArgs {
 // gather / scatter: copy the constrained particles' positions from slot order before the solves and
 // back after them (needed only around iterations where another pass moves those particles)
 // solve = false: only the gather and / or the scatter
-void launch_soft_iteration(const SoftArgs &a, bool gather, bool scatter, bool solve, hipStream_t st);
+void launch_soft_iteration(SoftArgs &a, bool gather, bool scatter, bool solve, hipStream_t st);
 
 // per-pass entries in the reference's data order (cn_passes.hip)
 void launch_ref_keys(const float4 *pos, uint32_t n, float inv_cell, uint32_t *keys, int32_t *cells,
