@@ -1671,23 +1671,14 @@ __global__ __launch_bounds__(kBlock) void k_fluid_lists(FluidArgs a, SubstepCons
 // (APPLY = false: vort[i] = (curl, |curl|), zero for particles that do not confine) and
 // physics_fluid_apply_vorticity_confinement.cs.hlsl:16-94 (APPLY = true).  Both walk the
 // post-update neighbor list (physics_solver.cpp:1262): the first cap in-radius neighbors in walk
-// order on the final positions, of which the same-material ones contribute.  The curl pass walks
-// the run table and, where a list buffer is given (nbr, neighbor-major), stores the list; the
-// confinement pass then reads it instead of walking again.  Inactive scenes are skipped whole
-// (their neighbors are their own).
-template <bool UNIFORM, bool APPLY>
-__global__ __launch_bounds__(kBlock) void k_fluid_vorticity(FluidArgs a, SubstepConsts c, float4 *__restrict__ vel,
-                                                            float4 *__restrict__ vort)
+// order on the final positions, of which the same-material ones contribute.  Inactive scenes are
+// skipped whole (their neighbors are their own).  each(s, t2, self, term) calls term(same material, dx,
+// dy, dz, the neighbor's velocity or (APPLY) curl) for every listed neighbor.
+template <bool APPLY, class Each>
+__device__ __forceinline__ void vorticity_particle(uint32_t i, const ParticleClass &pc, const FluidArgs &a,
+                                                   const SubstepConsts &c, float4 *vel, float4 *vort, Each &&each)
 {
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= c.n) return;
-    const ParticleClass pc = a.classes[UNIFORM ? 0u : a.cls[i]];
-    if (!a.active[pc.scene]) return;
     const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    if (pc.kind != CN_PARTICLE_KIND_FLUID) {
-        if (!APPLY) vort[i] = zero;
-        return;
-    }
     const cn_fluid_material &m = a.fm[pc.fluid_mat];
     const float conf = fmaxd(m.vorticity_confinement, 0.0f);
     const float4 s = a.pos[i];
@@ -1695,58 +1686,33 @@ __global__ __launch_bounds__(kBlock) void k_fluid_vorticity(FluidArgs a, Substep
         if (!APPLY) vort[i] = zero;
         return;
     }
-    float4 self = APPLY ? vort[i] : vel[i];
+    const float4 self = APPLY ? vort[i] : vel[i];
     if (APPLY && self.w <= kEps) return;
     const float h = fmaxd(m.smoothing_radius, 1.0e-4f);
-    const float t2 = a.fc[pc.fluid_mat].t2;
     float ax = 0.0f, ay = 0.0f, az = 0.0f;
     // one listed neighbor's term (same material, inside the kernel's support)
-    auto term = [&](uint32_t q, uint32_t qmat, float dx, float dy, float dz) {
-        if (qmat != pc.fluid_mat) return;
+    each(s, a.fc[pc.fluid_mat].t2, [&](bool same, float dx, float dy, float dz, const float4 &o) {
         const float dist = len3(dx, dy, dz);
-        if (dist <= kEps || dist >= h) return;
+        // every term is evaluated before the test decides whether it is added (no branch per neighbor)
+        const bool add = same && !(dist <= kEps || dist >= h);
         // FluidSpikyKernelGradient, physics_fluid_common.hlsli:45-54
         const float dw = spiky_dw(dist, h);
         const float gx = dw * fdiv(dx, dist), gy = dw * fdiv(dy, dist), gz = dw * fdiv(dz, dist);
+        float tx, ty, tz;
         if (APPLY) {
-            const float mj = vort[q].w;
-            ax = ax + mj * gx;
-            ay = ay + mj * gy;
-            az = az + mj * gz;
+            tx = o.w * gx;
+            ty = o.w * gy;
+            tz = o.w * gz;
         } else {
-            const float4 vj = vel[q];
-            const float wx = vj.x - self.x, wy = vj.y - self.y, wz = vj.z - self.z;
-            ax = ax + (wy * gz - wz * gy);
-            ay = ay + (wz * gx - wx * gz);
-            az = az + (wx * gy - wy * gx);
+            const float wx = o.x - self.x, wy = o.y - self.y, wz = o.z - self.z;
+            tx = wy * gz - wz * gy;
+            ty = wz * gx - wx * gz;
+            tz = wx * gy - wy * gx;
         }
-    };
-    if (c.cap > 0 && (!UNIFORM || neighbor_ok(pc, pc))) {
-        if (APPLY && a.nbr) {
-            // the list the curl pass wrote: the same neighbors in the same order (positions unchanged)
-            const uint32_t cnt = a.nbr_cnt[i];
-            for (uint32_t k = 0; k < cnt; ++k) {
-                const uint32_t q = a.nbr[(size_t)k * c.n + i];
-                const float4 pj = a.pos[q];
-                term(q, UNIFORM ? pc.fluid_mat : a.classes[a.cls[q]].fluid_mat, s.x - pj.x, s.y - pj.y, s.z - pj.z);
-            }
-        } else {
-            uint32_t cnt = 0;
-            walk_runs(a.cellc[i], run_table(a), c, [&](uint32_t q) {
-                if (q == i) return true;
-                const uint32_t qmat = UNIFORM ? pc.fluid_mat : a.classes[a.cls[q]].fluid_mat;
-                if (!UNIFORM && !neighbor_ok(pc, a.classes[a.cls[q]])) return true;
-                const float4 pj = a.pos[q];
-                if (pj.w <= kEps) return true;
-                const float dx = s.x - pj.x, dy = s.y - pj.y, dz = s.z - pj.z;
-                if (!(dot3(dx, dy, dz, dx, dy, dz) < t2)) return true;
-                if (!APPLY && a.nbr) a.nbr[(size_t)cnt * c.n + i] = q;  // for the confinement pass
-                term(q, qmat, dx, dy, dz);
-                return ++cnt < c.cap;
-            });
-            if (!APPLY && a.nbr) a.nbr_cnt[i] = cnt;
-        }
-    }
+        ax = add ? ax + tx : ax;
+        ay = add ? ay + ty : ay;
+        az = add ? az + tz : az;
+    });
     if (!APPLY) {
         vort[i] = make_float4(ax, ay, az, len3(ax, ay, az));
         return;
@@ -1759,6 +1725,56 @@ __global__ __launch_bounds__(kBlock) void k_fluid_vorticity(FluidArgs a, Substep
     const float fz = conf * (nx * self.y - ny * self.x);
     const float4 v = vel[i];
     vel[i] = make_float4(v.x + c.dt * fx, v.y + c.dt * fy, v.z + c.dt * fz, 0.0f);
+}
+
+// The same over the run table.  The curl pass stores the list where a list buffer is given (nbr,
+// neighbor-major); the confinement pass then reads it instead of walking again.
+template <bool UNIFORM, bool APPLY>
+__device__ __forceinline__ void vorticity_global(uint32_t i, const FluidArgs &a, const SubstepConsts &c, float4 *vel,
+                                                 float4 *vort)
+{
+    const ParticleClass pc = a.classes[UNIFORM ? 0u : a.cls[i]];
+    if (!a.active[pc.scene]) return;
+    if (pc.kind != CN_PARTICLE_KIND_FLUID) {
+        if (!APPLY) vort[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        return;
+    }
+    vorticity_particle<APPLY>(i, pc, a, c, vel, vort, [&](const float4 &s, float t2, auto &&term) {
+        if (c.cap == 0 || (UNIFORM && !neighbor_ok(pc, pc))) return;
+        auto other = [&](uint32_t q) { return APPLY ? vort[q] : vel[q]; };
+        auto same = [&](uint32_t q) { return UNIFORM || a.classes[a.cls[q]].fluid_mat == pc.fluid_mat; };
+        if (APPLY && a.nbr) {
+            // the list the curl pass wrote: the same neighbors in the same order (positions unchanged)
+            const uint32_t cnt = a.nbr_cnt[i];
+            for (uint32_t k = 0; k < cnt; ++k) {
+                const uint32_t q = a.nbr[(size_t)k * c.n + i];
+                const float4 pj = a.pos[q];
+                term(same(q), s.x - pj.x, s.y - pj.y, s.z - pj.z, other(q));
+            }
+            return;
+        }
+        uint32_t cnt = 0;
+        walk_runs(a.cellc[i], run_table(a), c, [&](uint32_t q) {
+            if (q == i) return true;
+            if (!UNIFORM && !neighbor_ok(pc, a.classes[a.cls[q]])) return true;
+            const float4 pj = a.pos[q];
+            if (pj.w <= kEps) return true;
+            const float dx = s.x - pj.x, dy = s.y - pj.y, dz = s.z - pj.z;
+            if (!(dot3(dx, dy, dz, dx, dy, dz) < t2)) return true;
+            if (!APPLY && a.nbr) a.nbr[(size_t)cnt * c.n + i] = q;  // for the confinement pass
+            term(same(q), dx, dy, dz, other(q));
+            return ++cnt < c.cap;
+        });
+        if (!APPLY && a.nbr) a.nbr_cnt[i] = cnt;
+    });
+}
+
+template <bool UNIFORM, bool APPLY>
+__global__ __launch_bounds__(kBlock) void k_fluid_vorticity(FluidArgs a, SubstepConsts c, float4 *__restrict__ vel,
+                                                            float4 *__restrict__ vort)
+{
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < c.n) vorticity_global<UNIFORM, APPLY>(i, a, c, vel, vort);
 }
 
 // FluidAnisotropyJacobiRotate, physics_fluid_anisotropy_common.hlsli:28-74 (rsqrt read as
@@ -1811,21 +1827,16 @@ __device__ __forceinline__ void sort_pair(float (&ev)[3], float (&ax)[3][3])
 
 // Render anisotropy: physics_fluid_build_render_anisotropy.cs.hlsl:34-171 with
 // physics_fluid_anisotropy_common.hlsli:9-156 (rcp and rsqrt read as correctly rounded 1/x and
-// 1/sqrt), over the post-update list walked again, twice: the weighted mean of the listed
+// 1/sqrt), over the post-update list taken twice: the weighted mean of the listed
 // neighbors, then their weighted covariance; four largest-pivot Jacobi rotations, axes sorted by
 // decreasing eigenvalue, scales 1.1 sqrt(eigenvalue) clamped to [r, 2r].  A pinned fluid particle
 // has no list (the reference reads a count its build never wrote there) and gets the isotropic
-// frame.  Written in particle-index order: out[k * n + particle] for axis k.
-template <bool UNIFORM>
-__global__ __launch_bounds__(kBlock) void k_fluid_render_aniso(FluidArgs a, SubstepConsts c,
-                                                               const uint32_t *__restrict__ id,
-                                                               float4 *__restrict__ out)
+// frame.  Written in particle-index order: out[k * n + particle] for axis k.  each(first, s, t2, f)
+// calls f(neighbor position) for every listed neighbor.
+template <class Each>
+__device__ __forceinline__ void aniso_particle(uint32_t i, const ParticleClass &pc, size_t pid, bool listed,
+                                               const FluidArgs &a, const SubstepConsts &c, float4 *out, Each &&each)
 {
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= c.n) return;
-    const ParticleClass pc = a.classes[UNIFORM ? 0u : a.cls[i]];
-    if (!a.active[pc.scene]) return;
-    const size_t pid = id[i];
     const size_t n = c.npid;
     const float radius = fmaxd(pc.radius, 1.0e-4f);
     float ax[3][3] = {{1.0f, 0.0f, 0.0f}, {0.0f, 1.0f, 0.0f}, {0.0f, 0.0f, 1.0f}};
@@ -1837,47 +1848,24 @@ __global__ __launch_bounds__(kBlock) void k_fluid_render_aniso(FluidArgs a, Subs
         const float iso = fmaxd(1.0f * radius, radius);
         const float4 s = a.pos[i];
         const float t2 = a.fc[pc.fluid_mat].t2;
-        const bool walk = s.w > kEps && c.cap > 0 && (!UNIFORM || neighbor_ok(pc, pc));
+        const bool walk = s.w > kEps && listed;
         // f(neighbor position, weight) per contributing entry of the list
-        auto weigh = [&](const float4 &pj, float d2, auto &&f) {
-            if (d2 > 0.0f) {
-                const float dist = fsqrt(d2);
-                if (dist < support) {
-                    const float x = dist * inv;
-                    f(pj, 1.0f - x * x * x);
-                }
-            }
-        };
-        // first = true: walk the run table (storing the list where a list buffer is given);
-        // otherwise read that list back: the same neighbors in the same order
-        auto each = [&](bool first, auto &&f) {
-            if (!first && a.nbr) {
-                const uint32_t cnt = a.nbr_cnt[i];
-                for (uint32_t k = 0; k < cnt; ++k) {
-                    const float4 pj = a.pos[a.nbr[(size_t)k * c.n + i]];
-                    const float dx = s.x - pj.x, dy = s.y - pj.y, dz = s.z - pj.z;
-                    weigh(pj, dot3(dx, dy, dz, dx, dy, dz), f);
-                }
-                return;
-            }
-            uint32_t cnt = 0;
-            walk_runs(a.cellc[i], run_table(a), c, [&](uint32_t q) {
-                if (q == i) return true;
-                if (!UNIFORM && !neighbor_ok(pc, a.classes[a.cls[q]])) return true;
-                const float4 pj = a.pos[q];
-                if (pj.w <= kEps) return true;
+        auto weighed = [&](bool first, auto &&f) {
+            each(first, s, t2, [&](const float4 &pj) {
                 const float dx = s.x - pj.x, dy = s.y - pj.y, dz = s.z - pj.z;
                 const float d2 = dot3(dx, dy, dz, dx, dy, dz);
-                if (!(d2 < t2)) return true;
-                if (first && a.nbr) a.nbr[(size_t)cnt * c.n + i] = q;
-                weigh(pj, d2, f);
-                return ++cnt < c.cap;
+                if (d2 > 0.0f) {
+                    const float dist = fsqrt(d2);
+                    if (dist < support) {
+                        const float x = dist * inv;
+                        f(pj, 1.0f - x * x * x);
+                    }
+                }
             });
-            if (first && a.nbr) a.nbr_cnt[i] = cnt;
         };
         float mx = 0.0f, my = 0.0f, mz = 0.0f, wsum = 0.0f;
         if (walk)
-            each(true, [&](const float4 &pj, float w) {
+            weighed(true, [&](const float4 &pj, float w) {
                 wsum = wsum + w;
                 mx = mx + pj.x * w;
                 my = my + pj.y * w;
@@ -1888,7 +1876,7 @@ __global__ __launch_bounds__(kBlock) void k_fluid_render_aniso(FluidArgs a, Subs
             my = fdiv(my, wsum);
             mz = fdiv(mz, wsum);
             float C[3][3] = {{0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}};
-            each(false, [&](const float4 &pj, float w) {
+            weighed(false, [&](const float4 &pj, float w) {
                 const float cc[3] = {pj.x - mx, pj.y - my, pj.z - mz};
 #pragma unroll
                 for (int r = 0; r < 3; ++r)
@@ -1948,6 +1936,183 @@ __global__ __launch_bounds__(kBlock) void k_fluid_render_aniso(FluidArgs a, Subs
     }
 #pragma unroll
     for (int k = 0; k < 3; ++k) out[k * n + pid] = make_float4(ax[k][0], ax[k][1], ax[k][2], sc[k]);
+}
+
+// The same over the run table: the list stored where a list buffer is given, walked again otherwise.
+template <bool UNIFORM>
+__device__ __forceinline__ void aniso_global(uint32_t i, const FluidArgs &a, const SubstepConsts &c,
+                                             const uint32_t *id, float4 *out)
+{
+    const ParticleClass pc = a.classes[UNIFORM ? 0u : a.cls[i]];
+    if (!a.active[pc.scene]) return;
+    const bool listed = c.cap > 0 && (!UNIFORM || neighbor_ok(pc, pc));
+    aniso_particle(i, pc, id[i], listed, a, c, out, [&](bool first, const float4 &s, float t2, auto &&f) {
+        if (!first && a.nbr) {
+            const uint32_t cnt = a.nbr_cnt[i];
+            for (uint32_t k = 0; k < cnt; ++k) f(a.pos[a.nbr[(size_t)k * c.n + i]]);
+            return;
+        }
+        uint32_t cnt = 0;
+        walk_runs(a.cellc[i], run_table(a), c, [&](uint32_t q) {
+            if (q == i) return true;
+            if (!UNIFORM && !neighbor_ok(pc, a.classes[a.cls[q]])) return true;
+            const float4 pj = a.pos[q];
+            if (pj.w <= kEps) return true;
+            const float dx = s.x - pj.x, dy = s.y - pj.y, dz = s.z - pj.z;
+            if (!(dot3(dx, dy, dz, dx, dy, dz) < t2)) return true;
+            if (first && a.nbr) a.nbr[(size_t)cnt * c.n + i] = q;
+            f(pj);
+            return ++cnt < c.cap;
+        });
+        if (first && a.nbr) a.nbr_cnt[i] = cnt;
+    });
+}
+
+// FLUID = false: the particles the tiled launch leaves out.
+template <bool UNIFORM, bool FLUID>
+__global__ __launch_bounds__(kBlock) void k_fluid_render_aniso(FluidArgs a, SubstepConsts c,
+                                                               const uint32_t *__restrict__ id,
+                                                               float4 *__restrict__ out)
+{
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= c.n) return;
+    if (!FLUID && a.classes[a.cls[i]].kind == CN_PARTICLE_KIND_FLUID) return;
+    aniso_global<UNIFORM>(i, a, c, id, out);
+}
+
+// The vorticity and anisotropy passes over the staged halos of the cell blocks, whose cells are the
+// substep's: final positions in LDS (with the velocities for the curl, |curl| in w for the
+// confinement), the neighbors found there and kept as a list of staged entries, which the confinement
+// pass reads again in the same staging.  Walked particle by particle through the run table, every
+// candidate cost a dependent load and a branch: 270 us for the curl of 200,000 particles and 207 us for
+// the anisotropy, against 79 and 89 us; the confinement (41 us, 38 from a list of slots) only follows
+// the curl's list.  What bounds them now: the walk's distance tests (all 27 cells: nothing bounds how
+// far the update moved a particle from its cell), and in the confinement the latency of a block's
+// staging, some two blocks to each workgroup the chip holds.
+// Blocks with a halo larger than the tile, or without a descriptor, walk the run table.
+constexpr int kPostCurl = 0, kPostConfine = 1, kPostAniso = 2;
+template <bool UNIFORM, int PASS>
+__global__ __launch_bounds__(kTileBlock) __attribute__((amdgpu_waves_per_eu(kDeltaWaves))) void k_fluid_post_tiled(
+    FluidArgs a, SubstepConsts c, float4 *__restrict__ vel, float4 *__restrict__ vort, const uint32_t *__restrict__ id,
+    float4 *__restrict__ out)
+{
+    extern __shared__ float4 dyn[];
+    __shared__ uint32_t hoff[kHalo + 1];
+    __shared__ uint32_t hstart[kHalo];
+    constexpr bool CURL = PASS == kPostCurl, CONFINE = PASS == kPostConfine;
+    const uint32_t room = a.tile + kTilePad, tid = threadIdx.x, nblk = a.nblk[1];
+    float4 *lpos = dyn;
+    float4 *lvel = lpos + room;
+    uint32_t *lcls = reinterpret_cast<uint32_t *>(lvel + (CURL ? room : 0u));
+    // each die takes a run of consecutive blocks, whose halos overlap
+    const uint32_t die = blockIdx.x % kXcds, wgs = (gridDim.x + kXcds - 1u - die) / kXcds;
+    const uint32_t per = (nblk + kXcds - 1u) / kXcds, end = min(nblk, per * (die + 1u));
+    TileState ts;
+    for (uint32_t blk = per * die + blockIdx.x / kXcds; blk < end; blk += wgs) {
+        tile_load(ts, blk, hoff, hstart, 0u, a, c);
+        __syncthreads();
+        if (ts.skip) {
+            __syncthreads();
+            continue;
+        }
+        if (!ts.lds) {
+            for (uint32_t i = ts.p0 + tid; i < ts.p1; i += kTileBlock) {
+                if constexpr (PASS == kPostAniso) {
+                    if (a.classes[UNIFORM ? 0u : a.cls[i]].kind == CN_PARTICLE_KIND_FLUID)
+                        aniso_global<UNIFORM>(i, a, c, id, out);
+                } else {
+                    vorticity_global<UNIFORM, CONFINE>(i, a, c, vel, vort);
+                }
+            }
+            __syncthreads();
+            continue;
+        }
+        const uint32_t total = hoff[kHalo], fill = total * kEntryScale, ref = UNIFORM ? 0u : a.cls[ts.p0];
+        bool mixed = false;
+        float4 lv[kStageCells], le[kStageCells];
+        float lw[kStageCells];
+        uint32_t lq[kStageCells];
+        stage_halo(
+            hoff, hstart,
+            [&](uint32_t u, uint32_t q) {
+                lv[u] = a.pos[q];
+                if (CURL) le[u] = vel[q];
+                if (CONFINE) lw[u] = vort[q].w;
+                if (!UNIFORM) lq[u] = a.cls[q];
+            },
+            [&](uint32_t u, uint32_t f, uint32_t) {
+                // component by component: the arrays stay in registers
+                if (CONFINE) {
+                    lpos[f] = make_float4(lv[u].x, lv[u].y, lv[u].z, lw[u]);
+                } else {
+                    const bool far = lv[u].w <= kEps;
+                    lpos[f] = make_float4(far ? kFarAway : lv[u].x, far ? kFarAway : lv[u].y, far ? kFarAway : lv[u].z, 0.0f);
+                }
+                if (CURL) lvel[f] = make_float4(le[u].x, le[u].y, le[u].z, 0.0f);
+                if (!UNIFORM) {
+                    lcls[f] = lq[u];
+                    mixed |= lq[u] != ref;
+                }
+            });
+        if (tid == 0) {  // what the filling entry names
+            lpos[total] = make_float4(kFarAway, kFarAway, kFarAway, 0.0f);
+            if (CURL) lvel[total] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (!UNIFORM) lcls[total] = ref;
+        }
+        const int any_mixed = __syncthreads_or(mixed ? 1 : 0);  // also the barrier after staging
+        const bool bu = UNIFORM || !any_mixed;
+        for (uint32_t i = ts.p0 + tid; i < ts.p1; i += kTileBlock) {
+            const ParticleClass pc = a.classes[UNIFORM ? 0u : a.cls[i]];
+            if (pc.kind != CN_PARTICLE_KIND_FLUID) continue;
+            const bool listed = c.cap > 0 && (!bu || neighbor_ok(pc, pc));
+            uint2 *li = list_words(a.list, i, list_rows(c.cap));
+            auto find = [&](const float4 &s, float t2) -> uint32_t {
+                const int4 ci = a.cellc[i];
+                const int hc = halo_cell(ts, ci);
+                const uint32_t fs = hoff[hc] + (i - hstart[hc]);
+                DensitySelf x;
+                x.s = s;
+                x.pc = pc;
+                RowCull rc = row_cull(s, ci, 0.0f, 0.0f, 3.4e38f);  // every cell
+                ListOut lo(li, c.cap);
+                if (bu) scan_rows<true>(hoff, hc, fs, lpos, lcls, x, t2, lo, a, rc);
+                else scan_rows<false>(hoff, hc, fs, lpos, lcls, x, t2, lo, a, rc);
+                return lo.finish(fill);
+            };
+            uint32_t words = 0;
+            auto entries = [&](auto &&f) {
+                if (!words) return;
+                each_word(li, words, [&](uint2 w) {
+                    uint32_t e[4];
+                    word_entries(w, e);
+#pragma unroll
+                    for (uint32_t u = 0; u < 4; ++u) f(e[u]);
+                });
+            };
+            if constexpr (PASS == kPostAniso) {
+                aniso_particle(i, pc, id[i], listed, a, c, out, [&](bool first, const float4 &s, float t2, auto &&f) {
+                    if (first) words = find(s, t2);
+                    entries([&](uint32_t e) { f(at16(lpos, e)); });
+                });
+            } else {
+                vorticity_particle<CONFINE>(i, pc, a, c, vel, vort, [&](const float4 &s, float t2, auto &&term) {
+                    if (!listed) return;
+                    if (CONFINE) {
+                        words = a.lcnt[i];
+                    } else {
+                        words = find(s, t2);
+                        a.lcnt[i] = words;
+                    }
+                    entries([&](uint32_t e) {
+                        const float4 pj = at16(lpos, e);
+                        term(bu || a.classes[at4(lcls, e)].fluid_mat == pc.fluid_mat, s.x - pj.x, s.y - pj.y, s.z - pj.z,
+                             CONFINE ? pj : at16(lvel, e));
+                    });
+                });
+            }
+        }
+        __syncthreads();
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -2114,12 +2279,34 @@ void launch_fluid_delta(const SceneBuffers &s, const SubstepConsts &c, uint32_t 
     }
 }
 
+// Halo capacity of the vorticity and anisotropy passes: two workgroups a CU, records of positions and
+// velocities (the curl's; the confinement pass has to stage the blocks that the curl pass listed).
+static uint32_t post_tile(const SubstepConsts &c)
+{
+    const uint32_t cls = c.uniform_class ? 0u : 4u;
+    return std::min<uint32_t>(std::min<uint32_t>(c.tile_max, kTileMost), lds_budget(c, 2) / (32u + cls) - kTilePad);
+}
+
 void launch_fluid_vorticity(const SceneBuffers &s, const SubstepConsts &c, hipStream_t st)
 {
-    const FluidArgs a = fluid_args(s, c, 0, 0);
+    FluidArgs a = fluid_args(s, c, 0, 0);
     float4 *vel = s.vel[s.cur];
     float4 *vort = s.cs;  // free between the last delta pass of a substep and the next density pass
-    if (c.uniform_class) {
+    if (tiled(c, 0)) {
+        const uint32_t cls = c.uniform_class ? 0u : 4u;
+        a.tile = post_tile(c);
+        const size_t lds = (size_t)(a.tile + kTilePad) * (16u + cls), more = (size_t)(a.tile + kTilePad) * 16u;
+        const dim3 grid(persistent_grid(c)), block(kTileBlock);
+        const uint32_t *id = nullptr;
+        float4 *out = nullptr;
+        if (c.uniform_class) {
+            hipLaunchKernelGGL((k_fluid_post_tiled<true, kPostCurl>), grid, block, lds + more, st, a, c, vel, vort, id, out);
+            hipLaunchKernelGGL((k_fluid_post_tiled<true, kPostConfine>), grid, block, lds, st, a, c, vel, vort, id, out);
+        } else {
+            hipLaunchKernelGGL((k_fluid_post_tiled<false, kPostCurl>), grid, block, lds + more, st, a, c, vel, vort, id, out);
+            hipLaunchKernelGGL((k_fluid_post_tiled<false, kPostConfine>), grid, block, lds, st, a, c, vel, vort, id, out);
+        }
+    } else if (c.uniform_class) {
         hipLaunchKernelGGL((k_fluid_vorticity<true, false>), dim3(grid_of(c.n)), dim3(kBlock), 0, st, a, c, vel, vort);
         hipLaunchKernelGGL((k_fluid_vorticity<true, true>), dim3(grid_of(c.n)), dim3(kBlock), 0, st, a, c, vel, vort);
     } else {
@@ -2130,11 +2317,25 @@ void launch_fluid_vorticity(const SceneBuffers &s, const SubstepConsts &c, hipSt
 
 void launch_fluid_render_aniso(const SceneBuffers &s, const SubstepConsts &c, float4 *out, hipStream_t st)
 {
-    const FluidArgs a = fluid_args(s, c, 0, 0);
-    if (c.uniform_class)
-        hipLaunchKernelGGL(k_fluid_render_aniso<true>, dim3(grid_of(c.n)), dim3(kBlock), 0, st, a, c, s.id[s.cur], out);
-    else
-        hipLaunchKernelGGL(k_fluid_render_aniso<false>, dim3(grid_of(c.n)), dim3(kBlock), 0, st, a, c, s.id[s.cur], out);
+    FluidArgs a = fluid_args(s, c, 0, 0);
+    const uint32_t *id = s.id[s.cur];
+    const dim3 each(grid_of(c.n));
+    if (tiled(c, 0)) {
+        a.tile = post_tile(c);
+        const size_t lds = (size_t)(a.tile + kTilePad) * (16u + (c.uniform_class ? 0u : 4u));
+        const dim3 grid(persistent_grid(c)), block(kTileBlock);
+        float4 *none = nullptr;
+        if (c.uniform_class) {
+            hipLaunchKernelGGL((k_fluid_post_tiled<true, kPostAniso>), grid, block, lds, st, a, c, none, none, id, out);
+        } else {
+            hipLaunchKernelGGL((k_fluid_post_tiled<false, kPostAniso>), grid, block, lds, st, a, c, none, none, id, out);
+            hipLaunchKernelGGL((k_fluid_render_aniso<false, false>), each, dim3(kBlock), 0, st, a, c, id, out);
+        }
+    } else if (c.uniform_class) {
+        hipLaunchKernelGGL((k_fluid_render_aniso<true, true>), each, dim3(kBlock), 0, st, a, c, id, out);
+    } else {
+        hipLaunchKernelGGL((k_fluid_render_aniso<false, true>), each, dim3(kBlock), 0, st, a, c, id, out);
+    }
 }
 
 void launch_fluid_lists(const SceneBuffers &s, const SubstepConsts &c, hipStream_t st)
