@@ -163,33 +163,27 @@ __device__ __forceinline__ float fdiv_rcp_neg(float a, float b, float y)
 }
 __device__ __forceinline__ float fdiv_rcp(float a, float b, float y) { return -fdiv_rcp_neg(a, b, y); }
 
-// 1 / b, correctly rounded, for a normal b > 0: the hardware estimate (within one ulp) refined by
-// two Newton steps in fma, which reach the correctly rounded reciprocal from any estimate within
-// two ulps except for the significand 1.11...1 (checked exhaustively over significands); that one
-// takes the IEEE division.
-__device__ __forceinline__ float frcp_newton(float b)
+// One Newton step in fma from an estimate y of 1 / b.  From this chip's reciprocal estimate, and from
+// its reciprocal square-root estimate of x where b is the root of x (fsqrt_rsq), it reaches the
+// correctly rounded reciprocal of every significand except 1.11...1 (checked on the device over all
+// of them, at exponents of either parity); that one takes the IEEE division.
+__device__ __forceinline__ float frcp_step(float b, float y) { return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y); }
+__device__ __forceinline__ float frcp_last_significand(float b, float y)
 {
-    float y = __builtin_amdgcn_rcpf(b);
-    y = __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
-    return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
-}
-__device__ __forceinline__ float frcp_exact(float b)
-{
-    float y = frcp_newton(b);
     if ((__float_as_uint(b) & 0x7fffffu) == 0x7fffffu) {
         __asm__ volatile("");  // a side effect keeps this rare path a branch rather than a select
         y = fdiv(1.0f, b);
     }
     return y;
 }
+// 1 / b, correctly rounded, for a normal b > 0 with a normal reciprocal; y0: the estimate it starts from.
+__device__ __forceinline__ float frcp_exact(float b, float y0) { return frcp_last_significand(b, frcp_step(b, y0)); }
 
 // 1 / b for b >= 1, +inf or NaN: frcp_exact while 1 / b stays normal (b < 2^126), else the IEEE
 // division.
 __device__ __forceinline__ float frcp_exact_ge1(float b)
 {
-    float y = __builtin_amdgcn_rcpf(b);
-    y = __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
-    y = __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
+    float y = frcp_step(b, __builtin_amdgcn_rcpf(b));
     if ((__float_as_uint(b) & 0x7fffffu) == 0x7fffffu || !(b < 0x1p126f)) {
         __asm__ volatile("");
         y = fdiv(1.0f, b);
@@ -197,20 +191,22 @@ __device__ __forceinline__ float frcp_exact_ge1(float b)
     return y;
 }
 
-// Square root by the hardware estimate (within one ulp) and the rounding test on its two
-// neighbours: s - ulp is the root when x - (s - ulp) * s <= 0, s + ulp when x - (s + ulp) * s > 0.
-// Equal to fsqrt for x == 0 and for 2^-96 <= x < inf, where fsqrt applies no scaling; for
-// 0 < x < 2^-96 the result is within a few ulps of the root and below 2^-47, which the fluid
-// terms consume only through dist <= eps tests and through d / h < 2^-25 (1 - d / h rounds to 1).
-__device__ __forceinline__ float fsqrt_nearzero_free(float x)
+// Square root of a finite x >= 2^-96 by the reciprocal square-root estimate y (within one ulp, handed
+// out for the reciprocal of the root) and one correction s + (x - s s) y / 2: equal to fsqrt for
+// every significand (checked on the device as above).  A test of the hardware root's two neighbours and
+// a reciprocal of its own from another estimate took eight operations more a neighbor: the delta pass
+// over 4.19M particles 475 us against 455.  0 gives NaN, and so does +inf.
+__device__ __forceinline__ float fsqrt_rsq(float x, float &y)
 {
-    const float s = __builtin_amdgcn_sqrtf(x);
-    const float sm = __uint_as_float(__float_as_uint(s) - 1u);
-    const float sp = __uint_as_float(__float_as_uint(s) + 1u);
-    const float rm = __builtin_fmaf(-sm, s, x);
-    const float rp = __builtin_fmaf(-sp, s, x);
-    const float t = rm <= 0.0f ? sm : s;
-    return rp > 0.0f ? sp : t;
+    y = __builtin_amdgcn_rsqf(x);
+    const float s = x * y;
+    return __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * y, s);
+}
+// The same for any x >= 0 short of +inf: below 2^-96 the result is 2^-48, which the fluid terms consume
+// only through dist <= eps tests and through d / h < 2^-25 (1 - d / h rounds to 1).
+__device__ __forceinline__ float fsqrt_nearzero_free(float x, float &y)
+{
+    return fsqrt_rsq(__builtin_fmaxf(x, 0x1p-96f), y);
 }
 __device__ __forceinline__ float fmaxd(float a, float b) { return a > b ? a : b; }
 __device__ __forceinline__ float fmind(float a, float b) { return a < b ? a : b; }

@@ -277,11 +277,12 @@ __device__ __forceinline__ void pair_quot_y(PairQuot &p, float dx, float dy, flo
     p.der = LIVE ? der : ((dist <= kEps || dist >= h) ? 0.0f : der);
 }
 
+// y0: the estimate of 1 / dist that its square root gave (fsqrt_rsq)
 template <bool FAST, bool LIVE = false>
 __device__ __forceinline__ void pair_quot(PairQuot &p, float dx, float dy, float dz, float dist, float h, float ih,
-                                          float k)
+                                          float k, float y0)
 {
-    pair_quot_y<FAST, LIVE>(p, dx, dy, dz, dist, h, ih, __fmul_rn(2.0f, k), FAST ? frcp_exact(dist) : 0.0f);
+    pair_quot_y<FAST, LIVE>(p, dx, dy, dz, dist, h, ih, __fmul_rn(2.0f, k), FAST ? frcp_exact(dist, y0) : 0.0f);
 }
 
 struct DensitySelf {
@@ -340,7 +341,8 @@ __device__ __forceinline__ DensityTerm density_term(const DensitySelf &x, const 
     DensityTerm t;
     const float dx = x.s.x - pj.x, dy = x.s.y - pj.y, dz = x.s.z - pj.z;
     t.d2 = dot3(dx, dy, dz, dx, dy, dz);
-    const float dist = fsqrt_nearzero_free(t.d2);
+    float y0;
+    const float dist = fsqrt_nearzero_free(t.d2, y0);
     const float omq = FAST ? __fadd_rn(1.0f, fdiv_rcp_neg(dist, x.h, x.ih)) : __fsub_rn(1.0f, fdiv(dist, x.h));
     // every term the callers add is a neighbor's (dist < h): the kernel's range test is left out
     t.w = spiky_w_om_in(omq, x.kw);
@@ -348,7 +350,7 @@ __device__ __forceinline__ DensityTerm density_term(const DensitySelf &x, const 
     if (TENSION && x.tension && !(dist <= kEps || dist >= x.h)) {
         // FluidSpikyKernelGradient, physics_fluid_common.hlsli:44-53, negated: der * -(d / dist)
         PairQuot p;
-        pair_quot<FAST>(p, dx, dy, dz, dist, x.h, x.ih, x.kw);
+        pair_quot<FAST>(p, dx, dy, dz, dist, x.h, x.ih, x.kw, y0);
         t.ngx = p.der * p.nnx;
         t.ngy = p.der * p.nny;
         t.ngz = p.der * p.nnz;
@@ -497,12 +499,13 @@ __device__ __forceinline__ DeltaTerm delta_term(const DeltaSelf &x, const float4
     DeltaTerm t;
     const float ddx = x.sx - cq.x, ddy = x.sy - cq.y, ddz = x.sz - cq.z;
     const float d2 = dot3(ddx, ddy, ddz, ddx, ddy, ddz);
-    const float dist = fsqrt_nearzero_free(d2);
-    t.live = d2 < x.t2 && !(dist <= kEps);
+    float y0;
+    const float dist = fsqrt_rsq(d2, y0);
+    t.live = d2 < x.t2 && dist > kEps;
     PairQuot p;
     // a listed neighbor (dist < h) whose term counts only when live (dist > eps)
-    pair_quot<true, true>(p, ddx, ddy, ddz, dist, x.h, x.ih, x.kw);
-    if (!x.fd) pair_quot<false, true>(p, ddx, ddy, ddz, dist, x.h, x.ih, x.kw);
+    pair_quot<true, true>(p, ddx, ddy, ddz, dist, x.h, x.ih, x.kw, y0);
+    if (!x.fd) pair_quot<false, true>(p, ddx, ddy, ddz, dist, x.h, x.ih, x.kw, y0);
     // sc * n with sc = -0.5 (Ci + Cj) der, as (0.5 (Ci + Cj) der) * -n
     const float msc = 0.5f * (x.Ci + cq.w) * p.der;
     float pdx = msc * p.nnx, pdy = msc * p.nny, pdz = msc * p.nnz;
@@ -1193,24 +1196,25 @@ __device__ __forceinline__ void delta_plain(const uint2 *p, uint32_t words, cons
                 q[u].y = x.sy - q[u].y;
                 q[u].z = x.sz - q[u].z;
                 d2[u] = dot3(q[u].x, q[u].y, q[u].z, q[u].x, q[u].y, q[u].z);
-                dist[u] = fsqrt_nearzero_free(d2[u]);
+                float y0;
+                dist[u] = fsqrt_rsq(d2[u], y0);
                 if (FAST) {
-                    y[u] = frcp_newton(dist[u]);
+                    y[u] = frcp_step(dist[u], y0);
                     sig = max(sig, __float_as_uint(dist[u]) & 0x7fffffu);
                 }
             }
-            // one test for the two: the significand that the Newton steps do not reach (frcp_exact)
+            // one test for the two: the significand that the Newton step does not reach
             if (FAST && sig == 0x7fffffu) {
                 __asm__ volatile("");
 #pragma unroll
-                for (uint32_t u = 0; u < 2; ++u) y[u] = frcp_exact(dist[u]);
+                for (uint32_t u = 0; u < 2; ++u) y[u] = frcp_last_significand(dist[u], y[u]);
             }
 #pragma unroll
             for (uint32_t u = 0; u < 2; ++u) {
                 PairQuot pq;
                 pair_quot_y<FAST, true>(pq, q[u].x, q[u].y, q[u].z, dist[u], x.h, x.ih, k2, y[u]);
                 const float msc = 0.5f * (x.Ci + q[u].w) * pq.der;
-                if (d2[u] < x.t2 && !(dist[u] <= kEps)) {
+                if (d2[u] < x.t2 && dist[u] > kEps) {
                     d.x = d.x + msc * pq.nnx;
                     d.y = d.y + msc * pq.nny;
                     d.z = d.z + msc * pq.nnz;
