@@ -1496,7 +1496,7 @@ cn_status upload_pool(cn_ctx *ctx, uint32_t count, const cn_scene_desc *descs)
         CN_HIP(ctx, dalloc(&s.lam, nlam));
         s.nsoft = (uint32_t)soft.size();
         CN_HIP(ctx, dalloc(&s.soft_ids, soft.size()));
-        CN_HIP(ctx, dalloc(&s.rigid_pick, soft.size()));
+        CN_HIP(ctx, dalloc(&s.rigid_pick, n));
         if (!soft.empty())
             CN_HIP(ctx, hipMemcpy(s.soft_ids, soft.data(), soft.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
         if (build_soft_tiles(n, pos.data(), soft, scene_of.data(), ctx->nscenes, topo, tiles)) {
@@ -1714,13 +1714,8 @@ void record_step(cn_ctx *ctx, SceneBuffers &s, const cn_step_params *p)
                 const bool gather = it == 0 || has_contacts, scatter = it + 1 == pid_iters || has_contacts;
                 sa.first = it == 0 ? 1u : 0u;
                 sa.keep_tets = sub + 1 == substeps && it + 1 == soft_iters ? 1u : 0u;
-                if (rigid_pid && it < contact_iters) {
-                    launch_soft_iteration(sa, gather, false, it < soft_iters, soft_st);
-                    launch_rigid_pid(s, c, it == 0, sa.tiles ? sa.solved : 0u, soft_st);
-                    if (scatter) launch_soft_iteration(sa, false, true, false, soft_st);
-                } else {
-                    launch_soft_iteration(sa, gather, scatter, it < soft_iters, soft_st);
-                }
+                if (rigid_pid && it == 0) launch_rigid_pick(s, c, soft_st);
+                launch_soft_iteration(sa, s, c, rigid_pid && it < contact_iters, gather, scatter, it < soft_iters, soft_st);
             }
             if (has_contacts && it < contact_iters) {
                 ProfScope ps(ctx, "contacts");

@@ -330,10 +330,13 @@ void launch_contact_partners(const SceneBuffers &s, const SubstepConsts &c, hipS
 void launch_contact_iteration(const SceneBuffers &s, const SubstepConsts &c, int din, hipStream_t st);
 void launch_contact_velocity(const SceneBuffers &s, const SubstepConsts &c, hipStream_t st);
 void launch_rigid_velocity(const SceneBuffers &s, const SubstepConsts &c, uint32_t iters, hipStream_t st);
-// the particle-rigid contacts of scenes solved in particle-index order, on the soft phase's positions;
-// pick: first call of the substep (each particle's slot and candidates are looked up once)
-// solved: soft iterations since the gather (tiled passes; 0 otherwise)
-void launch_rigid_pid(const SceneBuffers &s, const SubstepConsts &c, bool pick, uint32_t solved, hipStream_t st);
+// the particle-rigid contacts of scenes solved in particle-index order, on the soft phase's positions:
+// the substep's choice of work per particle, then (where the last tiled pass does not do it) an
+// iteration; solved: soft iterations since the gather (tiled passes; 0 otherwise)
+struct RigidPidArgs;
+RigidPidArgs rigid_pid_args(const SceneBuffers &s, uint32_t solved);
+void launch_rigid_pick(const SceneBuffers &s, const SubstepConsts &c, hipStream_t st);
+void launch_rigid_pid(const SceneBuffers &s, const SubstepConsts &c, uint32_t solved, hipStream_t st);
 void launch_tick_gather(const SceneBuffers &pool, const SceneBuffers &tick, const uint4 *seg, uint32_t nseg,
                         hipStream_t st);
 void launch_tick_scatter(const SceneBuffers &pool, const SceneBuffers &tick, const uint4 *seg, uint32_t nseg,
@@ -390,7 +393,7 @@ struct SoftArgs {
 // gather / scatter: copy the constrained particles' positions from slot order before the solves and
 // back after them (needed only around iterations where another pass moves those particles)
 // solve = false: only the gather and / or the scatter
-void launch_soft_iteration(SoftArgs &a, bool gather, bool scatter, bool solve, hipStream_t st);
+void launch_soft_iteration(SoftArgs &a, const SceneBuffers &s, const SubstepConsts &c, bool rigid, bool gather, bool scatter, bool solve, hipStream_t st);
 
 // per-pass entries in the reference's data order (cn_passes.hip)
 void launch_ref_keys(const float4 *pos, uint32_t n, float inv_cell, uint32_t *keys, int32_t *cells,

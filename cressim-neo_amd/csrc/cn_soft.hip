@@ -14,7 +14,7 @@
 
 #include <utility>
 
-#include "cn_internal.h"
+#include "cn_rigid.h"
 
 namespace cn {
 
@@ -223,8 +223,11 @@ __device__ __forceinline__ bool solve_tet(const float4 p0, const float4 p1, cons
 // What bounds it: the latency of a tile's three phases (load, solve, sum), 250 tiles to 64,000
 // particles being one a CU.
 constexpr int kTileThreads = 512;
-template <int G>
-__global__ __launch_bounds__(kTileThreads) void k_soft_tile(SoftArgs a)
+// RIGID: a scene's last group also solves the iteration's particle-rigid contacts of its particles (a
+// launch of their own took 5 us an iteration: a 256 x 256 cloth's step 829 us against 766, a 32^3 tet
+// block's 863 against 780).
+template <int G, bool RIGID>
+__global__ __launch_bounds__(kTileThreads) void k_soft_tile(SoftArgs a, RigidPidArgs ra, SubstepConsts c)
 {
     extern __shared__ float4 lp[];
     constexpr uint32_t A = G == 0 ? 2u : 4u;  // vertices per constraint
@@ -240,7 +243,7 @@ __global__ __launch_bounds__(kTileThreads) void k_soft_tile(SoftArgs a)
         lp[k] = pin[k < T.nown ? a.own[T.own0 + k] : a.halo[T.halo0 + (k - T.nown)]];
     __syncthreads();
     for (uint32_t k = tid; k < T.nent; k += kTileThreads) {
-        const uint32_t e = T.ent0 + k, cw = a.con[G][e], c = cw & ~kTileOwner;
+        const uint32_t e = T.ent0 + k, cw = a.con[G][e], con = cw & ~kTileOwner;
         uint32_t v[A], s[A];
 #pragma unroll
         for (uint32_t u = 0; u < A; u += 2) {
@@ -250,8 +253,8 @@ __global__ __launch_bounds__(kTileThreads) void k_soft_tile(SoftArgs a)
             s[u] = sw & 0xffffu;
             s[u + 1] = sw >> 16;
         }
-        const float2 prm = a.prm[G][c];
-        const float lambda = a.first ? 0.0f : a.lam_in[G][c];
+        const float2 prm = a.prm[G][con];
+        const float lambda = a.first ? 0.0f : a.lam_in[G][con];
         float lam = lambda;
         CorrRec r[A];
 #pragma unroll
@@ -259,14 +262,14 @@ __global__ __launch_bounds__(kTileThreads) void k_soft_tile(SoftArgs a)
         if constexpr (G == 0) {
             solve_edge(lp[v[0]], lp[v[1]], prm.x, prm.y, a, lambda, lam, r);
         } else if constexpr (G == 1) {
-            if (c < a.nb) solve_bend(lp[v[0]], lp[v[1]], lp[v[2]], prm.x, prm.y, a, lambda, lam, r);
+            if (con < a.nb) solve_bend(lp[v[0]], lp[v[1]], lp[v[2]], prm.x, prm.y, a, lambda, lam, r);
             else solve_dihedral(lp[v[0]], lp[v[1]], lp[v[2]], lp[v[3]], prm.x, prm.y, a, lambda, lam, r);
         } else {
             // A degenerate tet keeps its records, which therefore have a place in memory too.  Where the
             // compliance term alone exceeds the threshold and no inverse mass is negative none can
             // become degenerate within the step: they are written by its last iteration only (every
             // iteration: a pool of fluid, tet and cloth scenes 5,314 us a step against 4,912).
-            CorrRec *kept = a.corr_t + 4 * (size_t)c;
+            CorrRec *kept = a.corr_t + 4 * (size_t)con;
             const float4 p0 = lp[v[0]], p1 = lp[v[1]], p2 = lp[v[2]], p3 = lp[v[3]];
             const bool sure = fdiv(prm.y, fmaxd(a.dt * a.dt, kEps)) > kEps && p0.w >= 0.0f && p1.w >= 0.0f &&
                               p2.w >= 0.0f && p3.w >= 0.0f;
@@ -279,14 +282,17 @@ __global__ __launch_bounds__(kTileThreads) void k_soft_tile(SoftArgs a)
                 for (uint32_t u = 0; u < A; ++u) kept[u] = r[u];
             }
         }
-        if (cw & kTileOwner) a.lam_out[G][c] = lam;
+        if (cw & kTileOwner) a.lam_out[G][con] = lam;
 #pragma unroll
         for (uint32_t u = 0; u < A; ++u)
             if (s[u] != kTileNoRec) rec[s[u]] = r[u];
     }
     __syncthreads();
+    const SceneInfo &sc = a.scenes[T.scene];
+    const bool contacts = RIGID && (stages >> (G + 1)) == 0u && sc.rigid_pid;
     for (uint32_t k = tid; k < T.nown; k += kTileThreads) {
         float4 p = lp[k];
+        const uint32_t pid = a.own[T.own0 + k];
         const uint32_t k0 = a.starts[T.start0 + k], k1 = a.starts[T.start0 + k + 1];
         if (k0 != k1 && !(p.w <= kEps)) {
             float tx = 0.0f, ty = 0.0f, tz = 0.0f;
@@ -299,7 +305,8 @@ __global__ __launch_bounds__(kTileThreads) void k_soft_tile(SoftArgs a)
             p.y = p.y + ty;
             p.z = p.z + tz;
         }
-        pout[a.own[T.own0 + k]] = p;
+        if (RIGID && contacts && p.w > kEps) p = rigid_pid_particle(ra, c, sc.col0, ra.pick[pid], p);
+        pout[pid] = p;
     }
 }
 
@@ -428,16 +435,28 @@ __global__ __launch_bounds__(kSoftBlock) void k_soft_scatter(SoftArgs a)
     a.pos[a.slot_of[pid]] = a.posi[(steps & 1u ? (size_t)a.n : 0) + pid];
 }
 
-void launch_soft_iteration(SoftArgs &a, bool gather, bool scatter, bool solve, hipStream_t st)
+// The launch of a group's tiles.
+template <int G>
+static void launch_tile(const SoftArgs &a, const RigidPidArgs &ra, const SubstepConsts &c, bool rigid, hipStream_t st)
+{
+    if (!a.ntiles[G]) return;
+    hipLaunchKernelGGL((rigid ? k_soft_tile<G, true> : k_soft_tile<G, false>), dim3(a.ntiles[G]), dim3(kTileThreads),
+                       a.lds[G], st, a, ra, c);
+}
+
+// rigid: with the iteration's particle-rigid contacts in particle-index order, after the last group.
+void launch_soft_iteration(SoftArgs &a, const SceneBuffers &s, const SubstepConsts &c, bool rigid, bool gather, bool scatter,
+                           bool solve, hipStream_t st)
 {
     // physics_solver.cpp:915-1019: edges solve/apply, bends + dihedrals solve/apply, tets solve/apply
     if (gather) a.solved = 0;
     if (a.nsoft && gather) hipLaunchKernelGGL(k_soft_gather, dim3(grid_n(a.nsoft)), dim3(kSoftBlock), 0, st, a);
     const uint32_t g = grid_n(a.nsoft);
     if (solve && a.tiles) {
-        if (a.ntiles[0]) hipLaunchKernelGGL(k_soft_tile<0>, dim3(a.ntiles[0]), dim3(kTileThreads), a.lds[0], st, a);
-        if (a.ntiles[1]) hipLaunchKernelGGL(k_soft_tile<1>, dim3(a.ntiles[1]), dim3(kTileThreads), a.lds[1], st, a);
-        if (a.ntiles[2]) hipLaunchKernelGGL(k_soft_tile<2>, dim3(a.ntiles[2]), dim3(kTileThreads), a.lds[2], st, a);
+        const RigidPidArgs ra = rigid_pid_args(s, 0);
+        launch_tile<0>(a, ra, c, rigid, st);
+        launch_tile<1>(a, ra, c, rigid, st);
+        launch_tile<2>(a, ra, c, rigid, st);
         ++a.solved;
         for (int k = 0; k < 3; ++k) std::swap(a.lam_in[k], a.lam_out[k]);
     } else if (solve) {
@@ -455,6 +474,7 @@ void launch_soft_iteration(SoftArgs &a, bool gather, bool scatter, bool solve, h
             hipLaunchKernelGGL(k_apply_corrections, dim3(g), dim3(kSoftBlock), 0, st, a, a.inc_t_start, a.corr_t);
         }
     }
+    if (rigid && !(solve && a.tiles)) launch_rigid_pid(s, c, a.tiles ? a.solved : 0u, st);
     if (a.nsoft && scatter) hipLaunchKernelGGL(k_soft_scatter, dim3(g), dim3(kSoftBlock), 0, st, a);
 }
 

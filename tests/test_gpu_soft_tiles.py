@@ -133,3 +133,31 @@ def test_pool_of_different_groups(oracle, iters):
             for k, o in enumerate(oscs):
                 pos, _, vel = pool.readback_scene(k)
                 assert np.array_equal(pos, o.pos) and np.array_equal(vel, o.vel), (some, k)
+
+
+@pytest.mark.parametrize("solves,contacts", [(1, 3), (3, 1), (2, 2)])
+def test_contacts_after_the_last_group(oracle, solves, contacts):
+    """Scenes whose particle-rigid contacts are solved with the tiles of their last group (edges alone,
+    edges and bends, all three groups), in more and in fewer iterations than the constraints."""
+    walls = scenes.container((0.05, 0.505, 0.005), (3.0, 2.0, 2.0))
+    bodies = [star(300), chain(600), scenes.soft_block_part(7, 0.05, translation=(0.3, 0.7, 0.3)),
+              scenes.cloth_part(20, 0.03, translation=(0.3, 0.51, 0.3)),
+              scenes.soft_block_part(7, 0.05, translation=(0.25, 0.67, 0.3))]
+    ses = [scenes.compose([b], cnhip.fluid_material(0.03), walls, "walls") for b in bodies]
+    p = cnhip.default_params(dt=1 / 120, substeps=2, default_iterations=2, max_fluid_neighbors=64,
+                             soft_internal_iterations=solves, soft_contact_iterations=contacts)
+    oscs = [oracle.OracleScene(s) for s in ses]
+    free = [oracle.OracleScene(scene(b)) for b in bodies]
+    with cnhip.Solver(0) as pool:
+        pool.reserve(sum(s.n for s in ses), 64)
+        pool.upload_batch(ses)
+        for some in (None, [1, 3], None):
+            pool.step(p) if some is None else pool.step_scenes(p, some)
+            for k in range(len(ses)) if some is None else some:
+                oracle.step(oscs[k], p)
+                oracle.step(free[k], p)
+            for k, o in enumerate(oscs):
+                pos, _, vel = pool.readback_scene(k)
+                assert np.array_equal(pos, o.pos) and np.array_equal(vel, o.vel), (some, k)
+    # every scene had contacts but the third, whose block hangs clear of the walls
+    assert [not np.array_equal(o.pos, f.pos) for o, f in zip(oscs, free)] == [True, True, False, True, True]
