@@ -44,7 +44,7 @@ struct ContactArgs {
     float4 *vel;
     const float4 *prev;
     float4 *cur;              // fluid solver positions x* + delta (free particles: w = 0)
-    const float4 *dacc;       // current fluid delta
+    float4 *dacc;             // current fluid delta; w: the contacts' path of the substep
     const uint32_t *cls;
     const uint32_t *id;
     const ParticleClass *classes;
@@ -354,9 +354,18 @@ __global__ __launch_bounds__(kBlock) void k_contact_apply(ContactArgs a)
     p.z = p.z + d.z;
     a.pos[t] = p;
     if (pc.kind == CN_PARTICLE_KIND_FLUID) {
-        const float4 dl = a.dacc[t];
-        // D is of no use here: a scene with contacts keeps no candidate lists
-        a.cur[t] = make_float4(p.x + dl.x, p.y + dl.y, p.z + dl.z, 0.0f);
+        // The displacement bound of the candidate lists goes on from the delta pass's: its w keeps
+        // the length of the contacts' path so far, rounded up with the slack of the new position.  (Without
+        // it scenes with contacts walked in every iteration: 83 us against 52 over 262,144 fluid particles.)
+        float4 dl = a.dacc[t];
+        const float qx = p.x + dl.x, qy = p.y + dl.y, qz = p.z + dl.z;
+        const float slack = (fmaxd(fmaxd(fabsf(p.x), fabsf(p.y)), fabsf(p.z)) +
+                             fmaxd(fmaxd(fabsf(qx), fabsf(qy)), fabsf(qz))) * 4.76837158e-7f + 1.0e-30f;
+        if (d.x != 0.0f || d.y != 0.0f || d.z != 0.0f) {
+            dl.w = (dl.w + len3(d.x, d.y, d.z)) * 1.000001f + slack;
+            a.dacc[t].w = dl.w;
+        }
+        a.cur[t] = make_float4(qx, qy, qz, len3(dl.x, dl.y, dl.z) + slack + dl.w);
     }
 }
 

@@ -136,7 +136,7 @@ struct SubstepConsts {
     uint32_t tile_wide;      // halo capacity of the wide delta pass (previous delta read from HBM)
     uint32_t blk_cap;        // cell blocks with a stored halo descriptor
     uint32_t grid_max;       // workgroups of a persistent fluid launch (upper bound)
-    uint32_t superset;       // 1: LDS blocks of fluid-only scenes reuse iteration 0's candidate lists
+    uint32_t superset;       // 1: LDS blocks reuse iteration 0's candidate lists
     uint32_t fluid_iters;    // fluid iterations per substep
     uint32_t viscous;        // 1: some fluid material's viscosity term is on from the second iteration
     uint32_t all_active;     // 1: every scene takes part in the step

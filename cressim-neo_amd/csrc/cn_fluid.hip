@@ -670,13 +670,15 @@ __device__ __forceinline__ float delta_particle(uint32_t i, const DeltaPre &pre,
         if (!changed) break;
     }
     const float ex = cx - p.x, ey = cy - p.y, ez = cz - p.z;
-    a.dout[i] = make_float4(ex, ey, ez, 0.0f);
+    // w: how far contacts have moved x* in the substep (k_contact_apply)
+    const float moved = a.it > 0 ? di.w : 0.0f;
+    a.dout[i] = make_float4(ex, ey, ez, moved);
     const float nx = p.x + ex, ny = p.y + ey, nz = p.z + ez;
     // |delta| plus a few ulps of the position: D, the bound on the displacement since iteration 0
     // that the candidate lists go by; it also bounds the next iteration's relDelta for the CFL skip
     const float slack = fmaxd(fmaxd(fabsf(nx), fabsf(ny)), fabsf(nz)) * 4.76837158e-7f + 1.0e-30f;
     const float dl = len3(ex, ey, ez) + slack;
-    a.cur[i] = make_float4(nx, ny, nz, p.w > kEps ? dl : kNoMass);
+    a.cur[i] = make_float4(nx, ny, nz, p.w > kEps ? dl + moved : kNoMass);
     return dl * dl;
 }
 
@@ -1318,9 +1320,8 @@ __global__ __launch_bounds__(kTileBlock) __attribute__((amdgpu_waves_per_eu(kDen
             }
             const int any_mixed = __syncthreads_or(mixed ? 1 : 0);  // also the barrier after staging
             const bool bu = UNIFORM || !any_mixed;
-            // candidate lists apply to fluid-only scenes (only the fluid passes move their particles
-            // within a substep, and they record every displacement)
-            const bool sup = (BUILD || REUSE) && ts.fluid_only;
+            // the fluid passes and the contacts record every displacement of a fluid particle
+            const bool sup = BUILD || REUSE;
             // The candidates of iteration 0 (within h + skin of x*) hold particle i's list while
             // D_i + D_j < skin for every j in its 27 cells: a pair within h now was within
             // h + D_i + D_j then (D: displacement since iteration 0, x* to x* + delta).  D_j is

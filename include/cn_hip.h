@@ -217,11 +217,11 @@ typedef struct cn_step_params {
     uint32_t flags;                  /* CN_STEP_* bits (cn_default_step_params: CN_STEP_CANDIDATE_REUSE) */
 } cn_step_params;
 
-/* flags: in fluid-only scenes the fluid iterations after a substep's first take the neighbors from
- * the candidate lists its first iteration builds (neighbors within 1.05 h of the positions at the
- * first iteration) instead of walking the 27 cells again, in every cell block whose particles'
- * displacement since the first iteration plus the largest one in the block's halo stays below
- * 0.05 h; the other blocks walk.  The lists are the same either way (same neighbors, same order),
+/* flags: the fluid iterations after a substep's first take the neighbors from the candidate lists
+ * its first iteration builds (neighbors within 1.05 h of the positions at the first iteration) instead
+ * of walking the 27 cells again, in every cell block whose particles' displacement since the first
+ * iteration (by the fluid passes and by contacts) plus the largest one in the block's halo stays
+ * below 0.05 h; the other blocks walk.  The lists are the same either way (same neighbors, same order),
  * so the results are too.  The candidate lists take 198 bytes per particle, allocated on the first
  * step that asks (left off when they would exceed 4 GiB less 1 MiB).  On in
  * cn_default_step_params. */
