@@ -136,7 +136,11 @@ struct CorrRec {
 // (edges; bends and dihedrals; tets) a workgroup loads the tile's particles and those its constraints
 // reach (the halo), solves every constraint that touches one of its particles, and sums its own
 // particles' correction records, all in LDS.
-constexpr uint32_t kSoftTile = 256;
+// Constrained particles of a tile.  Up to kSoftFew of them tiles of 256 would leave CUs with fewer than
+// two, and what a pass takes is a tile's latency: half the particles a tile take a 32^3 tet block from
+// 752 to 667 us a step and a 256 x 256 cloth from 737 to 719.  Past that the larger tiles' fewer border
+// constraints count: 48 mixed scenes 4,807 against 4,868 us.
+constexpr uint32_t kSoftTile = 256, kSoftFew = 2 * 256 * kSoftTile;
 constexpr uint32_t kSoftTileLds = 76u * 1024u;  // two workgroups per CU
 constexpr uint32_t kTileOwner = 0x80000000u;    // constraint word: this tile writes its lambda
 constexpr uint16_t kTileNoRec = 0xffffu;        // record slot of a vertex that is not the tile's own

@@ -220,8 +220,8 @@ __device__ __forceinline__ bool solve_tet(const float4 p0, const float4 p1, cons
 // some 45 bytes instead of 144 and an edge 35 instead of 80, for 1.3 to 1.5 times the solves, and an
 // iteration takes half the launches: 48 mixed scenes 6,033 -> 4,955 us a step, a 256 x 256 cloth
 // 996 -> 829 us (both of 4 substeps and 4 iterations; 2 x 2 launches an iteration before, 2 now).
-// What bounds it: the latency of a tile's three phases (load, solve, sum), 250 tiles to 64,000
-// particles being one a CU.
+// What bounds it: the latency of a tile's three phases (load, solve, sum), 500 tiles of 128 to 64,000
+// particles being two a CU.
 constexpr int kTileThreads = 512;
 // RIGID: a scene's last group also solves the iteration's particle-rigid contacts of its particles (a
 // launch of their own took 5 us an iteration: a 256 x 256 cloth's step 829 us against 766, a 32^3 tet

@@ -208,7 +208,7 @@ bool build_soft_tiles(uint32_t n, const float *pos, const std::vector<uint32_t> 
     for (int g = 0; g < 3; ++g)
         for (uint32_t c = 0; c < topo.count[g]; ++c) out.stages[pid_scene[topo.vertex(g, c, 0)]] |= 1u << g;
     std::vector<uint32_t> tile_of(n, kNone), in_tile(n), first;
-    for (uint32_t most = kSoftTile; most >= 8u; most /= 2) {
+    for (uint32_t most = soft.size() <= kSoftFew ? kSoftTile / 2 : kSoftTile; most >= 8u; most /= 2) {
         // tiles, scene by scene (soft is ascending, and so are its scenes)
         out.own.assign(soft.begin(), soft.end());
         first.assign(1, 0u);

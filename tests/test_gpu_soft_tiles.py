@@ -77,6 +77,11 @@ def test_tile_borders(solver, oracle, n):
     same(solver, oracle, scene(chain(n)), params())
 
 
+@pytest.mark.parametrize("side", [362, 363])  # 131,044 and 131,769 particles: tiles of 128 and of 256
+def test_tile_sizes(solver, oracle, side):
+    same(solver, oracle, scene(scenes.cloth_part(side, 0.03)), params(2, 1), steps=1)
+
+
 # 2,779 records with the particles at their other ends fill the LDS of a tile; past that the whole-pool passes run
 @pytest.mark.parametrize("leaves", [300, 2700, 2900])
 def test_star(solver, oracle, leaves):
