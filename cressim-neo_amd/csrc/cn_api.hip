@@ -21,7 +21,7 @@
 using namespace cn;
 
 // Device scratch of cn_pass_sort_pairs_noalloc: two pair buffers of CN_NOALLOC_MAX_PAIRS entries and
-// the radix sort's per-tile digit counts for that many pairs (256 digits x 256 tiles + 256 totals).
+// the radix sort's per-tile digit counts for that many pairs (256 digits x 512 tiles + 256 totals).
 // Every GPU the library runs on holds its own copy from module load until the process ends.  In
 // host code `scratch` is only a stand-in for the symbol: its device address on the current GPU
 // comes from hipGetSymbolAddress (noalloc_scratch below), and only that address reaches a kernel.

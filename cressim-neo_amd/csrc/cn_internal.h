@@ -95,7 +95,7 @@ struct FluidConst {
 
 // ---- radix sort (cn_sort.hip) ----
 constexpr uint32_t kDirectTiles = 128;  // tiles whose counts a scatter workgroup sums itself
-size_t sort_scratch_words(uint32_t n);
+size_t sort_scratch_words(uint32_t n);  // for every sort of at most n pairs
 uint32_t sort_rounds(uint32_t n);   // a tile holds 256 x rounds pairs
 bool sort_one_group(uint32_t n);    // sorted in one launch, without counts
 uint2 *radix_sort_pairs(uint2 *buf_a, uint2 *buf_b, uint32_t n, uint32_t key_bits, uint32_t *scratch, bool counted,

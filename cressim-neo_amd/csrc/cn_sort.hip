@@ -50,9 +50,11 @@ struct PairOut {
 
 // Rounds of a tile: small tiles while their counts are summed directly, and in larger sorts as many
 // as leave every CU a few workgroups (a wave's ranks are a serial chain, some 300 ns a round).
+// The tiles grow at these sizes, so their number falls there: sort_scratch_words looks at both.
+constexpr uint32_t kRoundsFour = 1024u * kDirectTiles, kRoundsEight = 4u * 1024u * 1024u;
 uint32_t sort_rounds(uint32_t n)
 {
-    return n <= 1024u * kDirectTiles ? 4u : (n <= 4u * 1024u * 1024u ? 8u : 16u);
+    return n <= kRoundsFour ? 4u : (n <= kRoundsEight ? 8u : 16u);
 }
 static uint32_t sort_tiles(uint32_t n)
 {
@@ -251,10 +253,13 @@ __global__ __launch_bounds__(kOneThreads) void k_radix_one_group(PairIn in, Pair
     }
 }
 
-// Scratch words of a sort of at most n pairs (the tiles of a smaller sort may be more than n's).
+// Scratch words of every sort of at most n pairs: a smaller sort has more tiles than n's where n lies
+// past a size at which the tiles grow (4,000,000 pairs have 1,954, 5,000,000 have 1,221).
 size_t sort_scratch_words(uint32_t n)
 {
-    return (size_t)256 * std::max<uint32_t>(sort_tiles(n), kDirectTiles) + 256;
+    uint32_t tiles = sort_tiles(n);
+    for (uint32_t most : {kRoundsFour, kRoundsEight}) tiles = std::max(tiles, sort_tiles(std::min(n, most)));
+    return (size_t)256 * tiles + 256;
 }
 
 template <int R>
