@@ -369,11 +369,12 @@ __device__ __forceinline__ void density_add(DensitySum &d, const DensitySelf &x,
     }
 }
 
-// Calls f(collider) for every candidate collider of a slot in visit order, for a wave whose
-// particles belong to one scene (colliders col0 .. col0 + ncol).  Candidates held as a bitmask are
-// taken collider by collider over the whole wave, so each is read once through the scalar cache
-// (the tables are constant during a launch); a lane-by-lane walk of the bits made every collider a
-// round trip of vector loads, some 3 us of a block's latency near a wall.
+// Calls f(collider) for every candidate collider of a slot in visit order; col0 is the first collider of
+// the lane's scene, and a wave may hold particles of several (the launches of a thread per slot).
+// Candidates are taken collider by collider over the whole wave, by their index in the pool's table, so
+// each is read once through the scalar cache (the tables are constant during a launch); a lane-by-lane
+// walk of the bits made every collider a round trip of vector loads, some 3 us of a block's latency near
+// a wall.
 __device__ __forceinline__ Collider const_collider(const Collider *col)
 {
     typedef const __attribute__((address_space(4))) uint32_t *ConstWords;
@@ -394,10 +395,10 @@ __device__ __forceinline__ void each_collider(uint32_t word, const FluidArgs &a,
     uint32_t left = listed ? min(word & 0xffu, kBndListCap) : word;  // entries left, or bits left
     for (uint64_t any = __ballot(left != 0u); any; any = __ballot(left != 0u)) {
         // the next candidate of the first lane with one left; every lane whose next it is takes it
-        const uint32_t mine = !left ? kInvalid : (listed ? (uint32_t)*l : (uint32_t)__builtin_ctz(left));
+        const uint32_t mine = !left ? kInvalid : col0 + (listed ? (uint32_t)*l : (uint32_t)__builtin_ctz(left));
         const uint32_t k = (uint32_t)__builtin_amdgcn_readlane((int)mine, (int)__builtin_ctzll(any));
         if (mine == k) {
-            f(const_collider(a.col + __builtin_amdgcn_readfirstlane(col0) + k));
+            f(const_collider(a.col + k));
             left = listed ? left - 1u : left & (left - 1u);
             l += listed ? 1 : 0;
         }
