@@ -177,6 +177,7 @@ SIGNATURES = {
     "cn_validate_meta": (C.c_int, [_P, C.POINTER(Meta)]),
     "cn_synchronize": (C.c_int, [_P]),
     "cn_query": (C.c_int, [_P]),
+    "cn_objects_loaded": (C.c_uint64, []),
     "cn_pass_broadphase_keys": (C.c_int, [_P, _U, _P, C.c_float, _P, _P]),
     "cn_pass_sort_pairs": (C.c_int, [_P, _U, _P, _P]),
     "cn_pass_sort_pairs_noalloc": (C.c_int, [_P, _U, C.c_void_p, C.c_void_p]),
@@ -217,33 +218,10 @@ def hip_runtimes_mapped() -> list:
     return sorted(seen)
 
 
-class _PhdrInfo(C.Structure):
-    _fields_ = [("addr", C.c_void_p), ("name", C.c_char_p), ("phdr", C.c_void_p), ("phnum", C.c_uint16),
-                ("adds", C.c_ulonglong), ("subs", C.c_ulonglong)]
-
-
-_phdr_adds = C.c_ulonglong()
-
-
-@C.CFUNCTYPE(C.c_int, C.POINTER(_PhdrInfo), C.c_size_t, C.c_void_p)
-def _first_phdr(info, size, _):
-    _phdr_adds.value = info.contents.adds if size >= C.sizeof(_PhdrInfo) else 0
-    return 1  # the counter is the same in every record
-
-
-try:
-    _iterate_phdr = C.CDLL(None).dl_iterate_phdr
-except (AttributeError, OSError):  # pragma: no cover - another libc
-    _iterate_phdr = None
-
-
 def objects_loaded() -> int | None:
     """How many shared objects this process has loaded since it started (the dynamic linker's own
-    counter), or None where the linker does not tell."""
-    if _iterate_phdr is None:
-        return None
-    _iterate_phdr(_first_phdr, None)
-    return _phdr_adds.value or None
+    counter), or None where the linker keeps none or the library is not loaded."""
+    return (_lib.cn_objects_loaded() or None) if _lib is not None else None
 
 
 _single_at = None  # objects_loaded() when one runtime was last found mapped

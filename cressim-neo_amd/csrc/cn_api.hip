@@ -5,6 +5,7 @@
 // update and the fluid boundary velocity projection.  Every pass is a kernel on the context's
 // stream; nothing here synchronizes except readback, validation and profiling reads.
 #include <hip/hip_runtime.h>
+#include <link.h>
 
 #include <algorithm>
 #include <array>
@@ -684,6 +685,20 @@ uint2 *broadphase(cn_ctx *ctx, SceneBuffers &s, const SubstepConsts &c, uint32_t
 extern "C" {
 
 uint32_t cn_abi_version(void) { return CN_ABI_VERSION; }
+
+// The linker holds its lock while it calls back, so the callback takes no other lock: one that ran Python
+// would wait for the interpreter's while an importing thread holds that and waits for the linker's.
+uint64_t cn_objects_loaded(void)
+{
+    uint64_t adds = 0;
+    dl_iterate_phdr(
+        [](dl_phdr_info *info, size_t size, void *out) {
+            if (size >= offsetof(dl_phdr_info, dlpi_adds) + sizeof(info->dlpi_adds)) *(uint64_t *)out = info->dlpi_adds;
+            return 1;  // the counter is the same in every record
+        },
+        &adds);
+    return adds;
+}
 
 cn_status cn_ctx_create(const cn_device_desc *desc, cn_ctx **out)
 {

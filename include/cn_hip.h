@@ -268,6 +268,9 @@ typedef struct cn_device_desc {
 
 /* -------- context -------- */
 uint32_t cn_abi_version(void);
+/* How many shared objects the process has loaded since it started (the dynamic linker's own counter;
+ * 0 where it keeps none).  May be called from any thread. */
+uint64_t cn_objects_loaded(void);
 cn_status cn_ctx_create(const cn_device_desc *desc, cn_ctx **out_ctx);
 void cn_ctx_destroy(cn_ctx *ctx);
 const char *cn_last_error(const cn_ctx *ctx);
