@@ -18,10 +18,11 @@ constexpr float kEps = 1.0e-6f;              // kEpsilon, physics_base.hlsli:7
 constexpr uint32_t kInvalid = 0xffffffffu;   // kInvalidIndex, physics_base.hlsli:6
 constexpr float kKernelPi = 3.14159265359f;  // physics_fluid_common.hlsli:26
 constexpr float kBroadPhaseMargin = 0.05f;   // physics_shape_common.hlsli:10
-constexpr uint32_t kMaskColliders = 32;      // a scene of at most this many colliders: candidate bitmasks
+constexpr uint32_t kMaskColliders = 31;      // a scene of at most this many colliders: candidate bitmasks
 constexpr uint32_t kMaxColliders = 65535;    // colliders of one scene (16-bit candidate entries)
 constexpr uint32_t kBndList = 0x80000000u;   // candidate word: the low bits count list entries
 constexpr uint32_t kBndListCap = 32;         // candidate colliders a particle holds in a list
+static_assert(kMaskColliders <= 31 && kMaskColliders <= kBndListCap, "no mask reads as a list");
 constexpr uint32_t kColGroup = 32;           // colliders per group of the two-level candidate search
 constexpr int kBlock = 256;                  // threads per workgroup for per-particle kernels
 
