@@ -125,8 +125,14 @@ __device__ __forceinline__ void walk_rows(const uint32_t *hoff, int hc, F &&f)
 // counter; the counters hand out what is left, and none is touched when a chunk has no more blocks
 // than workgroups with a fixed first one.  (A counter's atomic is a round trip to the memory side of
 // about a microsecond: taking the first block and finding eight drained chunks by atomics cost a
-// launch over the 64,000-particle dam break some 10 us of its 40.)  Run by one thread.
-constexpr uint32_t kFixedPerDie = 96;  // workgroups of a die with a fixed first block: those resident
+// launch over the 64,000-particle dam break some 10 us of its 40.)  Run by one thread, when the block
+// before is done: a block taken while the one before was still worked on waited for it where the others
+// had none left (4,096 particles spread among 262 colliders, 6.6 ms a step against 4.3; a random fill of
+// 1,048,573, 5.86 against 5.69).
+// Workgroups of a die with a fixed first block: those of the density pass that are resident in a large
+// scene.  (64, what the delta pass keeps resident, left a third of the density pass's without work: a step
+// of 4,194,304 particles 17.3 ms against 16.3, of 1,048,573 5.6 against 5.7.)
+constexpr uint32_t kFixedPerDie = 96;
 struct BlockQueue {
     uint32_t die, open;  // open: bit d set while chunk d may have blocks
     bool helping;
@@ -1281,11 +1287,11 @@ __global__ __launch_bounds__(kTileBlock) __attribute__((amdgpu_waves_per_eu(kDen
     uint32_t after;
     for (uint32_t blk = BlockQueue::first(blockIdx.x, nblk); blk != kInvalid; blk = after) {
         tile_load(ts, blk, hoff, hstart, 0u, a, c);
-        if (tid == 0) s_blk = bq.next(queue, nblk);  // the next block, while this one's tables arrive
         __syncthreads();
-        after = s_blk;
         if (ts.skip) {
+            if (tid == 0) s_blk = bq.next(queue, nblk);
             __syncthreads();
+            after = s_blk;
             continue;
         }
         MetaAcc ma;
@@ -1451,7 +1457,9 @@ __global__ __launch_bounds__(kTileBlock) __attribute__((amdgpu_waves_per_eu(kDen
             if (tid == 0) ++ma.runs;
         }
         meta_to_wg(ma, s_meta);
+        if (tid == 0) s_blk = bq.next(queue, nblk);  // not before the block is done: see BlockQueue
         __syncthreads();
+        after = s_blk;
         if (tid == 0) s_hmax = s_omax = 0u;  // read again only after the next block's staging barrier
     }
     flush_wg_meta(s_meta, a);
@@ -1503,11 +1511,11 @@ __global__ __launch_bounds__(kTileBlock) __attribute__((amdgpu_waves_per_eu(kDel
     uint32_t after;
     for (uint32_t blk = first; blk != kInvalid; blk = after) {
         tile_load(ts, blk, hoff, hstart, WIDE || !use_d ? 0u : c.tile_wide, a, c);
-        if (tid == 0) s_blk = next();  // the next block, while this one's tables arrive
         __syncthreads();
-        after = s_blk;
         if (ts.skip) {
+            if (tid == 0) s_blk = next();
             __syncthreads();
+            after = s_blk;
             continue;
         }
         // the block's class
@@ -1634,7 +1642,9 @@ __global__ __launch_bounds__(kTileBlock) __attribute__((amdgpu_waves_per_eu(kDel
             particles(std::true_type{});
         else
             particles(std::false_type{});
+        if (tid == 0) s_blk = next();
         __syncthreads();
+        after = s_blk;
     }
     flush_disp(d2max, a);
 }
