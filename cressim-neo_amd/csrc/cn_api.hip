@@ -75,6 +75,7 @@ struct cn_ctx {
     bool uploaded = false;
     bool stepped = false;        // a cn_step ran since the upload (slot order differs from index order)
     float cell_size = 0.0f;      // derived on upload like the reference world
+    float fluid_blocks = 0.0f;   // cell blocks with fluid per particle, as uploaded (launch shapes)
     uint32_t morton_bits = 10;
     uint32_t bucket_bits_alloc = 4;  // bucket index bits the allocation holds
     float max_h = 0.0f;              // largest fluid smoothing radius of the scene
@@ -638,6 +639,7 @@ SubstepConsts make_consts(const cn_ctx *ctx, const SceneBuffers &s, const cn_ste
     c.tile_max = ctx->tile_max;
     c.blk_cap = s.blk_cap;
     c.grid_max = ctx->grid_max;
+    c.blocks = (uint32_t)(ctx->fluid_blocks * (float)s.n);
     c.superset = (p->flags & CN_STEP_CANDIDATE_REUSE) && s.slist ? 1u : 0u;
     c.fluid_iters = p->fluid_iterations > 0 ? p->fluid_iterations : std::max<uint32_t>(p->default_iterations, 1u);
     c.pairs = ctx->any_pairs ? 1u : 0u;
@@ -1078,6 +1080,34 @@ cn_status upload_tiles(cn_ctx *ctx, uint32_t n, const SoftTopology &topo, SoftTi
     return CN_OK;
 }
 
+// How many 4x4x4-cell blocks of a pool hold fluid, for the launch shapes of the fluid passes: every
+// fourth particle's block of the first kLook particles, told apart by a 16-bit hash (0.1 ms for 64,000).
+struct BlockEstimate {
+    static constexpr uint32_t kLook = 256u * 1024u;
+    std::vector<uint64_t> seen = std::vector<uint64_t>(65536 / 64);
+    uint32_t blocks = 0, looked = 0;
+    void add(uint32_t scene, const cn_particle_soa_view &pv, float inv_cell)
+    {
+        const uint32_t m = std::min<uint32_t>(pv.count, kLook - looked);
+        looked += m;
+        for (uint32_t i = 0; i < m; i += 4) {
+            if (pv.kinds[i] != CN_PARTICLE_KIND_FLUID) continue;
+            const float *p = pv.positions_inv_mass + 4ull * i;
+            uint32_t h = scene * 0x9e3779b1u;
+            for (int a = 0; a < 3; ++a) {
+                const float b = std::floor(0.25f * p[a] * inv_cell);
+                h = (h ^ (uint32_t)(std::fabs(b) < 1.0e9f ? (int32_t)b : 0)) * 0x85ebca6bu;
+                h ^= h >> 15;
+            }
+            uint64_t &w = seen[(h >> 22) & 1023u];
+            const uint64_t bit = 1ull << ((h >> 16) & 63u);
+            blocks += (w & bit) == 0;
+            w |= bit;
+        }
+    }
+    float per_particle() const { return looked ? (float)blocks / (float)looked : 0.0f; }
+};
+
 // Uploads a pool of independent scenes: particles, classes, materials and constraints are
 // concatenated with index offsets, colliders are visit-ordered per scene, and each scene gets its
 // own cell size and key range.  One scene is the plain path.
@@ -1158,6 +1188,7 @@ cn_status upload_pool(cn_ctx *ctx, uint32_t count, const cn_scene_desc *descs)
     ctx->fm_fluid_used.clear();
     uint32_t base = 0;
     double max_span = 1.0;
+    BlockEstimate est;
     for (uint32_t k = 0; k < count; ++k) {
         const cn_particle_soa_view *pv = descs[k].particles;
         const cn_scene_tables *tb = descs[k].tables;
@@ -1291,6 +1322,7 @@ cn_status upload_pool(cn_ctx *ctx, uint32_t count, const cn_scene_desc *descs)
                                                       tb->fluid_material_count, tb->fluid_materials);
         ctx->scene_cell[k] = cell;
         sinfo[k].inv_cell = 1.0f / std::max(cell, 1.0e-4f);
+        est.add(k, *pv, sinfo[k].inv_cell);
         float lo[3] = {3.4e38f, 3.4e38f, 3.4e38f}, hi[3] = {-3.4e38f, -3.4e38f, -3.4e38f};
         for (uint32_t i = 0; i < m; ++i)
             for (int a = 0; a < 3; ++a) {
@@ -1313,6 +1345,7 @@ cn_status upload_pool(cn_ctx *ctx, uint32_t count, const cn_scene_desc *descs)
     }
     ctx->scene_first[count] = base;
     ctx->cell_size = ctx->scene_cell[0];
+    ctx->fluid_blocks = est.per_particle();
     // key layout: [scene index | 3 x morton_bits]; coordinates beyond 2^morton_bits cells wrap and
     // their runs are filtered per particle
     ctx->scene_bits = count > 1 ? ceil_log2(count) : 0u;

@@ -136,6 +136,7 @@ struct SubstepConsts {
     uint32_t tile_delta;     // halo capacity of the delta pass from the second iteration on
     uint32_t tile_wide;      // halo capacity of the wide delta pass (previous delta read from HBM)
     uint32_t blk_cap;        // cell blocks with a stored halo descriptor
+    uint32_t blocks;         // cell blocks with fluid, estimated from the upload (launch shapes)
     uint32_t grid_max;       // workgroups of a persistent fluid launch (upper bound)
     uint32_t superset;       // 1: LDS blocks reuse iteration 0's candidate lists
     uint32_t fluid_iters;    // fluid iterations per substep

@@ -2195,12 +2195,14 @@ static uint32_t grid_of(uint32_t n) { return (n + kBlock - 1) / kBlock; }
 
 // LDS budget of one tiled workgroup (the static halo table and counters take some 2 KiB more).  In a
 // large scene three workgroups of the density pass and two of the delta pass share a CU's 160 KiB; a
-// scene whose cell blocks (some 400 particles each, fewer at its surface) leave a CU one or two
-// workgroups lets each have what the others would not use, so that fewer blocks need the wide layout
-// or the run table.
+// scene whose cell blocks leave a CU one or two workgroups (256 and 512 blocks, of some 400 particles in
+// a fluid at rest) lets each have what the others would not use, so that fewer blocks need the wide
+// layout or the run table.  A scene of few particles in many blocks (a spray, a thin sheet, many small
+// scenes) does not: 90,000 particles in 7,000 blocks took 16.9 ms a step with a CU to each workgroup.
 static uint32_t lds_budget(const SubstepConsts &c, uint32_t share)
 {
-    const uint32_t fits = c.n <= 96u * 1024u ? 1u : (c.n <= 192u * 1024u ? 2u : 3u);
+    const uint32_t by_n = c.n <= 96u * 1024u ? 1u : (c.n <= 192u * 1024u ? 2u : 3u);
+    const uint32_t fits = std::max(by_n, c.blocks <= 256u ? 1u : (c.blocks <= 512u ? 2u : 3u));
     return 156u * 1024u / std::min(share, fits) - 2u * 1024u;
 }
 
