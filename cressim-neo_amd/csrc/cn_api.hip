@@ -1080,17 +1080,17 @@ cn_status upload_tiles(cn_ctx *ctx, uint32_t n, const SoftTopology &topo, SoftTi
     return CN_OK;
 }
 
-// How many 4x4x4-cell blocks of a pool hold fluid, for the launch shapes of the fluid passes: every
-// fourth particle's block of the first kLook particles, told apart by a 16-bit hash (0.1 ms for 64,000).
+// How many 4x4x4-cell blocks of a pool hold fluid, for the launch shapes of the fluid passes: the blocks
+// of every kEvery-th of the first kLook particles, told apart by a 16-bit hash.
 struct BlockEstimate {
-    static constexpr uint32_t kLook = 256u * 1024u;
+    static constexpr uint32_t kLook = 256u * 1024u, kEvery = 16u;
     std::vector<uint64_t> seen = std::vector<uint64_t>(65536 / 64);
     uint32_t blocks = 0, looked = 0;
     void add(uint32_t scene, const cn_particle_soa_view &pv, float inv_cell)
     {
         const uint32_t m = std::min<uint32_t>(pv.count, kLook - looked);
         looked += m;
-        for (uint32_t i = 0; i < m; i += 4) {
+        for (uint32_t i = 0; i < m; i += kEvery) {
             if (pv.kinds[i] != CN_PARTICLE_KIND_FLUID) continue;
             const float *p = pv.positions_inv_mass + 4ull * i;
             uint32_t h = scene * 0x9e3779b1u;

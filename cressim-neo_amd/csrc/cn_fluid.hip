@@ -2198,7 +2198,8 @@ static uint32_t grid_of(uint32_t n) { return (n + kBlock - 1) / kBlock; }
 // scene whose cell blocks leave a CU one or two workgroups (256 and 512 blocks, of some 400 particles in
 // a fluid at rest) lets each have what the others would not use, so that fewer blocks need the wide
 // layout or the run table.  A scene of few particles in many blocks (a spray, a thin sheet, many small
-// scenes) does not: 90,000 particles in 7,000 blocks took 16.9 ms a step with a CU to each workgroup.
+// scenes) does not: 90,000 particles in 7,000 blocks took 16.9 ms a step with a CU
+// to each workgroup, and take 11.5.
 static uint32_t lds_budget(const SubstepConsts &c, uint32_t share)
 {
     const uint32_t by_n = c.n <= 96u * 1024u ? 1u : (c.n <= 192u * 1024u ? 2u : 3u);
