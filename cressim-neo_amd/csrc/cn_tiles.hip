@@ -67,14 +67,17 @@ struct Cut {
     uint32_t n;
 };
 
-// The tiles of one constraint group; false when one does not fit a workgroup's LDS.
+// Whether a group's tiles fit a workgroup's LDS; never: one particle's constraints alone do not.
+enum class Fit { yes, no, never };
+
+// The tiles of one constraint group.
 template <int GROUP>
-bool build_group(const Cut &cut, const SoftTopology &topo, SoftTilesHost::Group &G)
+Fit build_group(const Cut &cut, const SoftTopology &topo, SoftTilesHost::Group &G)
 {
     constexpr uint32_t A = GROUP == 0 ? 2u : 4u;
     G = SoftTilesHost::Group{};
     const uint32_t nc = topo.count[GROUP], ntile = (uint32_t)cut.first.size() - 1;
-    if (!nc) return true;
+    if (!nc) return Fit::yes;
     // the distinct tiles of a constraint's vertices, the first vertex's first
     auto tiles_of = [&](uint32_t c, uint32_t (&p)[4], uint32_t (&ts)[4]) {
         uint32_t m = 0;
@@ -96,6 +99,23 @@ bool build_group(const Cut &cut, const SoftTopology &topo, SoftTilesHost::Group 
         for (uint32_t q = 0; q < m; ++q) ++ent[ts[q] + 1];
         for (uint32_t k = 0; k < A; ++k)
             if (p[k] != kNone) ++deg[p[k]];
+    }
+    {
+        // the particle of the most constraints: its records, its position and those of its partners
+        const uint32_t hub = (uint32_t)(std::max_element(deg.begin(), deg.end()) - deg.begin());
+        const size_t records = deg[hub] * sizeof(CorrRec) + sizeof(float4);
+        if (records + (size_t)deg[hub] * (A - 1) * sizeof(float4) > kSoftTileLds) {
+            std::vector<uint32_t> partners;
+            for (uint32_t c = 0; c < nc; ++c) {
+                bool of = false;
+                for (uint32_t k = 0; k < A; ++k) of |= topo.vertex(GROUP, c, k) == hub;
+                for (uint32_t k = 0; of && k < A; ++k)
+                    if (const uint32_t q = topo.vertex(GROUP, c, k); q != kNone && q != hub) partners.push_back(q);
+            }
+            std::sort(partners.begin(), partners.end());
+            partners.erase(std::unique(partners.begin(), partners.end()), partners.end());
+            if (records + partners.size() * sizeof(float4) > kSoftTileLds) return Fit::never;
+        }
     }
     for (uint32_t t = 0; t < ntile; ++t) ent[t + 1] += ent[t];
     G.con.resize(ent[ntile]);
@@ -192,9 +212,9 @@ bool build_group(const Cut &cut, const SoftTopology &topo, SoftTilesHost::Group 
         G.halo.insert(G.halo.end(), R.halo.begin(), R.halo.end());
         G.starts.insert(G.starts.end(), R.starts.begin(), R.starts.end());
         G.lds = std::max(G.lds, R.lds);
-        if (!R.fits) return false;  // the runs still filling end before this returns
+        if (!R.fits) return Fit::no;  // the runs still filling end before this returns
     }
-    return true;
+    return Fit::yes;
 }
 
 }  // namespace
@@ -229,11 +249,11 @@ bool build_soft_tiles(uint32_t n, const float *pos, const std::vector<uint32_t> 
         }
         const Cut c{out.own, first, tile_of, in_tile, pid_scene, out.stages, n};
         // the groups are independent: the edges' and the bends' beside the tets'
-        std::future<bool> e = run_aside([&] { return build_group<0>(c, topo, out.group[0]); });
-        std::future<bool> b = run_aside([&] { return build_group<1>(c, topo, out.group[1]); });
-        const bool t = build_group<2>(c, topo, out.group[2]);
-        const bool fe = e.get(), fb = b.get();
-        if (t && fe && fb) return true;
+        std::future<Fit> e = run_aside([&] { return build_group<0>(c, topo, out.group[0]); });
+        std::future<Fit> b = run_aside([&] { return build_group<1>(c, topo, out.group[1]); });
+        const Fit fit[3] = {build_group<2>(c, topo, out.group[2]), e.get(), b.get()};
+        if (std::count(fit, fit + 3, Fit::yes) == 3) return true;
+        if (std::count(fit, fit + 3, Fit::never)) return false;
     }
     return false;
 }
