@@ -2032,7 +2032,7 @@ static cn_status step_impl(cn_ctx *ctx, const cn_step_params *p)
     if (p->max_fluid_neighbors > ctx->cap_alloc)
         return fail(ctx, CN_ERR_CAPACITY, "max_fluid_neighbors exceeds the neighbor slots of cn_scene_reserve");
     CN_HIP(ctx, hipSetDevice(ctx->device));
-    // candidate lists on first use, for scenes with fluid, when they fit the 32-bit list addressing
+    // candidate lists on first use, for scenes with fluid, when they stay within a pool's list bytes
     if ((p->flags & CN_STEP_CANDIDATE_REUSE) && !ctx->s.slist && ctx->has_fluid &&
         (uint64_t)list_slots(ctx->capacity) * kSuperSlots * sizeof(uint16_t) <= kListBytesMax) {
         CN_HIP(ctx, hipStreamSynchronize(ctx->stream));

@@ -163,7 +163,6 @@ __device__ __forceinline__ float fdiv_rcp_neg(float a, float b, float y)
     const float r = __builtin_fmaf(-q0, b, a);
     return __builtin_fmaf(-r, y, -q0);  // -(a / b)
 }
-__device__ __forceinline__ float fdiv_rcp(float a, float b, float y) { return -fdiv_rcp_neg(a, b, y); }
 
 // One Newton step in fma from an estimate y of 1 / b.  From this chip's reciprocal estimate, and from
 // its reciprocal square-root estimate of x where b is the root of x (fsqrt_rsq), it reaches the
@@ -275,24 +274,10 @@ __device__ __forceinline__ float spiky_dw_k(float d, float h, float k)
 }
 __device__ __forceinline__ float spiky_w(float d, float h) { return spiky_w_k(d, h, spiky_coef(h)); }
 __device__ __forceinline__ float spiky_dw(float d, float h) { return spiky_dw_k(d, h, spiky_coef(h)); }
-__device__ __forceinline__ float cohesion_kernel(float d, float h, float c1, float c2)
-{
-    if (d <= kEps || d >= h) return 0.0f;
-    const float q = fdiv(d, h);
-    const float a = __fmul_rn(__fmul_rn(__fmul_rn(c1, q), q), q);
-    const float b = __fmul_rn(__fmul_rn(c2, q), q);
-    return __fsub_rn(__fadd_rn(a, b), 1.0f);
-}
-
 // The same kernels from q = d / h supplied by the caller (the per-neighbor fluid terms share
 // one quotient between the kernels of a pair).
-__device__ __forceinline__ float spiky_w_om(float d, float h, float omq, float k)  // omq = 1 - d / h
-{
-    if (d >= h) return 0.0f;
-    return __fmul_rn(__fmul_rn(k, omq), omq);
-}
-// The same for a pair known to lie within h (a listed neighbor: its squared distance is below the
-// threshold whose rounded root is h), where the range test is always false.
+// omq = 1 - d / h, for a pair known to lie within h (a listed neighbor: its squared distance is below the
+// threshold whose rounded root is h), where the kernel's range test is always false.
 __device__ __forceinline__ float spiky_w_om_in(float omq, float k) { return __fmul_rn(__fmul_rn(k, omq), omq); }
 __device__ __forceinline__ float cohesion_q(float d, float h, float q, float c1, float c2)
 {

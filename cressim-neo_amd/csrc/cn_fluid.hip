@@ -237,17 +237,17 @@ struct DensitySum {
 };
 
 // Quotients of one neighbor pair, held negated where that saves the final negation of
-// fdiv_rcp: nn = -(dx, dy, dz) / dist, nq = -(dist / h), omq = 1 - dist / h (as 1 + nq) and the spiky
+// fdiv_rcp_neg: nn = -(dx, dy, dz) / dist, nq = -(dist / h), omq = 1 - dist / h (as 1 + nq) and the spiky
 // derivative der = (-2 k (1 - q)) / h (FluidSpikyKernelDerivative, physics_fluid_common.hlsli:31-42;
 // 0 unless eps < dist < h), computed as -((2 k omq) / h).  The consumers take -(a b) = (-a) b and
 // x - (-y) = x + y, which are exact, so every result has the bits of the plain forms.  FAST divides
-// through reciprocals (fdiv_rcp: 1 / dist once per pair, 1 / h once per particle); quot_fast_ok
+// through reciprocals (fdiv_rcp_neg: 1 / dist once per pair, 1 / h once per particle); quot_fast_ok
 // says when that is exact, and the other particles take the IEEE divisions.
 struct PairQuot {
     float nnx, nny, nnz, nq, omq, der;  // nq = -(dist / h)
 };
 
-// fdiv_rcp is exact for every quotient of pair_quot when h <= 1024 and each coordinate of the
+// fdiv_rcp_neg is exact for every quotient of pair_quot when h <= 1024 and each coordinate of the
 // particle has magnitude >= 2^-62: a nonzero coordinate difference is then >= 2^-86 (both values
 // are multiples of 2^-86, or the difference exceeds half the larger one), the live distances lie
 // in (eps, h), and with h in [1e-4, 1024] the spiky numerator 2 k (1 - q) lies in
@@ -296,7 +296,7 @@ struct DensitySelf {
     float4 s;
     float h, t2, kw, ih;  // ih = 1 / h
     bool tension;
-    bool fd;          // the neighbor quotients may use fdiv_rcp (pair_quot)
+    bool fd;          // the neighbor quotients may use fdiv_rcp_neg (pair_quot)
 };
 
 // Returns false (and writes the unreachable record) for particles that take no part in the solve.
@@ -2014,8 +2014,8 @@ __global__ __launch_bounds__(kBlock) void k_fluid_render_aniso(FluidArgs a, Subs
 // pass reads again in the same staging.  Walked particle by particle through the run table, every
 // candidate cost a dependent load and a branch: 270 us for the curl of 200,000 particles and 207 us for
 // the anisotropy, against 79 and 89 us; the confinement (41 us, 38 from a list of slots) only follows
-// the curl's list.  What bounds them now: the walk's distance tests (all 27 cells: nothing bounds how
-// far the update moved a particle from its cell), and in the confinement the latency of a block's
+// the curl's list.  What bounds them now: the walk's distance tests (all 27 cells: the passes'
+// bound on how far a particle has moved from its cell is not looked at), and in the confinement the latency of a block's
 // staging, some two blocks to each workgroup the chip holds.
 // Blocks with a halo larger than the tile, or without a descriptor, walk the run table.
 constexpr int kPostCurl = 0, kPostConfine = 1, kPostAniso = 2;

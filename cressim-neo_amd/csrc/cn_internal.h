@@ -25,9 +25,7 @@ constexpr uint32_t kStateDelta = kIterStateWords * kXcds * kQueueStride;
 constexpr uint32_t kStateWideQueue = 2 * kIterStateWords * kXcds * kQueueStride;
 constexpr uint32_t kStateWideCount = kStateWideQueue + kIterStateWords;
 constexpr uint32_t kStateMaxDisp = kStateWideCount + 1;
-constexpr uint32_t kStatePrevDisp = kStateMaxDisp + kIterStateWords;  // the last iteration's word of the
-                                                                        // previous substep
-constexpr uint32_t kStateWords = kStatePrevDisp + 1;
+constexpr uint32_t kStateWords = kStateMaxDisp + kIterStateWords;
 // per-block halo descriptor: start slot and exclusive particle offset of each of the 6x6x6 halo
 // cells (x fastest), the halo particle total, a purity flag, the block's particle range and the
 // cell coordinates of its low corner
@@ -72,7 +70,7 @@ inline size_t list_entries(size_t n, uint32_t entries)
     return list_slots(n) * list_rows(entries ? entries : 1u) + 2 * 4 * kListGroup;
 }
 // Bytes of the entries themselves (slots x entries) that cn_scene_reserve and the candidate lists
-// allow.
+// allow a pool: larger workloads are split into pools.
 constexpr uint64_t kListBytesMax = 0xffffffffull - 0x100000ull;
 // halo particles a list entry can name (a byte offset of 16-byte records), less the filling entry
 constexpr uint32_t kTileMost = 4095;
@@ -138,7 +136,7 @@ struct CorrRec {
 // particles' correction records, all in LDS.
 // Constrained particles of a tile.  Up to kSoftFew of them tiles of 256 would leave CUs with fewer than
 // two, and what a pass takes is a tile's latency: half the particles a tile take a 32^3 tet block from
-// 752 to 667 us a step and a 256 x 256 cloth from 737 to 719.  Past that the larger tiles' fewer border
+// 785 to 708 us a step and a 253 x 253 cloth from 767 to 747.  Past that the larger tiles' fewer border
 // constraints count: 48 mixed scenes 4,807 against 4,868 us.
 constexpr uint32_t kSoftTile = 256, kSoftFew = 2 * 256 * kSoftTile;
 constexpr uint32_t kSoftTileLds = 76u * 1024u;  // two workgroups per CU
@@ -215,7 +213,7 @@ struct SceneBuffers {
     uint32_t *elem_run = nullptr;
     uint32_t *run_key = nullptr;
     uint32_t *run_start = nullptr;  // n + 1
-    int4 *run_info = nullptr;       // (cx, cy, cz, pure)
+    int4 *run_info = nullptr;       // (cx, cy, cz, kRunPure | run_class or 0)
     uint32_t *bucket = nullptr;     // (1 << bucket_bits) + 1
     uint32_t bucket_bits = 0;
     uint2 *tile_counts = nullptr;   // runs and blocks per 1024-key tile (scanned when there are many)

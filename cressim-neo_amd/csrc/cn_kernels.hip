@@ -186,7 +186,7 @@ struct EmitArgs {
     uint32_t *blk_first_run, *nblk;
     uint32_t prefix_shift, fluid_scenes;
     uint32_t *work;  // the substep's queue counters (the max-displacement words past nwork are kept)
-    uint32_t nwork, last_word, prev_word;
+    uint32_t nwork;
     uint32_t *meta;
 };
 
@@ -262,7 +262,6 @@ __global__ __launch_bounds__(kBlock) void k_run_emit(EmitArgs a)
     }
     // the queue counters, cleared by every workgroup's share
     for (uint32_t w = blockIdx.x * kBlock + threadIdx.x; w < a.nwork; w += gridDim.x * kBlock) a.work[w] = 0;
-    if (blockIdx.x == 0 && threadIdx.x == 0) a.work[a.prev_word] = a.work[a.last_word];
     // the longest run: the tile's largest, and an atomic only when it beats the value already stored
     // (one look at that word per tile: one per wave of particles cost 105 us of a launch at 4,194,304)
     __syncthreads();
@@ -317,8 +316,6 @@ void launch_runs(SceneBuffers &s, const SubstepConsts &c, const uint2 *sorted, u
     a.fluid_scenes = c.key_mode == CN_KEY_MORTON ? c.fluid_scenes : 0u;
     a.work = s.iter_state;
     a.nwork = kStateMaxDisp;
-    a.last_word = kStateMaxDisp + std::min<uint32_t>(std::max<uint32_t>(c.fluid_iters, 1u), kIterStateWords) - 1;
-    a.prev_word = kStatePrevDisp;
     a.meta = s.meta;
     hipLaunchKernelGGL(k_run_count, dim3(nb), dim3(kBlock), 0, st, sorted, c.n, s.tile_counts, s.nblk);
     if (a.scanned) hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(1024), 0, st, s.tile_counts, nb);

@@ -222,7 +222,7 @@ typedef struct cn_step_params {
  * of walking the 27 cells again, in every cell block whose particles' displacement since the first
  * iteration (by the fluid passes and by contacts) plus the largest one in the block's halo stays
  * below 0.05 h; the other blocks walk.  The lists are the same either way (same neighbors, same order),
- * so the results are too.  The candidate lists take 198 bytes per particle, allocated on the first
+ * so the results are too.  The candidate lists take 196 bytes per particle, allocated on the first
  * step that asks (left off when they would exceed 4 GiB less 1 MiB).  On in
  * cn_default_step_params. */
 #define CN_STEP_CANDIDATE_REUSE 1u
