@@ -60,3 +60,24 @@ def test_pool_of_both_kinds(oracle):
             oracle.step(osc, params())
         np.testing.assert_array_equal(got[k][0], osc.pos, err_msg=f"scene {k}")
         np.testing.assert_array_equal(got[k][2], osc.vel, err_msg=f"scene {k}")
+
+
+@pytest.mark.parametrize("colliders", [31, 32, 33])
+def test_edits_across_the_border(solver, oracle, colliders):
+    """Walls switched off, moved and back on: the enabled colliders of a scene cross the border both ways."""
+    sc = studded(colliders, 5)
+    osc = oracle.OracleScene(sc)
+    solver.reserve(sc.n, 64)
+    solver.upload(sc)
+    for s, (off, dx) in enumerate([(0, 0.0), (2, 0.0), (1, 0.03), (0, 0.03)]):
+        print(f"{colliders} colliders, {off} off", flush=True)
+        cols = sc.colliders.copy()
+        cols["center"][0] += np.float32(dx)
+        cols["enabled"][len(cols) - off:] = 0
+        solver.set_scene_colliders(0, cols)
+        osc.colliders[:] = cols
+        solver.step(params())
+        oracle.step(osc, params())
+        pos, _, vel = solver.readback()
+        np.testing.assert_array_equal(pos, osc.pos, err_msg=f"edit {s}")
+        np.testing.assert_array_equal(vel, osc.vel, err_msg=f"edit {s}")
